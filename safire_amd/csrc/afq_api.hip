@@ -137,6 +137,8 @@ void run_exchange(afq_ham H, hipStream_t s, int W, const double* G) {
   else if (H->precision == AFQ_INT8_SPLIT)
     launch_exchange_i8(s, W, H->M, H->N, H->K, G, H->Lnak_q, H->Lnak_u, H->Lnak_ord, H->ws.Kl,
                        H->ws.exx);
+  else if (H->precision == AFQ_FP64 && exchange_f64_supported(H->M, H->N))
+    launch_exchange_f64(s, W, H->M, H->N, H->K, G, H->Lnak, H->Lnak_r, H->ws.Kl, H->ws.exx);
   else
     launch_exchange(s, H->precision, W, H->M, H->N, H->K, G, L_for(H), H->ws.Kl, H->ws.exx);
 }
@@ -144,6 +146,8 @@ void run_exchange(afq_ham H, hipStream_t s, int W, const double* G) {
 int exchange_chunks(afq_ham H, int W) {
   if (H->precision == AFQ_BF16X3) return exchange_bf16_chunks(W, H->N, H->K);
   if (H->precision == AFQ_INT8_SPLIT) return exchange_i8_chunks(W, H->N, H->K);
+  if (H->precision == AFQ_FP64 && exchange_f64_supported(H->M, H->N))
+    return exchange_f64_chunks(W, H->N, H->K);
   return exx_nchunks(W, H->N, H->K);
 }
 
@@ -251,7 +255,13 @@ int afq_ham_create(int M, int N, int K, const double* h_h, const double* h_Likn,
       AFQ_HIP(hipMemcpy(H->Likn, h_Likn, MM * K * sizeof(double), hipMemcpyHostToDevice));
       AFQ_HIP(hipMemcpy(H->h, h_h, MM * sizeof(double), hipMemcpyHostToDevice));
       AFQ_HIP(hipMemset(H->stats, 0, 7 * sizeof(unsigned long long)));
+      H->real_trial = true;
+      for (size_t e = 0; e < NM; ++e) H->real_trial = H->real_trial && h_PsiT[2 * e + 1] == 0.0;
       setup_hamiltonian(H, nullptr);
+      if (H->real_trial) {
+        dalloc(&H->Lnak_r, (size_t)K * N * real_lnak_row(M));
+        launch_real_rows(nullptr, (long)K * N, M, real_lnak_row(M), H->Lnak, H->Lnak_r);
+      }
       if (exchange_bf16_supported(M, N)) {
         dalloc(&H->Lnak_b, exchange_bf16_elems(M, N, K));
         split_lnak_bf16(nullptr, M, N, K, H->Lnak, H->Lnak_b);
@@ -292,6 +302,7 @@ int afq_ham_destroy(afq_ham H) {
     dfree(H->vMF);
     dfree(H->P1);
     dfree(H->H1);
+    dfree(H->Lnak_r);
     dfree(H->Lnak_f);
     dfree(H->Likn_f);
     dfree(H->Lnak_ord);

@@ -168,6 +168,8 @@ struct afq_ham_s {
   double* vMF = nullptr;     // c128 [K]
   double* P1 = nullptr;      // c128 [M][M]
   double* H1 = nullptr;      // c128 [M][M]
+  bool real_trial = false;   // every imaginary part of PsiT is zero (so is Im Lnak)
+  double* Lnak_r = nullptr;  // f64 [K][N][M padded to 16]: Re Lnak, only with a real trial
   float* Lnak_f = nullptr;   // c64 [K][N][M]   (FP32 contraction copies)
   float* Likn_f = nullptr;   // f32 [M*M][K]
   __bf16* Lnak_b = nullptr;  // bf16 [6 planes][K][16 NT][32 KC]  (BF16X3 exchange)
@@ -217,6 +219,13 @@ void launch_gemm_nt_z(hipStream_t s, int precision, int m, int n, int k, double 
 // k_energy.hip
 int device_cus();                        // compute units of the current device (cached)
 int exx_nchunks(int W, int N, int K);   // chunks of Cholesky vectors the exchange kernel uses
+// k_exchange_f64.hip: the exchange of the FP64 form on up to 128 orbitals; Lreal (may be NULL) is
+// the zero-padded real Lnak of a real trial
+bool exchange_f64_supported(int M, int N);
+int exchange_f64_chunks(int W, int N, int K);   // tr(T^2) partials per walker
+int real_lnak_row(int M);                       // padded row length of Lreal
+void launch_exchange_f64(hipStream_t s, int W, int M, int N, int K, const double* G,
+                         const double* Lnak, const double* Lreal, double* Kl, double* part);
 void launch_split_reduce(hipStream_t s, int m, int n, int splits, double alpha,
                          const double* split_ws, double* C, long ldc);
 // k_gemm_bf16.hip: the BF16X3 form of the Cholesky GEMMs (three-product complex multiplication,
@@ -301,6 +310,8 @@ void launch_population_control(hipStream_t s, int W, double* wbuf, long ldw, lon
 // k_setup.hip
 void setup_hamiltonian(afq_ham_s* H, hipStream_t s);
 void launch_v0(hipStream_t s, int M, int K, const double* Likn, double* v0);
+// dst[row][0..ld) = Re src[row][0..M), zero-padded
+void launch_real_rows(hipStream_t s, long rows, int M, int ld, const double* src, double* dst);
 void launch_zero_imag(hipStream_t s, int n, double* v);
 // P1 [M][M] c128 on the host as the reference applies it: |x| <= 1e-8 dropped, imaginary
 // roundoff dropped when P1 is real to 1e-14

@@ -100,6 +100,15 @@ __global__ void k_zgemm_small(int n, double alpha, const cd* __restrict__ A,
   C[e] = s;
 }
 
+__global__ void k_real_rows(long rows, int M, int ld, const cd* __restrict__ src,
+                            double* __restrict__ dst) {
+  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= rows * ld) return;
+  const long r = e / ld;
+  const int k = (int)(e - r * ld);
+  dst[e] = k < M ? src[r * M + k].re : 0.0;
+}
+
 __global__ void k_to_f32(long n, const double* __restrict__ x, float* __restrict__ y) {
   const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (e < n) y[e] = (float)x[e];
@@ -120,6 +129,12 @@ void launch_half_rotate(hipStream_t s, int M, int N, int K, const double* PsiT, 
 // v0[i][l] = -1/2 sum_{j,n} L[i][j][n] L[l][j][n]  (RealDenseHamiltonian.cpp:163-180)
 void launch_v0(hipStream_t s, int M, int K, const double* Likn, double* v0) {
   hipLaunchKernelGGL(k_v0, blocks((long)M * M), dim3(256), 0, s, M, K, Likn, v0);
+  AFQ_HIP(hipGetLastError());
+}
+
+void launch_real_rows(hipStream_t s, long rows, int M, int ld, const double* src, double* dst) {
+  hipLaunchKernelGGL(k_real_rows, blocks(rows * ld), dim3(256), 0, s, rows, M, ld, (const cd*)src,
+                     dst);
   AFQ_HIP(hipGetLastError());
 }
 

@@ -1,0 +1,85 @@
+"""Exchange and Coulomb energy kernels at the edges of their tiles: row and column packing across
+walkers and Cholesky vectors, remainders of every tile, one walker to many, real and complex trial
+orbitals, walkers with a non-finite Green's function."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+if not torch.cuda.is_available():  # pragma: no cover
+    pytest.skip("no GPU", allow_module_level=True)
+
+from safire_amd import afqmc as A  # noqa: E402
+
+SHAPES = [  # (M, N, K, W)
+    (16, 1, 3, 1), (17, 2, 70, 3), (24, 6, 21, 64), (31, 8, 9, 130), (32, 16, 4, 9),
+    (33, 17, 7, 9), (48, 12, 11, 300), (64, 16, 33, 70), (64, 24, 5, 11), (65, 25, 3, 6),
+    (77, 19, 13, 13), (96, 9, 15, 20), (97, 28, 6, 33), (128, 31, 3, 140), (128, 32, 9, 5),
+]
+
+
+def make(M, N, K, W, complex_trial):
+    rng = np.random.default_rng([M, N, K, W, int(complex_trial)])
+    h = rng.standard_normal((M, M))
+    h = h + h.T
+    L = rng.standard_normal((M, M, K)) * np.exp(-5.0 * np.arange(K) / K) / np.sqrt(M)
+    L = L + L.transpose(1, 0, 2)
+    q = rng.standard_normal((M, M)) + (1j * rng.standard_normal((M, M)) if complex_trial else 0.0)
+    PsiT = np.linalg.qr(q)[0][:, :N].conj().T.astype(np.complex128)
+    G = rng.standard_normal((W, N, M)) + 1j * rng.standard_normal((W, N, M))
+    return h, L, PsiT, G
+
+
+def reference(h, L, PsiT, G):
+    """(E, scale): the energies and, per component, the sum of the magnitudes of their terms."""
+    Lnak = np.einsum("ai,ijn->naj", PsiT, L)
+    T = np.einsum("wbk,nak->wnba", G, Lnak)
+    kl = np.einsum("wnaa->wn", T)
+    e1 = 2 * np.einsum("waj,aj->w", G, PsiT @ h)
+    exx = -np.einsum("wnab,wnba->w", T, T)
+    E = np.stack([e1, exx, 2 * (kl ** 2).sum(1)], 1)
+    mag = np.abs(T)
+    S = np.stack([2 * np.einsum("waj,aj->w", np.abs(G), np.abs(PsiT @ h)),
+                  np.einsum("wnab,wnba->w", mag, mag),
+                  2 * (np.einsum("wnaa->wn", mag) ** 2).sum(1)], 1)
+    return E, S
+
+
+def energies(h, L, PsiT, G, form):
+    ham = A.HamiltonianOperations(h, L, PsiT, 0.0, 0.01)
+    ham.reserve(len(G))
+    ham.set_precision(form)
+    E = torch.full((len(G), 3), 7.0, dtype=torch.complex128, device="cuda")
+    ham.energy(A.to_device(G), E)
+    torch.cuda.synchronize()
+    out = E.cpu().numpy()
+    ham.close()
+    return out
+
+
+@pytest.mark.parametrize("complex_trial", [False, True])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_energy_fp64_tile_edges(shape, complex_trial):
+    h, L, PsiT, G = make(*shape, complex_trial)
+    want, scale = reference(h, L, PsiT, G)
+    got = energies(h, L, PsiT, G, 0)
+    # products of M terms, each rounded to 2^-53, squared and summed
+    assert np.max(np.abs(got - want) / scale) < 1e-13
+
+
+@pytest.mark.parametrize("complex_trial", [False, True])
+@pytest.mark.parametrize("shape", [(24, 6, 21, 5), (77, 19, 13, 7), (128, 32, 9, 5)])
+@pytest.mark.parametrize("form", [0, 3])
+def test_energy_keeps_non_finite_walkers_apart(shape, complex_trial, form):
+    h, L, PsiT, G = make(*shape, complex_trial)
+    clean = energies(h, L, PsiT, G, form)
+    G[1, 0, 3] = complex(np.nan, 0.0)
+    G[2, shape[1] - 1, shape[0] - 1] = complex(0.5, np.inf)
+    G[4, 0, 0] = complex(-np.inf, 1.0)
+    got = energies(h, L, PsiT, G, form)
+    for w in range(shape[3]):
+        if w in (1, 2, 4):
+            assert not np.isfinite(got[w, 1:].real).any()
+        else:
+            assert np.array_equal(got[w], clean[w])
