@@ -135,7 +135,7 @@ void run_exchange(afq_ham H, hipStream_t s, int W, const double* G) {
   if (H->precision == AFQ_BF16X3)
     launch_exchange_bf16(s, W, H->M, H->N, H->K, G, H->Lnak_b, H->ws.Kl, H->ws.exx);
   else if (H->precision == AFQ_INT8_SPLIT)
-    launch_exchange_i8(s, W, H->M, H->N, H->K, G, H->Lnak_q, H->Lnak_u, H->Lnak_ord, H->ws.Kl,
+    launch_exchange_i8(s, W, H->M, H->N, H->K, G, H->real_trial, H->Lnak_q, H->Lnak_u, H->Lnak_ord, H->ws.Kl,
                        H->ws.exx);
   else if (H->precision == AFQ_FP64 && exchange_f64_supported(H->M, H->N))
     launch_exchange_f64(s, W, H->M, H->N, H->K, G, H->Lnak, H->Lnak_r, H->ws.Kl, H->ws.exx);
@@ -145,7 +145,7 @@ void run_exchange(afq_ham H, hipStream_t s, int W, const double* G) {
 
 int exchange_chunks(afq_ham H, int W) {
   if (H->precision == AFQ_BF16X3) return exchange_bf16_chunks(W, H->N, H->K);
-  if (H->precision == AFQ_INT8_SPLIT) return exchange_i8_chunks(W, H->N, H->K);
+  if (H->precision == AFQ_INT8_SPLIT) return exchange_i8_chunks(W, H->M, H->N, H->K, H->real_trial);
   if (H->precision == AFQ_FP64 && exchange_f64_supported(H->M, H->N))
     return exchange_f64_chunks(W, H->N, H->K);
   return exx_nchunks(W, H->N, H->K);
@@ -271,13 +271,11 @@ int afq_ham_create(int M, int N, int K, const double* h_h, const double* h_Likn,
         split_planes_bf16(nullptr, (long)MM, K, false, H->Likn, H->Likn_g);
       }
       if (exchange_i8_supported(M, N)) {
-        dalloc(&H->Lnak_q, exchange_i8_bytes(M, N, K));
+        dalloc(&H->Lnak_q, exchange_i8_bytes(M, N, K, H->real_trial));
         dalloc(&H->Lnak_u, (size_t)K * N);
-        split_lnak_i8(nullptr, M, N, K, H->Lnak, H->Lnak_q, H->Lnak_u);
-        if (N > 16) {
-          dalloc(&H->Lnak_ord, (size_t)K);
-          exchange_i8_orders(nullptr, M, N, K, H->Lnak, H->Lnak_ord);
-        }
+        split_lnak_i8(nullptr, M, N, K, H->Lnak, H->real_trial, H->Lnak_q, H->Lnak_u);
+        dalloc(&H->Lnak_ord, (size_t)K);
+        exchange_i8_orders(nullptr, M, N, K, H->Lnak, H->Lnak_ord);
       }
       AFQ_HIP(hipDeviceSynchronize());
     } catch (...) {

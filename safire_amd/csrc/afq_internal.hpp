@@ -175,9 +175,9 @@ struct afq_ham_s {
   __bf16* Lnak_b = nullptr;  // bf16 [6 planes][K][16 NT][32 KC]  (BF16X3 exchange)
   __bf16* Lnak_g = nullptr;  // bf16 [6 planes][K][N*M padded to 32]   (BF16X3 vbias)
   __bf16* Likn_g = nullptr;  // bf16 [2 planes][M*M][K padded to 32]   (BF16X3 vHS)
-  int8_t* Lnak_q = nullptr;  // i8 [5 or 6 slices][re,im][K][N][Mp] (INT8_SPLIT exchange)
+  int8_t* Lnak_q = nullptr;  // i8 [6 slices][re(, im)][K][N][Mp] (INT8_SPLIT exchange)
   double* Lnak_u = nullptr;  // f64 [K][N]   power-of-two unit of each Lnak row
-  int* Lnak_ord = nullptr;   // i32 [K]      slice-product order of each vector (N > 16)
+  int* Lnak_ord = nullptr;   // i32 [K]      slice-product order of each vector
   // [7]: eloc total/upper/lower, weight total/upper, population control calls/collapses
   unsigned long long* stats = nullptr;
   // back-propagation: the caller's field ring [fields_W][nfields][K] c128 and its position
@@ -245,17 +245,17 @@ int exchange_bf16_chunks(int W, int N, int K);
 void split_lnak_bf16(hipStream_t s, int M, int N, int K, const double* Lnak, __bf16* Lb);
 void launch_exchange_bf16(hipStream_t s, int W, int M, int N, int K, const double* G,
                           const __bf16* Lb, double* Kl, double* exx_part);
-// k_exchange_i8.hip: the exchange on int8 MFMA, Ozaki-split rows (N <= 16, M <= 128)
+// k_exchange_i8.hip: the exchange on int8 MFMA, Ozaki-split rows (N <= 32, M <= 128); real: Im Lnak
+// is zero and only its real slices are kept
 bool exchange_i8_supported(int M, int N);
-int exchange_i8_row(int M);                        // Mp: padded row length of the slices
-size_t exchange_i8_bytes(int M, int N, int K);     // size of the Lnak slices
-int exchange_i8_chunks(int W, int N, int K);   // tr(T^2) partials per walker
-void split_lnak_i8(hipStream_t s, int M, int N, int K, const double* Lnak, int8_t* Lq,
+int exchange_i8_row(int M);                                // Mp: padded row length of the slices
+size_t exchange_i8_bytes(int M, int N, int K, bool real);  // size of the Lnak slices
+int exchange_i8_chunks(int W, int M, int N, int K, bool real);   // tr(T^2) partials per walker
+void split_lnak_i8(hipStream_t s, int M, int N, int K, const double* Lnak, bool real, int8_t* Lq,
                    double* Lu);
-int exchange_i8_slices(int N);                     // slices of each Lnak row
-// per Cholesky vector the slice-product order of the 17..32-electron kernel (set-up, synchronous)
+// per Cholesky vector the slice-product order (set-up, synchronous)
 void exchange_i8_orders(hipStream_t s, int M, int N, int K, const double* Lnak, int* ord);
-void launch_exchange_i8(hipStream_t s, int W, int M, int N, int K, const double* G,
+void launch_exchange_i8(hipStream_t s, int W, int M, int N, int K, const double* G, bool real,
                         const int8_t* Lq, const double* Lu, const int* ord, double* Kl,
                         double* exx_part);
 void launch_exchange(hipStream_t s, int precision, int W, int M, int N, int K, const double* G,

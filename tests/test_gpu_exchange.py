@@ -69,6 +69,18 @@ def test_energy_fp64_tile_edges(shape, complex_trial):
 
 
 @pytest.mark.parametrize("complex_trial", [False, True])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_energy_int8_tile_edges(shape, complex_trial):
+    h, L, PsiT, G = make(*shape, complex_trial)
+    want, scale = reference(h, L, PsiT, G)
+    got = energies(h, L, PsiT, G, 3)
+    # six base-254 slices leave 254^-5 / 2 of a row's unit in each factor and drop products of
+    # order 6 and up (vectors of smaller size: of an order that keeps them below that): with row
+    # maxima at most ~30 times the typical element here, under 2e-9 of the summed magnitudes
+    assert np.max(np.abs(got - want) / scale) < 2e-9
+
+
+@pytest.mark.parametrize("complex_trial", [False, True])
 @pytest.mark.parametrize("shape", [(24, 6, 21, 5), (77, 19, 13, 7), (128, 32, 9, 5)])
 @pytest.mark.parametrize("form", [0, 3])
 def test_energy_keeps_non_finite_walkers_apart(shape, complex_trial, form):
