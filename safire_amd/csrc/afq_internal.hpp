@@ -310,6 +310,8 @@ void launch_population_control(hipStream_t s, int W, double* wbuf, long ldw, lon
 // k_setup.hip
 void setup_hamiltonian(afq_ham_s* H, hipStream_t s);
 void launch_v0(hipStream_t s, int M, int K, const double* Likn, double* v0);
+// whether L[i][j][n] equals L[j][i][n] bit for bit for all i, j, n (synchronises the stream)
+bool likn_symmetric(hipStream_t s, int M, int K, const double* Likn);
 // dst[row][0..ld) = Re src[row][0..M), zero-padded
 void launch_real_rows(hipStream_t s, long rows, int M, int ld, const double* src, double* dst);
 void launch_zero_imag(hipStream_t s, int n, double* v);
@@ -332,6 +334,10 @@ void launch_ph_1body(hipStream_t s, int nw, int ndet, int nex, int nact, int nel
 void launch_ph_woodbury(hipStream_t s, int nb, int nmo, int nel, int nact, const double* A,
                         const int* ref, const double* Phi, long ldw, double* G, double* ov,
                         double* QQ0, double* work);
+// the same with the reference at orbitals 0..nel-1 (A's first nel rows)
+void launch_ph_reference_G(hipStream_t s, int nb, int nmo, int nel, int nact, const double* A,
+                           const double* Aref, const double* Phi, long ldw, double* G, double* ov,
+                           double* QQ0);
 void launch_ph_spin_weights(hipStream_t s, int nw, int nu, const int* cp, const int* ci,
                             const double* cv, const double* rup, const double* rdn, double* wgt,
                             double* ov);
@@ -361,7 +367,8 @@ void launch_ph_log_overlap(hipStream_t s, int nw, const double* Ov, const double
                            double* out);
 void launch_ph0_products(hipStream_t s, int nw, int nmo, int nel, int nact, int nchol,
                          const double* Phi, long ldw, const double* A, const double* haj,
-                         const double* Lna, double* Phit, double* TAB, double* Hp, double* P);
+                         const double* Lna, bool lna_complex, double* Phit, double* TAB,
+                         double* Hp, double* P);
 void launch_ph0_config(hipStream_t s, int nw, int nc, int nel, int nact, int nchol,
                        const int* conf, const double* TAB, const double* Hp, const double* P,
                        double E0, double* ld, double* Emsd, double* KE, const double* KEr,
@@ -370,6 +377,38 @@ void launch_ph0_ratios(hipStream_t s, int nw, int nc, double* r, double* log_ov)
 void launch_ph0_assemble(hipStream_t s, int nw, int nu, int nd, const double* wgt0,
                          const double* Em0, const double* wgt1, const double* Em1,
                          const double* r1, double* acc);
+// k_phmsd_exc.hip: an expansion's excited determinants as rank-nex corrections of the reference
+// (the reference determinant at orbitals 0..nel-1, every particle at nel or above)
+struct PhShell {
+  int nex, ndet, row;   // rank, determinants, first row of the ratio and weight arrays
+  int qoff;             // first element of the shell's Q per walker: Q[w][qoff + (e nex + q) ndet + d]
+  const int* iexcit;    // device [ndet][2 nex]
+};
+int ph_exc_vectors(int nel, int nact);               // vectors per workgroup; 0: not supported
+int ph_exc_groups(int nel, int nact, int nchol);     // groups of vectors (8 complex sums each)
+void launch_ph_ratios_q(hipStream_t s, int nw, int nel, int nact, long qtot, int nshell, int maxdet,
+                        int maxnex, const PhShell* shells, const double* QQ0, double* ratio,
+                        double* Q);
+void launch_ph_weights(hipStream_t s, int nw, int nu, const int* cp, const int* ci,
+                       const double* cv, const double* own, const double* other, double* wgt,
+                       double* sum);
+void launch_ph_exc(hipStream_t s, bool down, int nw, int nel, int nact, int nchol, long qtot,
+                   int nshell, int maxnex, int nu_own, int nu_up, const PhShell* shells,
+                   const double* T, const double* QQ0, const double* Q, const double* wgt,
+                   double* KE, const int* cp, const int* ci, const double* cv, const double* rup,
+                   const double* rdn, double* part);
+void launch_ph_exc_finish(hipStream_t s, int nw, int nu, int gu, int gd, double E0, const double* wgt,
+                          const double* pu, const double* pd, const double* log_ov, double* E,
+                          double* ov);
+void launch_ph_expansion_R(hipStream_t s, int nw, int nel, int nact, int nu, long qtot,
+                           const int* rp, const int* ru, const int* rq, const double* QQ0,
+                           const double* Q, const double* wgt, double* R, double* ov);
+void launch_ph_density(hipStream_t s, int nw, int nup, int ndn, int nact, int nmo, bool fold,
+                       const double* R0, const double* A0, const double* G0, const double* R1,
+                       const double* A1, const double* G1, const double* ov, double* U0, double* U1,
+                       double* F);
+void launch_ph_rows_of_vectors(hipStream_t s, int nmo, int nchol, bool fold, const double* Likn,
+                               double* out);
 void launch_ph_accumulate_R(hipStream_t s, int nw, int ndet, int nex, int nact, int nelec,
                             const int* iexcit, const int* refc, const double* Rc,
                             const double* ov, const double* wgt, double* R);

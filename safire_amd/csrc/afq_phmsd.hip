@@ -53,8 +53,13 @@ struct Spin {
   std::vector<std::complex<double>> hA;         // host copy of the orbital rows [nact][nmo]
   double* A = nullptr;             // c128 [nact][nmo]
   int* refc = nullptr;             // [nel]
-  double* Lna = nullptr;           // c128 [nchol][nact][nmo]
-  double* haj = nullptr;           // c128 [nact][nmo]
+  double* Lna = nullptr;           // c128 [nchol + 1][nact][nmo]: Lna_n = A L_n, then haj
+  double* haj = nullptr;           // c128 [nact][nmo]: the last vector of Lna
+  double* Lna_r = nullptr;         // f64 [nchol + 1][nact][nmo], only when the orbitals are real
+  PhShell* dshell = nullptr;       // the shells on the GPU
+  int maxdet = 0, maxnex = 0;
+  long qtot = 0;                   // sum of nex^2 ndet: elements of Q per walker
+  int *rp = nullptr, *ru = nullptr, *rq = nullptr;   // (hole, particle) lists of k_ph_expansion_R
   std::vector<Shell> shells;
   int *cp = nullptr, *ci = nullptr;  // couplings of this spin's excitations with the other's
   double* cv = nullptr;
@@ -150,7 +155,9 @@ struct afq_ph_t {
   int energy_alg = AFQ_PH_ENERGY_WOODBURY;
   double E0 = 0.0;
   afq::Spin spin[2];
-  double* Lstack = nullptr;        // c128 [nchol][2 nact][nmo]: both spins' Lna per vector
+  bool fold = false;               // Likn is symmetric: Lvec holds its rows l <= k
+  bool staged = false;             // the energy runs on k_phmsd_exc.hip's kernels
+  double* Lvec = nullptr;          // f64 [nchol][nmo (nmo + 1) / 2 or nmo^2]: the vectors as rows
   double* h = nullptr;             // f64 [nmo][nmo]
   double* Likn = nullptr;          // f64 [nmo * nmo][nchol]
   // propagator state (afq_ph_prepare) and the step's per-walker workspace
@@ -165,13 +172,15 @@ struct afq_ph_t {
   std::vector<void*> step_owned;
   std::vector<void*> owned;
   // workspace for one walker block
-  double *G[2] = {nullptr, nullptr}, *QQ0[2] = {nullptr, nullptr}, *work = nullptr;
+  double *G[2] = {nullptr, nullptr}, *QQ0[2] = {nullptr, nullptr};
   double *ratios[2] = {nullptr, nullptr}, *wgt[2] = {nullptr, nullptr};
   double *Ov = nullptr, *Ov2 = nullptr, *log_ov = nullptr, *Eref = nullptr, *Ex = nullptr,
          *acc = nullptr;
   double *Twina = nullptr, *Swia = nullptr, *KEa = nullptr, *KEb = nullptr, *KEl = nullptr,
          *R = nullptr;
-  double *Racc = nullptr, *Gblk = nullptr, *split = nullptr, *p2ws = nullptr;
+  double *Q[2] = {nullptr, nullptr}, *Rexp[2] = {nullptr, nullptr}, *RA[2] = {nullptr, nullptr},
+         *part[2] = {nullptr, nullptr};
+  double *F = nullptr, *Gblk = nullptr, *split = nullptr, *p2ws = nullptr;
   double* Emsd = nullptr;          // c128 [2][max nunique][wblock][4] (energy_alg0)
   double* Tinv0 = nullptr;         // c128 [max nunique][wblock][nel][nel] (energy_alg0)
   long split_elems = 0, p2ws_doubles = 0;
@@ -203,17 +212,35 @@ int ph_guard(F&& f) {
 }
 
 // Step 1 of energy_alg1 / MixedDensityMatrix: the reference G, QQ0 and log overlap of both spins
-// and the excitation overlap ratios (row 0 = the reference).
+// and the excitation overlap ratios (row 0 = the reference) with the inverses Q behind them.
 void ph_overlaps_block(afq_ph_t* ph, hipStream_t s, int nb, const double* const Phi[2], long ldw) {
   Spin* S = ph->spin;
   launch_ph_fill(s, nb, 0.0, 0.0, ph->log_ov);
   for (int sp = 0; sp < 2; ++sp) {
-    launch_ph_woodbury(s, nb, ph->nmo, S[sp].nel, ph->nact, S[sp].A, S[sp].refc, Phi[sp], ldw,
-                       ph->G[sp], ph->log_ov, ph->QQ0[sp], ph->work);
-    launch_ph_fill(s, nb, 1.0, 0.0, ph->ratios[sp]);
-    for (const Shell& sh : S[sp].shells)
-      launch_ph_overlaps(s, nb, sh.ndet, sh.nex, ph->nact, S[sp].nel, sh.iexcit, ph->QQ0[sp],
-                         ph->ratios[sp] + 2L * sh.row * nb);
+    launch_ph_reference_G(s, nb, ph->nmo, S[sp].nel, ph->nact, S[sp].A, S[sp].A, Phi[sp], ldw,
+                          ph->G[sp], ph->log_ov, ph->QQ0[sp]);
+    launch_ph_ratios_q(s, nb, S[sp].nel, ph->nact, S[sp].qtot, (int)S[sp].shells.size(),
+                       S[sp].maxdet, S[sp].maxnex, S[sp].dshell, ph->QQ0[sp], ph->ratios[sp],
+                       ph->Q[sp]);
+  }
+}
+
+// weights W_s[u] = ratio_s[u] sum_d C_s[u][d] ratio_other[d]; sum (may be NULL): their sum
+void ph_weights_block(afq_ph_t* ph, hipStream_t s, int nb, int sp, double* sum) {
+  const Spin& S = ph->spin[sp];
+  launch_ph_weights(s, nb, S.nunique, S.cp, S.ci, S.cv, ph->ratios[sp], ph->ratios[1 - sp],
+                    ph->wgt[sp], sum);
+}
+
+// The expansion's R of both spins (Rexp) and its overlap relative to the reference (Ov)
+void ph_expansion_block(afq_ph_t* ph, hipStream_t s, int nb, const double* const Phi[2], long ldw) {
+  Spin* S = ph->spin;
+  ph_overlaps_block(ph, s, nb, Phi, ldw);
+  for (int sp = 0; sp < 2; ++sp) {
+    ph_weights_block(ph, s, nb, sp, nullptr);
+    launch_ph_expansion_R(s, nb, S[sp].nel, ph->nact, S[sp].nunique, S[sp].qtot, S[sp].rp, S[sp].ru,
+                          S[sp].rq, ph->QQ0[sp], ph->Q[sp], ph->wgt[sp], ph->Rexp[sp],
+                          sp == 0 ? ph->Ov : ph->Ov2);
   }
 }
 
@@ -221,34 +248,14 @@ void ph_overlaps_block(afq_ph_t* ph, hipStream_t s, int nb, const double* const 
 // [0, nact) and [nact, 2 nact) of d_Gc [nb][2 nact][nmo]; d_logov [nb] = log Ov + log_ov.
 void ph_density_block(afq_ph_t* ph, hipStream_t s, int nb, const double* const Phi[2], long ldw,
                       double* d_Gc, double* d_logov) {
-  Spin* S = ph->spin;
   const int na = ph->nact;
-  ph_overlaps_block(ph, s, nb, Phi, ldw);
-  for (int sp = 0; sp < 2; ++sp) {
-    // weights W[u] = ratio_s[u] sum_d C[u][d] ratio_other[d] (the up spin's also give Ov)
-    launch_ph_spin_weights(s, nb, S[sp].nunique, S[sp].cp, S[sp].ci, S[sp].cv, ph->ratios[sp],
-                           ph->ratios[1 - sp], ph->wgt[sp], sp == 0 ? ph->Ov : ph->Ov2);
-    // calculate_R: the reference, then every shell in determinant blocks
-    launch_ph_fill(s, (long)nb * S[sp].nel * na, 0.0, 0.0, ph->Racc);
-    launch_ph_accumulate_R(s, nb, 1, 0, na, S[sp].nel, nullptr, S[sp].refc, nullptr, nullptr,
-                           ph->wgt[sp], ph->Racc);
-    for (const Shell& sh : S[sp].shells)
-      for (int d0 = 0; d0 < sh.ndet; d0 += kPhDetBlock) {
-        const int nbk = std::min(kPhDetBlock, sh.ndet - d0);
-        const int* iex = sh.iexcit + 2L * sh.nex * d0;
-        launch_ph_compact_R(s, nb, nbk, sh.nex, na, S[sp].nel, iex, S[sp].refc, ph->QQ0[sp],
-                            ph->R);
-        launch_ph_accumulate_R(s, nb, nbk, sh.nex, na, S[sp].nel, iex, S[sp].refc, ph->R,
-                               ph->ratios[sp] + 2L * (sh.row + d0) * nb,
-                               ph->wgt[sp] + 2L * (sh.row + d0) * nb, ph->Racc);
-      }
-    launch_ph_rg(s, nb, S[sp].nel, na, ph->nmo, 2 * na, sp * na, ph->Racc, ph->G[sp], ph->Ov,
-                 d_Gc);
-  }
+  ph_expansion_block(ph, s, nb, Phi, ldw);
+  for (int sp = 0; sp < 2; ++sp)
+    launch_ph_rg(s, nb, ph->spin[sp].nel, na, ph->nmo, 2 * na, sp * na, ph->Rexp[sp], ph->G[sp],
+                 ph->Ov, d_Gc);
   launch_ph_log_overlap(s, nb, ph->Ov, ph->log_ov, d_logov);
 }
 
-// PHMSD::energy_alg1 over all walkers, in walker blocks
 // PHMSD::energy_alg0 (PHMSD.cpp:122-370), COLLINEAR walkers, in walker blocks: each unique
 // configuration's own G and single-determinant energy, its overlap relative to the spin's
 // reference configuration, the up spin's Cholesky traces carried to the down configurations
@@ -266,7 +273,7 @@ void ph_energy_alg0(afq_ph_t* ph, hipStream_t s, int nw, const double* d_wbuf, l
     launch_ph_fill(s, nb, 0.0, 0.0, ph->log_ov);
     for (int sp = 0; sp < 2; ++sp) {
       launch_ph0_products(s, nb, nmo, S[sp].nel, na, K, Phi[sp], ldw, S[sp].A, S[sp].haj,
-                          S[sp].Lna, ph->G[sp], ph->QQ0[sp], ph->Swia, ph->Twina);
+                          S[sp].Lna_r ? S[sp].Lna_r : S[sp].Lna, S[sp].Lna_r == nullptr, ph->G[sp], ph->QQ0[sp], ph->Swia, ph->Twina);
       launch_ph0_config(s, nb, S[sp].nunique, S[sp].nel, na, K, S[sp].dconf, ph->QQ0[sp],
                         ph->Swia, ph->Twina, sp == 0 ? ph->E0 : 0.0, ph->ratios[sp],
                         ph->Emsd + sp * em1, sp == 0 ? ph->KEa : nullptr,
@@ -276,13 +283,39 @@ void ph_energy_alg0(afq_ph_t* ph, hipStream_t s, int nw, const double* d_wbuf, l
         launch_ph_couple_ke(s, nb, K, nd, S[1].cp, S[1].ci, S[1].cv, ph->ratios[0], ph->KEa,
                             nullptr, ph->KEb);
     }
-    launch_ph_spin_weights(s, nb, nu, S[0].cp, S[0].ci, S[0].cv, ph->ratios[0], ph->ratios[1],
-                           ph->wgt[0], ph->Ov);
-    launch_ph_spin_weights(s, nb, nd, S[1].cp, S[1].ci, S[1].cv, ph->ratios[1], ph->ratios[0],
-                           ph->wgt[1], ph->Ov2);
+    ph_weights_block(ph, s, nb, 0, ph->Ov);
+    ph_weights_block(ph, s, nb, 1, nullptr);
     launch_ph0_assemble(s, nb, nu, nd, ph->wgt[0], ph->Emsd, ph->wgt[1], ph->Emsd + em1,
                         ph->ratios[1], ph->acc);
     launch_ph_finalize(s, nb, ph->acc, ph->Ov, ph->log_ov, d_E + 6L * w0, d_ov + 2L * w0);
+  }
+}
+
+// PHMSD::energy_alg1 over all walkers, in walker blocks: the products T of the reference's G with the
+// half-rotated vectors and haj (one GEMM per spin), then each spin's determinants as corrections of
+// the reference (k_phmsd_exc.hip)
+void ph_energy_staged(afq_ph_t* ph, hipStream_t s, int nw, const double* d_wbuf, long ldw,
+                      double* d_E, double* d_ov) {
+  const int nmo = ph->nmo, na = ph->nact, K = ph->nchol;
+  Spin* S = ph->spin;
+  for (int w0 = 0; w0 < nw; w0 += ph->wblock) {
+    const int nb = std::min(ph->wblock, nw - w0);
+    const double* Phi[2] = {d_wbuf + 2 * (long)w0 * ldw,
+                            d_wbuf + 2 * ((long)w0 * ldw + (long)nmo * S[0].nel)};
+    ph_overlaps_block(ph, s, nb, Phi, ldw);
+    for (int sp = 0; sp < 2; ++sp) ph_weights_block(ph, s, nb, sp, nullptr);
+    for (int sp = 0; sp < 2; ++sp) {
+      launch_gemm_nt_z(s, AFQ_FP64, nb * S[sp].nel, (K + 1) * na, nmo, 1.0, ph->G[sp], nmo,
+                       S[sp].Lna_r ? S[sp].Lna_r : S[sp].Lna, nmo, S[sp].Lna_r == nullptr,
+                       ph->Twina, (long)(K + 1) * na);
+      launch_ph_exc(s, sp == 1, nb, S[sp].nel, na, K, S[sp].qtot, (int)S[sp].shells.size(),
+                    S[sp].maxnex, S[sp].nunique, S[0].nunique, S[sp].dshell, ph->Twina, ph->QQ0[sp],
+                    ph->Q[sp], ph->wgt[sp], ph->KEa, S[sp].cp, S[sp].ci, S[sp].cv, ph->ratios[0],
+                    ph->ratios[1], ph->part[sp]);
+    }
+    launch_ph_exc_finish(s, nb, S[0].nunique, ph_exc_groups(S[0].nel, na, K),
+                         ph_exc_groups(S[1].nel, na, K), ph->E0, ph->wgt[0], ph->part[0],
+                         ph->part[1], ph->log_ov, d_E + 6L * w0, d_ov + 2L * w0);
   }
 }
 
@@ -292,9 +325,14 @@ void ph_energy_all(afq_ph_t* ph, hipStream_t s, int nw, const double* d_wbuf, lo
       ph_energy_alg0(ph, s, nw, d_wbuf, ldw, d_E, d_ov);
       return;
     }
+    if (ph->staged) {
+      ph_energy_staged(ph, s, nw, d_wbuf, ldw, d_E, d_ov);
+      return;
+    }
+    // S and B of one vector do not fit LDS: determinant by determinant from the compact R matrices
     const int nmo = ph->nmo, na = ph->nact, K = ph->nchol;
     Spin* S = ph->spin;
-    const int nu = S[0].nunique, nd = S[1].nunique;
+    const int nd = S[1].nunique;
     for (int w0 = 0; w0 < nw; w0 += ph->wblock) {
       const int nb = std::min(ph->wblock, nw - w0);
       const double* Phi[2] = {d_wbuf + 2 * (long)w0 * ldw,
@@ -303,8 +341,7 @@ void ph_energy_all(afq_ph_t* ph, hipStream_t s, int nw, const double* d_wbuf, lo
       // 1. reference G, log overlap, QQ0 and the excitation overlap ratios of both spins
       ph_overlaps_block(ph, s, nb, Phi, ldw);
       // 2a. weights and the multi-determinant overlap
-      launch_ph_spin_weights(s, nb, nu, S[0].cp, S[0].ci, S[0].cv, ph->ratios[0], ph->ratios[1],
-                             ph->wgt[0], ph->Ov);
+      ph_weights_block(ph, s, nb, 0, ph->Ov);
       // 3a. reference energy of the up spin (KE row 0 = its Cholesky trace), times Ov
       launch_ph_reference_energy(s, nb, S[0].nel, nmo, K, na, 1.0, ph->E0, ph->G[0], S[0].Lna,
                                  S[0].haj, ph->Eref, ph->KEa, ph->Twina, ph->Swia);
@@ -329,8 +366,7 @@ void ph_energy_all(afq_ph_t* ph, hipStream_t s, int nw, const double* d_wbuf, lo
       launch_ph_couple_ke(s, nb, K, nd, S[1].cp, S[1].ci, S[1].cv, ph->ratios[0], ph->KEa,
                           ph->ratios[1], ph->KEb);
       // 2b. weights of the down determinants
-      launch_ph_spin_weights(s, nb, nd, S[1].cp, S[1].ci, S[1].cv, ph->ratios[1], ph->ratios[0],
-                             ph->wgt[1], ph->Ov2);
+      ph_weights_block(ph, s, nb, 1, nullptr);
       // 3b. reference energy of the down spin (E0 only with the up spin), the cross term
       launch_ph_reference_energy(s, nb, S[1].nel, nmo, K, na, 1.0, 0.0, ph->G[1], S[1].Lna,
                                  S[1].haj, ph->Eref, ph->KEa, ph->Twina, ph->Swia);
@@ -359,17 +395,26 @@ void ph_energy_all(afq_ph_t* ph, hipStream_t s, int nw, const double* d_wbuf, lo
     }
 }
 
-// PHMSD::vbias over all walkers, in walker blocks
+long ph_vec_size(const afq_ph_t* ph) {
+  return ph->fold ? (long)ph->nmo * (ph->nmo + 1) / 2 : (long)ph->nmo * ph->nmo;
+}
+
+// PHMSD::vbias over all walkers, in walker blocks: sqrt(dt) sum_lk L_n[l][k] F[l][k] with the
+// spin-summed density F in the orbital basis (folded onto l <= k for symmetric vectors), an eighth
+// to a sixteenth of the products that the half-rotated vectors of both spins take
 void ph_vbias_all(afq_ph_t* ph, hipStream_t s, int nw, const double* d_wbuf, long ldw, double dt,
                   double* d_v) {
     const int nmo = ph->nmo, na = ph->nact, K = ph->nchol;
-    const int kx = 2 * na * nmo;
+    const long kx = ph_vec_size(ph);
+    Spin* S = ph->spin;
     for (int w0 = 0; w0 < nw; w0 += ph->wblock) {
       const int nb = std::min(ph->wblock, nw - w0);
       const double* Phi[2] = {d_wbuf + 2 * (long)w0 * ldw,
                               d_wbuf + 2 * ((long)w0 * ldw + (long)nmo * ph->spin[0].nel)};
-      ph_density_block(ph, s, nb, Phi, ldw, ph->Gblk, ph->Eref);   // log overlap unused
-      launch_gemm_nt_z(s, AFQ_FP64, nb, K, kx, std::sqrt(dt), ph->Gblk, kx, ph->Lstack, kx, true,
+      ph_expansion_block(ph, s, nb, Phi, ldw);
+      launch_ph_density(s, nb, S[0].nel, S[1].nel, na, nmo, ph->fold, ph->Rexp[0], S[0].A, ph->G[0],
+                        ph->Rexp[1], S[1].A, ph->G[1], ph->Ov, ph->RA[0], ph->RA[1], ph->F);
+      launch_gemm_nt_z(s, AFQ_FP64, nb, K, (int)kx, std::sqrt(dt), ph->F, kx, ph->Lvec, kx, false,
                        d_v + 2L * w0 * K, K, ph->split, ph->split_elems);
     }
 }
@@ -463,17 +508,29 @@ void ph_vmf(afq_ph_t* ph, hipStream_t st, double dt, double* d_vmf) {
         }
     }
     for (auto& g : G) g /= ov;
-    // 3. vbias of the mean-field density: sqrt(dt) sum_s sum_{a,k} Lna_s[n][a][k] G_s[a][k]
-    std::vector<double> flat(2 * G.size());
-    for (size_t e = 0; e < G.size(); ++e) {
-      flat[2 * e] = G[e].real();
-      flat[2 * e + 1] = G[e].imag();
-    }
-    AFQ_HIP(hipMemcpyAsync(ph->Gblk, flat.data(), flat.size() * sizeof(double),
+    // 3. vbias of the mean-field density: sqrt(dt) sum_s sum_{a,k} Lna_s[n][a][k] G_s[a][k], taken
+    // in the orbital basis, D[l][k] = sum_s sum_a A_s[a][l] G_s[a][k], as ph_vbias_all does
+    std::vector<zc> D((size_t)nmo * nmo, 0.0);
+    for (int s = 0; s < 2; ++s)
+      for (int a = 0; a < na; ++a)
+        for (int l = 0; l < nmo; ++l) {
+          const zc x = ph->spin[s].hA[(size_t)a * nmo + l];
+          const zc* g = G.data() + ((size_t)s * na + a) * nmo;
+          for (int k = 0; k < nmo; ++k) D[(size_t)l * nmo + k] += x * g[k];
+        }
+    std::vector<double> flat;
+    for (int l = 0; l < nmo; ++l)
+      for (int k = ph->fold ? l : 0; k < nmo; ++k) {
+        zc x = D[(size_t)l * nmo + k];
+        if (ph->fold && k > l) x += D[(size_t)k * nmo + l];
+        flat.push_back(x.real());
+        flat.push_back(x.imag());
+      }
+    AFQ_HIP(hipMemcpyAsync(ph->F, flat.data(), flat.size() * sizeof(double),
                            hipMemcpyHostToDevice, st));
-    const int kx = 2 * na * nmo;
-    launch_gemm_nt_z(st, AFQ_FP64, 1, ph->nchol, kx, std::sqrt(dt), ph->Gblk, kx, ph->Lstack, kx,
-                     true, d_vmf, ph->nchol);
+    const int kx = (int)ph_vec_size(ph);
+    launch_gemm_nt_z(st, AFQ_FP64, 1, ph->nchol, kx, std::sqrt(dt), ph->F, kx, ph->Lvec, kx, false,
+                     d_vmf, ph->nchol);
     AFQ_HIP(hipStreamSynchronize(st));
 }
 
@@ -487,8 +544,7 @@ void ph_overlap_all(afq_ph_t* ph, hipStream_t s, int nw, const double* d_wbuf, l
     const double* Phi[2] = {d_wbuf + 2 * (long)w0 * ldw,
                             d_wbuf + 2 * ((long)w0 * ldw + (long)nmo * S[0].nel)};
     ph_overlaps_block(ph, s, nb, Phi, ldw);
-    launch_ph_spin_weights(s, nb, S[0].nunique, S[0].cp, S[0].ci, S[0].cv, ph->ratios[0],
-                           ph->ratios[1], ph->wgt[0], ph->Ov);
+    ph_weights_block(ph, s, nb, 0, ph->Ov);
     launch_ph_log_overlap(s, nb, ph->Ov, ph->log_ov, d_ov + 2L * w0);
   }
 }
@@ -609,6 +665,39 @@ int afq_ph_create(int nmo, int nup, int ndn, int nchol, int ndet, const int* occ
         row += sh.ndet;
         max_nex = std::max(max_nex, n);
       }
+      {
+        std::vector<PhShell> tab;
+        for (const Shell& sh : S.shells) {
+          tab.push_back(PhShell{sh.nex, sh.ndet, sh.row, (int)S.qtot, sh.iexcit});
+          S.qtot += (long)sh.nex * sh.nex * sh.ndet;
+          S.maxdet = std::max(S.maxdet, sh.ndet);
+          S.maxnex = std::max(S.maxnex, sh.nex);
+        }
+        S.dshell = dev_copy(own, tab.data(), tab.size());
+        // per hole p and particle v the determinants and elements (e, q) of their Q with
+        // p_e = p, v_q = v, in determinant order
+        const int nvir = nmo - nel[s];
+        std::vector<std::vector<std::pair<int, int>>> lists((size_t)nel[s] * nvir);
+        for (const PhShell& sh : tab)
+          for (int d = 0; d < sh.ndet; ++d) {
+            const auto& x = unique[s][sh.nex][d];
+            for (int e = 0; e < sh.nex; ++e)
+              for (int q = 0; q < sh.nex; ++q)
+                lists[(size_t)x[e] * nvir + (x[sh.nex + q] - nel[s])].push_back(
+                    {sh.row + d, sh.qoff + (e * sh.nex + q) * sh.ndet + d});
+          }
+        std::vector<int> lp(1, 0), lu, lq;
+        for (const auto& l : lists) {
+          for (const auto& e : l) {
+            lu.push_back(e.first);
+            lq.push_back(e.second);
+          }
+          lp.push_back((int)lu.size());
+        }
+        S.rp = dev_copy(own, lp.data(), lp.size());
+        S.ru = dev_copy(own, lu.data(), lu.size());
+        S.rq = dev_copy(own, lq.data(), lq.size());
+      }
       S.nunique = row;
       S.confs.assign(1, std::vector<int>());
       for (int k = 0; k < nel[s]; ++k) S.confs[0].push_back(ref[s][k] - s * nmo);
@@ -669,19 +758,19 @@ int afq_ph_create(int nmo, int nup, int ndn, int nchol, int ndet, const int* occ
       const double* ho = orbmats + (nref == 2 ? s : 0) * 2 * nmm;
       S.hA.resize(nmm);
       for (size_t e = 0; e < nmm; ++e) S.hA[e] = {ho[2 * e], ho[2 * e + 1]};
-      S.Lna = dev_alloc<double>(own, 2 * nmm * nchol);
-      S.haj = dev_alloc<double>(own, 2 * nmm);
+      S.Lna = dev_alloc<double>(own, 2 * nmm * (nchol + 1));
+      S.haj = S.Lna + 2 * nmm * nchol;
       launch_half_rotate(st, nmo, nmo, nchol, S.A, dh, dL, S.haj, S.Lna);
+      bool real = true;
+      for (size_t e = 0; e < nmm; ++e) real = real && ho[2 * e + 1] == 0.0;
+      if (real) {
+        S.Lna_r = dev_alloc<double>(own, nmm * (nchol + 1));
+        launch_real_rows(st, (long)nmo * (nchol + 1), nmo, nmo, S.Lna, S.Lna_r);
+      }
     }
-    {
-      double* stackA = dev_alloc<double>(own, 4 * nmm);
-      AFQ_HIP(hipMemcpy(stackA, P->spin[0].A, 2 * nmm * sizeof(double), hipMemcpyDeviceToDevice));
-      AFQ_HIP(hipMemcpy(stackA + 2 * nmm, P->spin[1].A, 2 * nmm * sizeof(double),
-                        hipMemcpyDeviceToDevice));
-      P->Lstack = dev_alloc<double>(own, 4 * nmm * nchol);
-      double* hstack = dev_alloc<double>(own, 4 * nmm);
-      launch_half_rotate(st, nmo, 2 * nmo, nchol, stackA, dh, dL, hstack, P->Lstack);
-    }
+    P->fold = likn_symmetric(st, nmo, nchol, dL);
+    P->Lvec = dev_alloc<double>(own, (size_t)ph_vec_size(P.get()) * nchol);
+    launch_ph_rows_of_vectors(st, nmo, nchol, P->fold, dL, P->Lvec);
     AFQ_HIP(hipStreamSynchronize(st));
     // --- workspace for one walker block
     const long nb = walker_block, K = nchol, na = nmo;
@@ -696,25 +785,31 @@ int afq_ph_create(int nmo, int nup, int ndn, int nchol, int ndet, const int* occ
       P->QQ0[s] = dev_alloc<double>(own, 2 * nb * na * nel[s]);
       P->ratios[s] = dev_alloc<double>(own, 2 * nb * P->spin[s].nunique);
       P->wgt[s] = dev_alloc<double>(own, 2 * nb * P->spin[s].nunique);
+      P->Q[s] = dev_alloc<double>(own, 2 * nb * P->spin[s].qtot);
+      P->Rexp[s] = dev_alloc<double>(own, 2 * nb * nel[s] * na);
+      P->RA[s] = dev_alloc<double>(own, 2 * nb * nel[s] * nmo);
+      P->part[s] = dev_alloc<double>(own, 16L * nb * ph_exc_groups(nel[s], (int)na, nchol));
     }
-    P->work = dev_alloc<double>(own, 2L * maxel * nmo);
+    P->staged = ph_exc_vectors(nup, (int)na) > 0 && ph_exc_vectors(ndn, (int)na) > 0;
+    P->F = dev_alloc<double>(own, 2 * nb * ph_vec_size(P.get()));
     P->Ov = dev_alloc<double>(own, 2 * nb);
     P->Ov2 = dev_alloc<double>(own, 2 * nb);
     P->log_ov = dev_alloc<double>(own, 2 * nb);
     P->Eref = dev_alloc<double>(own, 6 * nb);
     P->Ex = dev_alloc<double>(own, 6 * nb);
     P->acc = dev_alloc<double>(own, 6 * nb);
-    P->Twina = dev_alloc<double>(own, 2 * nb * maxel * K * na);
+    P->Twina = dev_alloc<double>(own, 2 * nb * maxel * (K + 1) * na);
     P->Swia = dev_alloc<double>(own, 2 * nb * maxel * na);
     P->KEa = dev_alloc<double>(own, 2L * maxu * nb * K);
     P->KEb = dev_alloc<double>(own, 2L * maxu * nb * K);
-    P->KEl = dev_alloc<double>(own, 2 * std::max(dblk, 1L) * nb * K);
-    P->R = dev_alloc<double>(own, 2 * nb * dblk * max_nex * na);
-    P->Racc = dev_alloc<double>(own, 2 * nb * maxel * na);
+    if (!P->staged) {
+      P->KEl = dev_alloc<double>(own, 2 * std::max(dblk, 1L) * nb * K);
+      P->R = dev_alloc<double>(own, 2 * nb * dblk * max_nex * na);
+    }
     P->Gblk = dev_alloc<double>(own, 2 * nb * 2 * na * nmo);
     P->Emsd = dev_alloc<double>(own, 16L * maxu * nb);
     if (maxel <= 32) P->Tinv0 = dev_alloc<double>(own, 2L * maxu * nb * maxel * maxel);
-    P->p2ws_doubles = ph_2body_workspace((int)nb, (int)na, maxel, (int)K);
+    if (!P->staged) P->p2ws_doubles = ph_2body_workspace((int)nb, (int)na, maxel, (int)K);
     if (P->p2ws_doubles > 0) P->p2ws = dev_alloc<double>(own, P->p2ws_doubles);
     P->split_elems = (long)kMaxSplits * nb * K;
     P->split = dev_alloc<double>(own, 2 * P->split_elems);

@@ -1067,6 +1067,19 @@ void launch_ph_1body(hipStream_t s, int nw, int ndet, int nex, int nact, int nel
   AFQ_HIP(hipGetLastError());
 }
 
+void launch_ph_reference_G(hipStream_t s, int nb, int nmo, int nel, int nact, const double* A,
+                           const double* Aref, const double* Phi, long ldw, double* G, double* ov,
+                           double* QQ0) {
+  if (nb <= 0) return;
+  // T = A[ref] Phi, log det accumulated into ov (wrapped), G = T^-T Phi^T
+  launch_green(s, nb, nmo, nel, Aref, Phi, ldw, G, ov, 2, 1.0, cd{0.0, 0.0}, nullptr, 0.0, 0.0,
+               nullptr, 0);
+  hipLaunchKernelGGL(k_ph_qq0, dim3((unsigned)(((long)nb * nact * nel + 255) / 256)), dim3(256),
+                     0, s, nb, nmo, nel, nact, reinterpret_cast<const cd*>(A),
+                     reinterpret_cast<const cd*>(G), reinterpret_cast<cd*>(QQ0));
+  AFQ_HIP(hipGetLastError());
+}
+
 void launch_ph_woodbury(hipStream_t s, int nb, int nmo, int nel, int nact, const double* A,
                         const int* ref, const double* Phi, long ldw, double* G, double* ov,
                         double* QQ0, double* work) {
@@ -1075,13 +1088,7 @@ void launch_ph_woodbury(hipStream_t s, int nb, int nmo, int nel, int nact, const
                      0, s, nel, nmo, nact, ref, reinterpret_cast<const cd*>(A),
                      reinterpret_cast<cd*>(work));
   AFQ_HIP(hipGetLastError());
-  // T = A[ref] Phi, log det accumulated into ov (wrapped), G = T^-T Phi^T
-  launch_green(s, nb, nmo, nel, work, Phi, ldw, G, ov, 2, 1.0, cd{0.0, 0.0}, nullptr, 0.0, 0.0,
-               nullptr, 0);
-  hipLaunchKernelGGL(k_ph_qq0, dim3((unsigned)(((long)nb * nact * nel + 255) / 256)), dim3(256),
-                     0, s, nb, nmo, nel, nact, reinterpret_cast<const cd*>(A),
-                     reinterpret_cast<const cd*>(G), reinterpret_cast<cd*>(QQ0));
-  AFQ_HIP(hipGetLastError());
+  launch_ph_reference_G(s, nb, nmo, nel, nact, A, work, Phi, ldw, G, ov, QQ0);
 }
 
 void launch_ph_spin_weights(hipStream_t s, int nw, int nu, const int* cp, const int* ci,
@@ -1253,7 +1260,8 @@ void launch_ph_log_overlap(hipStream_t s, int nw, const double* Ov, const double
 // k_ph0_config; Phi_w = Phi + w ldw (c128 [nmo][nel]).
 void launch_ph0_products(hipStream_t s, int nw, int nmo, int nel, int nact, int nchol,
                          const double* Phi, long ldw, const double* A, const double* haj,
-                         const double* Lna, double* Phit, double* TAB, double* Hp, double* P) {
+                         const double* Lna, bool lna_complex, double* Phit, double* TAB,
+                         double* Hp, double* P) {
   if (nw <= 0) return;
   hipLaunchKernelGGL(k_ph0_transpose, dim3((unsigned)(((long)nel * nmo + 255) / 256), nw),
                      dim3(256), 0, s, nmo, nel, reinterpret_cast<const cd*>(Phi), ldw,
@@ -1261,8 +1269,8 @@ void launch_ph0_products(hipStream_t s, int nw, int nmo, int nel, int nact, int 
   AFQ_HIP(hipGetLastError());
   launch_gemm_nt_z(s, AFQ_FP64, nw * nel, nact, nmo, 1.0, Phit, nmo, A, nmo, true, TAB, nact);
   launch_gemm_nt_z(s, AFQ_FP64, nw * nel, nact, nmo, 1.0, Phit, nmo, haj, nmo, true, Hp, nact);
-  launch_gemm_nt_z(s, AFQ_FP64, nw * nel, nchol * nact, nmo, 1.0, Phit, nmo, Lna, nmo, true, P,
-                   (long)nchol * nact);
+  launch_gemm_nt_z(s, AFQ_FP64, nw * nel, nchol * nact, nmo, 1.0, Phit, nmo, Lna, nmo,
+                   lna_complex, P,                   (long)nchol * nact);
 }
 
 void launch_ph0_config(hipStream_t s, int nw, int nc, int nel, int nact, int nchol,

@@ -100,6 +100,16 @@ __global__ void k_zgemm_small(int n, double alpha, const cd* __restrict__ A,
   C[e] = s;
 }
 
+// flag = 1 if any L[i][j][n] differs from L[j][i][n] (one workgroup per i < j pair)
+__global__ void k_asymmetric(int M, int K, const double* __restrict__ Likn, int* __restrict__ flag) {
+  const int i = blockIdx.x, j = blockIdx.y;
+  if (j <= i) return;
+  bool diff = false;
+  for (int n = threadIdx.x; n < K; n += blockDim.x)
+    diff |= !(Likn[((long)i * M + j) * K + n] == Likn[((long)j * M + i) * K + n]);
+  if (diff) *flag = 1;
+}
+
 __global__ void k_real_rows(long rows, int M, int ld, const cd* __restrict__ src,
                             double* __restrict__ dst) {
   const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -130,6 +140,24 @@ void launch_half_rotate(hipStream_t s, int M, int N, int K, const double* PsiT, 
 void launch_v0(hipStream_t s, int M, int K, const double* Likn, double* v0) {
   hipLaunchKernelGGL(k_v0, blocks((long)M * M), dim3(256), 0, s, M, K, Likn, v0);
   AFQ_HIP(hipGetLastError());
+}
+
+bool likn_symmetric(hipStream_t s, int M, int K, const double* Likn) {
+  int* flag = nullptr;
+  AFQ_HIP(hipMalloc(&flag, sizeof(int)));
+  int host = 1;
+  try {
+    AFQ_HIP(hipMemsetAsync(flag, 0, sizeof(int), s));
+    hipLaunchKernelGGL(k_asymmetric, dim3(M, M), dim3(128), 0, s, M, K, Likn, flag);
+    AFQ_HIP(hipGetLastError());
+    AFQ_HIP(hipMemcpyAsync(&host, flag, sizeof(int), hipMemcpyDeviceToHost, s));
+    AFQ_HIP(hipStreamSynchronize(s));
+  } catch (...) {
+    (void)hipFree(flag);
+    throw;
+  }
+  AFQ_HIP(hipFree(flag));
+  return host == 0;
 }
 
 void launch_real_rows(hipStream_t s, long rows, int M, int ld, const double* src, double* dst) {
