@@ -116,6 +116,10 @@ void run_vbias(afq_ham H, hipStream_t s, int W, const double* G, double* v, int 
   if (H->precision == AFQ_BF16X3)
     launch_gemm_bf16(s, W, H->K, (int)NM, alpha, G, NM, H->Lnak_g, true, v, H->K, H->ws.split,
                      H->ws.split_elems);
+  else if (H->real_trial)
+    launch_gemm_real(s, H->precision, W, H->K, (int)NM, alpha, G, NM,
+                     H->precision == AFQ_FP64 ? (const void*)H->Lvb_d : (const void*)H->Lvb_f, v,
+                     H->K, true, H->ws.split, H->ws.split_elems, cfg);
   else
     launch_gemm_nt_z(s, H->precision, W, H->K, (int)NM, alpha, G, NM, L_for(H), NM, true, v,
                      H->K, H->ws.split, H->ws.split_elems, cfg);
@@ -129,6 +133,22 @@ void run_vhs(afq_ham H, hipStream_t s, int W, const double* X, double* V, int cf
     launch_gemm_nt_z(s, H->precision, W, MM, H->K, std::sqrt(H->dt), X, H->K, Likn_for(H),
                      H->K, false, V, MM, nullptr, 0, cfg);
 }
+
+// vHS for the walkers' propagation: the upper triangle only when the Cholesky vectors are symmetric
+VKind run_vhs_step(afq_ham H, hipStream_t s, int W, const double* X, double* V, int cfg) {
+  const int precision = H->precision;
+  if (!H->sym || precision == AFQ_BF16X3) {
+    run_vhs(H, s, W, X, V, cfg);
+    return VKind::full;
+  }
+  const int np = H->M * (H->M + 1) / 2;
+  launch_gemm_real(s, precision, W, np, H->K, std::sqrt(H->dt), X, H->K,
+                   precision == AFQ_FP64 ? (const void*)H->Lp_d : (const void*)H->Lp_f, V, np, false,
+                   nullptr, 0, cfg);
+  return VKind::packed;
+}
+
+const double* P1r_of(afq_ham H) { return H->P1_real ? H->P1r : nullptr; }
 
 // the exchange contraction in the handle's precision: Kl and per-chunk tr(T^2) partials
 void run_exchange(afq_ham H, hipStream_t s, int W, const double* G) {
@@ -250,6 +270,7 @@ int afq_ham_create(int M, int N, int K, const double* h_h, const double* h_Likn,
       dalloc(&H->H1, 2 * MM);
       dalloc(&H->Lnak_f, 2 * NM * K);
       dalloc(&H->Likn_f, MM * K);
+      dalloc(&H->P1r, 2 * MM);
       dalloc(&H->stats, 7);
       AFQ_HIP(hipMemcpy(H->PsiT, h_PsiT, 2 * NM * sizeof(double), hipMemcpyHostToDevice));
       AFQ_HIP(hipMemcpy(H->Likn, h_Likn, MM * K * sizeof(double), hipMemcpyHostToDevice));
@@ -261,6 +282,18 @@ int afq_ham_create(int M, int N, int K, const double* h_h, const double* h_Likn,
       if (H->real_trial) {
         dalloc(&H->Lnak_r, (size_t)K * N * real_lnak_row(M));
         launch_real_rows(nullptr, (long)K * N, M, real_lnak_row(M), H->Lnak, H->Lnak_r);
+        dalloc(&H->Lvb_d, (size_t)K * gemm_real_row((int)NM));
+        dalloc(&H->Lvb_f, (size_t)K * gemm_real_row((int)NM));
+        launch_pad_rows(nullptr, K, (int)NM, 0, H->Lnak, true, H->Lvb_d);
+        launch_pad_rows(nullptr, K, (int)NM, 0, H->Lnak, true, H->Lvb_f);
+      }
+      H->sym = likn_symmetric(nullptr, M, K, H->Likn);
+      if (H->sym) {
+        const long np = (long)M * (M + 1) / 2;
+        dalloc(&H->Lp_d, (size_t)np * gemm_real_row(K));
+        dalloc(&H->Lp_f, (size_t)np * gemm_real_row(K));
+        launch_pad_rows(nullptr, np, K, M, H->Likn, false, H->Lp_d);
+        launch_pad_rows(nullptr, np, K, M, H->Likn, false, H->Lp_f);
       }
       if (exchange_bf16_supported(M, N)) {
         dalloc(&H->Lnak_b, exchange_bf16_elems(M, N, K));
@@ -301,6 +334,11 @@ int afq_ham_destroy(afq_ham H) {
     dfree(H->P1);
     dfree(H->H1);
     dfree(H->Lnak_r);
+    dfree(H->P1r);
+    dfree(H->Lvb_d);
+    dfree(H->Lvb_f);
+    dfree(H->Lp_d);
+    dfree(H->Lp_f);
     dfree(H->Lnak_f);
     dfree(H->Likn_f);
     dfree(H->Lnak_ord);
@@ -517,7 +555,7 @@ int afq_autotune(afq_ham H, int W, const char* cache_path, int* cfg_out, void* s
     H->cfg_vbias = tune(key("vbias", K, NM), true,
                         [&](int c) { run_vbias(H, s, W, ws.G, ws.X, c); });
     H->cfg_vhs = tune(key("vhs", (long)M * M, K), false,
-                      [&](int c) { run_vhs(H, s, W, ws.X, ws.V, c); });
+                      [&](int c) { run_vhs_step(H, s, W, ws.X, ws.V, c); });
     AFQ_HIP(hipStreamSynchronize(s));
     write_tile_cache(cache_path, cache);
     if (cfg_out) {
@@ -567,7 +605,7 @@ int afq_det_propagate(int nb, int M, int N, double* Phi, long ldw, const double*
   return guard([&] {
     AFQ_CHECK(nb >= 0 && M > 0 && N >= 0 && N <= M, AFQ_EBADSHAPE, "bad shape");
     AFQ_CHECK(order >= 0, AFQ_EINVAL, "negative Taylor order");
-    launch_propagate(S(stream), nb, M, N, Phi, ldw, P1, V, order);
+    launch_propagate(S(stream), nb, M, N, Phi, ldw, P1, nullptr, V, VKind::full, order);
   });
 }
 
@@ -653,7 +691,8 @@ int afq_propagate(afq_ham H, int W, double* wbuf, long ldw, const double* V, voi
   return guard([&] {
     check_ham(H);
     check_walkers(H, W, ldw);
-    launch_propagate(S(stream), W, H->M, H->N, wbuf, ldw, H->P1, V, H->params.taylor_n);
+    launch_propagate(S(stream), W, H->M, H->N, wbuf, ldw, H->P1, P1r_of(H), V, VKind::full,
+                     H->params.taylor_n);
   });
 }
 
@@ -702,13 +741,14 @@ int afq_step(afq_ham H, int W, double* wbuf, long ldw, const double* xi, double 
         launch_store_fields(s, W, K, ws.X, H->fields, H->nfields, H->hist_pos);
     }
     // 3. vHS = sqrt(dt) L X           4. Phi <- P1 exp(iV) P1 Phi
+    VKind kind = VKind::full;
     {
       RegionScope r(tm, s, R_VHS);
-      run_vhs(H, s, W, ws.X, ws.V, H->cfg_vhs);
+      kind = run_vhs_step(H, s, W, ws.X, ws.V, H->cfg_vhs);
     }
     {
       RegionScope r(tm, s, R_PROPAGATE);
-      launch_propagate(s, W, M, N, wbuf, ldw, H->P1, ws.V, p.taylor_n);
+      launch_propagate(s, W, M, N, wbuf, ldw, H->P1, P1r_of(H), ws.V, kind, p.taylor_n);
     }
     // 5. new overlap (hybrid) or local energy
     if (p.hybrid) {
@@ -821,14 +861,25 @@ int afq_back_propagate(afq_ham H, int W, int nbpsteps, int nstabilize, double* d
     for (int ni = nbpsteps - 1; ni >= 0; --ni) {
       // newest entry first: the position already points at the next step's slot
       slot = slot == 0 ? nf - 1 : slot - 1;
-      // vHS = sqrt(dt) L X of the stored fields (FP64), then V <- -V^H
-      launch_gemm_nt_z(s, AFQ_FP64, W, MM, K, std::sqrt(H->dt), H->fields + 2L * slot * K,
-                       (long)nf * K, H->Likn, K, false, H->ws.V, MM);
-      launch_neg_adjoint(s, W, M, H->ws.V);
+      // vHS = sqrt(dt) L X of the stored fields (FP64), applied as -V^H: a symmetric V needs only
+      // the signs of its real parts changed, which the propagation does as it reads it
+      const double* X = H->fields + 2L * slot * K;
+      VKind kind = VKind::full;
+      if (H->sym) {
+        const int np = M * (M + 1) / 2;
+        launch_gemm_real(s, AFQ_FP64, W, np, K, std::sqrt(H->dt), X, (long)nf * K, H->Lp_d, H->ws.V,
+                         np, false);
+        kind = VKind::packed_adjoint;
+      } else {
+        launch_gemm_nt_z(s, AFQ_FP64, W, MM, K, std::sqrt(H->dt), X, (long)nf * K, H->Likn, K, false,
+                         H->ws.V, MM);
+        launch_neg_adjoint(s, W, M, H->ws.V);
+      }
       for (int nr = 0; nr < nrefs; ++nr) {
         double* Phi = d_refs + 2L * nr * NM;
         const long ld = (long)nrefs * NM;
-        launch_propagate(s, W, M, N, Phi, ld, H->P1H, H->ws.V, H->params.taylor_n);
+        launch_propagate(s, W, M, N, Phi, ld, H->P1H, H->P1_real ? H->P1r + MM : nullptr, H->ws.V,
+                         kind, H->params.taylor_n);
         if (ni == 0 || ni % nstabilize == 0) {
           launch_ph_fill(s, W, 0.0, 0.0, H->bp_ldet);
           launch_orthogonalize(s, W, M, N, Phi, ld, H->bp_ldet);

@@ -169,6 +169,13 @@ struct afq_ham_s {
   double* P1 = nullptr;      // c128 [M][M]
   double* H1 = nullptr;      // c128 [M][M]
   bool real_trial = false;   // every imaginary part of PsiT is zero (so is Im Lnak)
+  bool sym = false;          // Likn[i][j] == Likn[j][i]: V_w is symmetric and kept as a triangle
+  double* P1r = nullptr;     // f64 [2][M][M]: P1 and its transpose, when P1 is real
+  bool P1_real = false;
+  double* Lvb_d = nullptr;   // f64 [K][N*M padded to 16]: real Lnak rows (vbias of a real trial)
+  float* Lvb_f = nullptr;    // f32 copy
+  double* Lp_d = nullptr;    // f64 [M(M+1)/2][K padded to 16]: rows i <= j of Likn (symmetric vHS)
+  float* Lp_f = nullptr;     // f32 copy
   double* Lnak_r = nullptr;  // f64 [K][N][M padded to 16]: Re Lnak, only with a real trial
   float* Lnak_f = nullptr;   // c64 [K][N][M]   (FP32 contraction copies)
   float* Likn_f = nullptr;   // f32 [M*M][K]
@@ -216,6 +223,19 @@ void launch_gemm_nt_z(hipStream_t s, int precision, int m, int n, int k, double 
                       const double* A, long lda, const void* B, long ldb, bool b_complex,
                       double* C, long ldc, double* split_ws = nullptr, long split_ws_elems = 0,
                       int cfg = 0);
+// k_gemm_real.hip: the same product with a real B, rows zero-padded to gemm_real_row(k) elements (f64
+// for AFQ_FP64, else f32). nanmix: an Inf or NaN in A makes both parts of its row's sums NaN, as the
+// zero imaginary part of a complex B does. FP32 gives launch_gemm_nt_z's bits.
+int gemm_real_row(int k);
+// padded rows dst[row][0..gemm_real_row(k)) = src[row][0..k) (the real part of a complex src);
+// packed_n > 0: the packed_n (packed_n + 1) / 2 rows i <= j of the n x n rows of src
+void launch_pad_rows(hipStream_t s, long rows, int k, int packed_n, const double* src, bool complex_src,
+                     double* dst);
+void launch_pad_rows(hipStream_t s, long rows, int k, int packed_n, const double* src, bool complex_src,
+                     float* dst);
+void launch_gemm_real(hipStream_t s, int precision, int m, int n, int k, double alpha,
+                      const double* A, long lda, const void* B, double* C, long ldc, bool nanmix,
+                      double* split_ws = nullptr, long split_ws_elems = 0, int cfg = 0);
 // k_energy.hip
 int device_cus();                        // compute units of the current device (cached)
 int exx_nchunks(int W, int N, int K);   // chunks of Cholesky vectors the exchange kernel uses
@@ -265,8 +285,14 @@ void launch_energy_finalize(hipStream_t s, int W, int K, int nchunk, int walker_
 void launch_e1(hipStream_t s, int W, int M, int N, const double* G, const double* haj,
                double E0, double scl, double* E);
 // k_propagate.hip
+enum class VKind {
+  full,          // V_w [M][M]
+  packed,        // its upper triangle, row by row (symmetric V)
+  packed_adjoint // the same, applied as -V^H
+};
+// P1r: the real P1 as f64 [M][M], NULL when P1 is complex
 void launch_propagate(hipStream_t s, int nb, int M, int N, double* Phi, long ldw,
-                      const double* P1, const double* V, int order);
+                      const double* P1, const double* P1r, const double* V, VKind kind, int order);
 // k_qr.hip
 void launch_orthogonalize(hipStream_t s, int nb, int M, int N, double* Phi, long ldw,
                           double* logdetR);
@@ -320,7 +346,7 @@ void launch_zero_imag(hipStream_t s, int n, double* v);
 void sparsify_one_body_propagator(int M, double* P);
 void build_one_body_propagator(hipStream_t s, int M, int K, double dt, const double* h,
                                const double* v0, const double* Likn, const double* vMF,
-                               double* H1, double* P1);
+                               double* H1, double* P1, double* P1r, bool* real);
 // k_phmsd.hip
 // ws: ph_2body_workspace() doubles for the staged kernel (NULL or too small: the per-walker one)
 long ph_2body_workspace(int nw, int nact, int nelec, int nchol);
@@ -407,8 +433,8 @@ void launch_ph_density(hipStream_t s, int nw, int nup, int ndn, int nact, int nm
                        const double* R0, const double* A0, const double* G0, const double* R1,
                        const double* A1, const double* G1, const double* ov, double* U0, double* U1,
                        double* F);
-void launch_ph_rows_of_vectors(hipStream_t s, int nmo, int nchol, bool fold, const double* Likn,
-                               double* out);
+void launch_ph_rows_of_vectors(hipStream_t s, int nmo, int nchol, bool fold, int ld,
+                               const double* Likn, double* out);
 void launch_ph_accumulate_R(hipStream_t s, int nw, int ndet, int nex, int nact, int nelec,
                             const int* iexcit, const int* refc, const double* Rc,
                             const double* ov, const double* wgt, double* R);

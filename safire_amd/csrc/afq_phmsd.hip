@@ -55,7 +55,7 @@ struct Spin {
   int* refc = nullptr;             // [nel]
   double* Lna = nullptr;           // c128 [nchol + 1][nact][nmo]: Lna_n = A L_n, then haj
   double* haj = nullptr;           // c128 [nact][nmo]: the last vector of Lna
-  double* Lna_r = nullptr;         // f64 [nchol + 1][nact][nmo], only when the orbitals are real
+  double* Lna_r = nullptr;         // f64 [nchol + 1][nact][nmo padded to 16], only with real orbitals
   PhShell* dshell = nullptr;       // the shells on the GPU
   int maxdet = 0, maxnex = 0;
   long qtot = 0;                   // sum of nex^2 ndet: elements of Q per walker
@@ -157,7 +157,10 @@ struct afq_ph_t {
   afq::Spin spin[2];
   bool fold = false;               // Likn is symmetric: Lvec holds its rows l <= k
   bool staged = false;             // the energy runs on k_phmsd_exc.hip's kernels
-  double* Lvec = nullptr;          // f64 [nchol][nmo (nmo + 1) / 2 or nmo^2]: the vectors as rows
+  double* Lvec = nullptr;          // f64 [nchol][nmo (nmo + 1) / 2 or nmo^2, padded to 16]: the vectors as rows
+  double* Lp = nullptr;            // f64 [nmo (nmo + 1) / 2][nchol padded to 16] (fold): rows l <= k
+  double* P1r = nullptr;           // f64 [2][nmo][nmo]: P1 and its transpose, when P1 is real
+  bool P1_real = false;
   double* h = nullptr;             // f64 [nmo][nmo]
   double* Likn = nullptr;          // f64 [nmo * nmo][nchol]
   // propagator state (afq_ph_prepare) and the step's per-walker workspace
@@ -305,9 +308,13 @@ void ph_energy_staged(afq_ph_t* ph, hipStream_t s, int nw, const double* d_wbuf,
     ph_overlaps_block(ph, s, nb, Phi, ldw);
     for (int sp = 0; sp < 2; ++sp) ph_weights_block(ph, s, nb, sp, nullptr);
     for (int sp = 0; sp < 2; ++sp) {
-      launch_gemm_nt_z(s, AFQ_FP64, nb * S[sp].nel, (K + 1) * na, nmo, 1.0, ph->G[sp], nmo,
-                       S[sp].Lna_r ? S[sp].Lna_r : S[sp].Lna, nmo, S[sp].Lna_r == nullptr,
-                       ph->Twina, (long)(K + 1) * na);
+      const int rows = nb * S[sp].nel, cols = (K + 1) * na;
+      if (S[sp].Lna_r)
+        launch_gemm_real(s, AFQ_FP64, rows, cols, nmo, 1.0, ph->G[sp], nmo, S[sp].Lna_r, ph->Twina,
+                         cols, true);
+      else
+        launch_gemm_nt_z(s, AFQ_FP64, rows, cols, nmo, 1.0, ph->G[sp], nmo, S[sp].Lna, nmo, true,
+                         ph->Twina, cols);
       launch_ph_exc(s, sp == 1, nb, S[sp].nel, na, K, S[sp].qtot, (int)S[sp].shells.size(),
                     S[sp].maxnex, S[sp].nunique, S[0].nunique, S[sp].dshell, ph->Twina, ph->QQ0[sp],
                     ph->Q[sp], ph->wgt[sp], ph->KEa, S[sp].cp, S[sp].ci, S[sp].cv, ph->ratios[0],
@@ -414,8 +421,8 @@ void ph_vbias_all(afq_ph_t* ph, hipStream_t s, int nw, const double* d_wbuf, lon
       ph_expansion_block(ph, s, nb, Phi, ldw);
       launch_ph_density(s, nb, S[0].nel, S[1].nel, na, nmo, ph->fold, ph->Rexp[0], S[0].A, ph->G[0],
                         ph->Rexp[1], S[1].A, ph->G[1], ph->Ov, ph->RA[0], ph->RA[1], ph->F);
-      launch_gemm_nt_z(s, AFQ_FP64, nb, K, (int)kx, std::sqrt(dt), ph->F, kx, ph->Lvec, kx, false,
-                       d_v + 2L * w0 * K, K, ph->split, ph->split_elems);
+      launch_gemm_real(s, AFQ_FP64, nb, K, (int)kx, std::sqrt(dt), ph->F, kx, ph->Lvec,
+                       d_v + 2L * w0 * K, K, false, ph->split, ph->split_elems);
     }
 }
 
@@ -529,8 +536,8 @@ void ph_vmf(afq_ph_t* ph, hipStream_t st, double dt, double* d_vmf) {
     AFQ_HIP(hipMemcpyAsync(ph->F, flat.data(), flat.size() * sizeof(double),
                            hipMemcpyHostToDevice, st));
     const int kx = (int)ph_vec_size(ph);
-    launch_gemm_nt_z(st, AFQ_FP64, 1, ph->nchol, kx, std::sqrt(dt), ph->F, kx, ph->Lvec, kx, false,
-                     d_vmf, ph->nchol);
+    launch_gemm_real(st, AFQ_FP64, 1, ph->nchol, kx, std::sqrt(dt), ph->F, kx, ph->Lvec, d_vmf,
+                     ph->nchol, false);
     AFQ_HIP(hipStreamSynchronize(st));
 }
 
@@ -764,13 +771,20 @@ int afq_ph_create(int nmo, int nup, int ndn, int nchol, int ndet, const int* occ
       bool real = true;
       for (size_t e = 0; e < nmm; ++e) real = real && ho[2 * e + 1] == 0.0;
       if (real) {
-        S.Lna_r = dev_alloc<double>(own, nmm * (nchol + 1));
-        launch_real_rows(st, (long)nmo * (nchol + 1), nmo, nmo, S.Lna, S.Lna_r);
+        S.Lna_r = dev_alloc<double>(own, (size_t)nmo * gemm_real_row(nmo) * (nchol + 1));
+        launch_pad_rows(st, (long)nmo * (nchol + 1), nmo, 0, S.Lna, true, S.Lna_r);
       }
     }
     P->fold = likn_symmetric(st, nmo, nchol, dL);
-    P->Lvec = dev_alloc<double>(own, (size_t)ph_vec_size(P.get()) * nchol);
-    launch_ph_rows_of_vectors(st, nmo, nchol, P->fold, dL, P->Lvec);
+    const int ldv = gemm_real_row((int)ph_vec_size(P.get()));
+    P->Lvec = dev_alloc<double>(own, (size_t)ldv * nchol);
+    AFQ_HIP(hipMemsetAsync(P->Lvec, 0, sizeof(double) * ldv * nchol, st));
+    launch_ph_rows_of_vectors(st, nmo, nchol, P->fold, ldv, dL, P->Lvec);
+    if (P->fold) {
+      const long np = (long)nmo * (nmo + 1) / 2;
+      P->Lp = dev_alloc<double>(own, (size_t)np * gemm_real_row(nchol));
+      launch_pad_rows(st, np, nchol, nmo, dL, false, P->Lp);
+    }
     AFQ_HIP(hipStreamSynchronize(st));
     // --- workspace for one walker block
     const long nb = walker_block, K = nchol, na = nmo;
@@ -916,6 +930,7 @@ int afq_ph_prepare(afq_ph ph, double dt, int W, void* stream) {
       ph->v0 = dev_alloc<double>(own, (size_t)M * M);
       ph->H1 = dev_alloc<double>(own, 2 * (size_t)M * M);
       ph->P1 = dev_alloc<double>(own, 2 * (size_t)M * M);
+      ph->P1r = dev_alloc<double>(own, 2 * (size_t)M * M);
       ph->stats = dev_alloc<unsigned long long>(own, 7);
       AFQ_HIP(hipMemset(ph->stats, 0, 7 * sizeof(unsigned long long)));
       afq_default_params(&ph->params);
@@ -925,7 +940,8 @@ int afq_ph_prepare(afq_ph ph, double dt, int W, void* stream) {
     ph_vmf(ph, s, dt, ph->vMF);
     launch_zero_imag(s, K, ph->vMF);
     launch_v0(s, M, K, ph->Likn, ph->v0);
-    build_one_body_propagator(s, M, K, dt, ph->h, ph->v0, ph->Likn, ph->vMF, ph->H1, ph->P1);
+    build_one_body_propagator(s, M, K, dt, ph->h, ph->v0, ph->Likn, ph->vMF, ph->H1, ph->P1,
+                              ph->P1r, &ph->P1_real);
     ph->dt = dt;
     if (W > ph->wcap) {
       const size_t w = (size_t)W;
@@ -976,11 +992,19 @@ int afq_ph_step(afq_ph ph, int W, double* d_wbuf, long ldw, const double* d_xi, 
     launch_construct_X(s, W, K, p.vbias_bound, p.use_cp_constraint || p.project_force_bias,
                        p.free_projection, ph->vMF, d_xi, ph->X, ph->HW, ph->mf);
     // 3. vHS = sqrt(dt) L X (Real3IndexFactorization::vHS), 4. both spins' Slater matrices
-    launch_gemm_nt_z(s, AFQ_FP64, W, M * M, K, std::sqrt(ph->dt), ph->X, K, ph->Likn, K, false,
-                     ph->V, (long)M * M);
-    launch_propagate(s, W, M, ph->spin[0].nel, d_wbuf, ldw, ph->P1, ph->V, p.taylor_n);
-    launch_propagate(s, W, M, ph->spin[1].nel, d_wbuf + 2L * M * ph->spin[0].nel, ldw, ph->P1,
-                     ph->V, p.taylor_n);
+    VKind kind = VKind::full;
+    if (ph->fold) {
+      const int np = M * (M + 1) / 2;
+      launch_gemm_real(s, AFQ_FP64, W, np, K, std::sqrt(ph->dt), ph->X, K, ph->Lp, ph->V, np, false);
+      kind = VKind::packed;
+    } else {
+      launch_gemm_nt_z(s, AFQ_FP64, W, M * M, K, std::sqrt(ph->dt), ph->X, K, ph->Likn, K, false,
+                       ph->V, (long)M * M);
+    }
+    const double* P1r = ph->P1_real ? ph->P1r : nullptr;
+    launch_propagate(s, W, M, ph->spin[0].nel, d_wbuf, ldw, ph->P1, P1r, ph->V, kind, p.taylor_n);
+    launch_propagate(s, W, M, ph->spin[1].nel, d_wbuf + 2L * M * ph->spin[0].nel, ldw, ph->P1, P1r,
+                     ph->V, kind, p.taylor_n);
     // 5. new overlap (hybrid) or local energy and overlap (PHMSD::energy)
     if (p.hybrid)
       ph_overlap_all(ph, s, W, d_wbuf, ldw, ph->ovw);

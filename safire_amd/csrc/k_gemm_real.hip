@@ -1,0 +1,268 @@
+// MFMA GEMM C[m][n] = alpha * sum_k A[m][k] * B[n][k] with complex A (c128) and a real B whose rows are
+// zero-padded to a multiple of 16 (ldb): the Cholesky contractions of a step whose vectors are real
+// (vHS, Real3IndexFactorization.hpp:297-313) or whose trial is (vbias, 350-361).
+//
+// A 256-thread workgroup owns a TM x TN tile of C, each wavefront TM/2 x TN/2 of it; a k slice (16
+// values, 8 for 128-row FP64 tiles) of A and B goes through LDS, double-buffered with one barrier per slice, in
+// 16-byte pieces: consecutive lanes load consecutive pieces of a row. Rows in LDS are padded to an odd
+// multiple of 16 bytes, so that the 16 rows of a fragment fall into different banks. FP32 converts A
+// when it is staged. Along a 16-wide chunk lane group g takes k = k0 + 4 g + s in step s (FP32), the
+// order of k_gemm_nt: both kernels give the same bits for the same split of k.
+//
+// Bound: MFMA. 128-row tiles take 10 LDS reads for 64 FP32 or 32 FP64 MFMAs (2048 matrix cycles) per
+// slice and wavefront; the 64 x 64 tiles of k_gemm_nt 8-byte reads of single elements for half as
+// many MFMAs, and twice the loads of B. Per launch, with the triangle of a symmetric vHS and the real
+// vectors of a real trial against k_gemm_nt on the full ones (M 128, N 32, K 640, 1024 walkers):
+// vHS FP64 905 -> 474 us, FP32 660 -> 288 us; vbias FP64 475 -> 227 us, FP32 277 -> 140 us. M 64,
+// N 16, K 320, 512 walkers, FP64: vHS 68 -> 46 us.
+#include "afq_internal.hpp"
+
+#include <algorithm>
+
+namespace afq {
+
+namespace {
+
+template <typename R, int TM, int TN, int KS>
+__global__ __launch_bounds__(256, 2) void k_gemm_real(int m, int n, int k, int kchunk, double alpha,
+                                                      const double* __restrict__ A, long lda,
+                                                      const R* __restrict__ B, long ldb,
+                                                      double* __restrict__ C, long ldc,
+                                                      long split_stride, int nanmix) {
+  typedef typename acc_of<R>::type acc_t;
+  constexpr bool F = sizeof(R) == 4;
+  constexpr int SPS = KS / 4;                    // MFMA k steps of a slice
+  constexpr int RA = KS * 2 * sizeof(R) + 16;    // staged row of A: an odd multiple of 16 bytes
+  constexpr int RB = KS * sizeof(R) + 16;        // staged row of B
+  static_assert(!F || KS == 16, "the FP32 sums keep 16-wide chunks");
+  constexpr int MT = TM / 32, NT = TN / 32;      // 16-wide tiles of a wavefront
+  constexpr int PA = TM * KS / 256;              // elements of A per thread and slice
+  constexpr int BP = KS * (int)sizeof(R) / 16;   // 16-byte pieces of a row of B
+  constexpr int PB = (TN * BP + 255) / 256;      // ... per thread and slice
+  __shared__ __attribute__((aligned(16))) char sA[2][TM * RA];
+  __shared__ __attribute__((aligned(16))) char sB[2][TN * RB];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int g = lane >> 4, r16 = lane & 15;
+  const int wm = (wave >> 1) * (TM / 2), wn = (wave & 1) * (TN / 2);
+  // column tiles fastest: consecutive workgroups (dealt round-robin to the XCDs) share rows of A,
+  // and each XCD's L2 holds an eighth of B
+  const int tile_n = blockIdx.x, tile_m = blockIdx.y;
+  const int kbeg = blockIdx.z * kchunk, kend = min(k, kbeg + kchunk);
+  C += blockIdx.z * split_stride;
+
+  double2 pa[PA];
+  uint4 pb[PB];
+  auto gload = [&](int k0) {
+#pragma unroll
+    for (int i = 0; i < PA; ++i) {
+      const int e = tid + 256 * i, row = e / KS, q = e % KS;
+      const int gm = tile_m * TM + row;
+      pa[i] = double2{0.0, 0.0};
+      if (gm < m && k0 + q < kend)
+        pa[i] = *reinterpret_cast<const double2*>(A + 2 * ((long)gm * lda + k0 + q));
+    }
+#pragma unroll
+    for (int i = 0; i < PB; ++i) {
+      const int e = tid + 256 * i, row = e / BP, q = e % BP;
+      const int gn = min(tile_n * TN + row, n - 1);
+      if (PB * 256 == TN * BP || row < TN)
+        pb[i] = *reinterpret_cast<const uint4*>(B + (long)gn * ldb + k0 + q * (16 / (int)sizeof(R)));
+    }
+  };
+  auto sstore = [&](int buf) {
+#pragma unroll
+    for (int i = 0; i < PA; ++i) {
+      const int e = tid + 256 * i, row = e / KS, q = e % KS;
+      R re = (R)pa[i].x, im = (R)pa[i].y;
+      if (nanmix) {   // the zero imaginary part of B in a complex product: Inf or NaN spreads
+        const R bad = (re - re) + (im - im);
+        re += bad;
+        im += bad;
+      }
+      R* p = reinterpret_cast<R*>(sA[buf] + row * RA) + 2 * q;
+      p[0] = re;
+      p[1] = im;
+    }
+#pragma unroll
+    for (int i = 0; i < PB; ++i) {
+      const int e = tid + 256 * i, row = e / BP, q = e % BP;
+      if (PB * 256 == TN * BP || row < TN)
+        *reinterpret_cast<uint4*>(sB[buf] + row * RB + 16 * q) = pb[i];
+    }
+  };
+
+  acc_t cr[MT][NT], ci[MT][NT];
+#pragma unroll
+  for (int a = 0; a < MT; ++a)
+#pragma unroll
+    for (int b = 0; b < NT; ++b) {
+      cr[a][b] = acc_t{0, 0, 0, 0};
+      ci[a][b] = acc_t{0, 0, 0, 0};
+    }
+  if (kbeg < kend) {
+    gload(kbeg);
+    sstore(0);
+  }
+  __syncthreads();
+  for (int k0 = kbeg, buf = 0; k0 < kend; k0 += KS, buf ^= 1) {
+    const bool more = k0 + KS < kend;
+    if (more) gload(k0 + KS);
+    R ar[MT][SPS], ai[MT][SPS], br[NT][SPS];
+    // lane group g: steps s = 0 .. SPS - 1 at k0 + SPS g + s, contiguous in its row
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      const char* p = sA[buf] + (wm + 16 * t + r16) * RA + g * SPS * 2 * (int)sizeof(R);
+#pragma unroll
+      for (int h = 0; h < (F ? SPS / 2 : SPS); ++h) {
+        if constexpr (F) {
+          const float4 x = reinterpret_cast<const float4*>(p)[h];
+          ar[t][2 * h] = x.x;
+          ai[t][2 * h] = x.y;
+          ar[t][2 * h + 1] = x.z;
+          ai[t][2 * h + 1] = x.w;
+        } else {
+          const double2 x = reinterpret_cast<const double2*>(p)[h];
+          ar[t][h] = x.x;
+          ai[t][h] = x.y;
+        }
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const char* p = sB[buf] + (wn + 16 * t + r16) * RB + g * SPS * (int)sizeof(R);
+      if constexpr (F) {
+        const float4 x = *reinterpret_cast<const float4*>(p);
+        br[t][0] = x.x;
+        br[t][1] = x.y;
+        br[t][2] = x.z;
+        br[t][3] = x.w;
+      } else {
+#pragma unroll
+        for (int h = 0; h < SPS / 2; ++h) {
+          const double2 x = reinterpret_cast<const double2*>(p)[h];
+          br[t][2 * h] = x.x;
+          br[t][2 * h + 1] = x.y;
+        }
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < SPS; ++s)
+#pragma unroll
+      for (int a = 0; a < MT; ++a)
+#pragma unroll
+        for (int b = 0; b < NT; ++b) {
+          cr[a][b] = mfma16x16x4(ar[a][s], br[b][s], cr[a][b]);
+          ci[a][b] = mfma16x16x4(ai[a][s], br[b][s], ci[a][b]);
+        }
+    // the other buffer was last read in the previous slice, before the barrier that ended it
+    if (more) sstore(buf ^ 1);
+    __syncthreads();
+  }
+#pragma unroll
+  for (int a = 0; a < MT; ++a)
+#pragma unroll
+    for (int b = 0; b < NT; ++b) {
+      const int col = tile_n * TN + wn + 16 * b + r16;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = tile_m * TM + wm + 16 * a + acc_row<R>(g, r);
+        if (row < m && col < n) {
+          const double2 v = double2{alpha * (double)cr[a][b][r], alpha * (double)ci[a][b][r]};
+          *reinterpret_cast<double2*>(C + 2 * ((long)row * ldc + col)) = v;
+        }
+      }
+    }
+}
+
+// Bp[row][0..ldb) = src[r(row)][0..k), zero-padded; packed: row p of the upper triangle i <= j of an
+// n x n set of rows is source row i n + j
+template <typename D>
+__global__ void k_pad_rows(long rows, int k, int ldb, int n, int packed,
+                           const double* __restrict__ src, int stride, D* __restrict__ dst) {
+  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= rows * ldb) return;
+  const long p = e / ldb;
+  const int c = (int)(e - p * ldb);
+  long r = p;
+  if (packed) {
+    // i: largest with i (2 n - i + 1) / 2 <= p
+    int i = (int)((2.0 * n + 1.0 - sqrt((2.0 * n + 1.0) * (2.0 * n + 1.0) - 8.0 * (double)p)) * 0.5);
+    i = max(0, min(i, n - 1));
+    while ((long)i * (2 * n - i + 1) / 2 > p) --i;
+    while (i + 1 < n && (long)(i + 1) * (2 * n - i) / 2 <= p) ++i;
+    r = (long)i * n + i + (p - (long)i * (2 * n - i + 1) / 2);
+  }
+  dst[e] = c < k ? (D)src[(r * k + c) * stride] : (D)0;
+}
+
+}  // namespace
+
+int gemm_real_row(int k) { return (k + 15) / 16 * 16; }
+
+void launch_pad_rows(hipStream_t s, long rows, int k, int packed_n, const double* src, bool complex_src,
+                     double* dst) {
+  const int ldb = gemm_real_row(k);
+  hipLaunchKernelGGL(k_pad_rows<double>, dim3((unsigned)((rows * ldb + 255) / 256)), dim3(256), 0, s,
+                     rows, k, ldb, packed_n, packed_n > 0 ? 1 : 0, src, complex_src ? 2 : 1, dst);
+  AFQ_HIP(hipGetLastError());
+}
+
+void launch_pad_rows(hipStream_t s, long rows, int k, int packed_n, const double* src, bool complex_src,
+                     float* dst) {
+  const int ldb = gemm_real_row(k);
+  hipLaunchKernelGGL(k_pad_rows<float>, dim3((unsigned)((rows * ldb + 255) / 256)), dim3(256), 0, s,
+                     rows, k, ldb, packed_n, packed_n > 0 ? 1 : 0, src, complex_src ? 2 : 1, dst);
+  AFQ_HIP(hipGetLastError());
+}
+
+void launch_gemm_real(hipStream_t s, int precision, int m, int n, int k, double alpha,
+                      const double* A, long lda, const void* B, double* C, long ldc, bool nanmix,
+                      double* split_ws, long split_ws_elems, int cfg) {
+  if (m <= 0 || n <= 0) return;
+  const bool f32 = precision != AFQ_FP64;
+  // the splits of launch_gemm_nt_z: the FP32 sums keep their order
+  int splits = split_ws ? gemm_splits(m, n, k) : 1;
+  if ((long)splits * m * n > split_ws_elems) splits = 1;
+  int kchunk = (k + splits - 1) / splits;
+  kchunk = (kchunk + 31) & ~31;
+  splits = std::max(1, (k + kchunk - 1) / kchunk);
+  // The largest tile that still gives two workgroups per CU (128 x 128 FP32: four, so that a partly
+  // filled last round costs little), else 64 x 32: 512 walkers of 64 orbitals are 264 64 x 64 tiles
+  // of vHS, one workgroup on most CUs with every load exposed.
+  // cfg (FP32; 0: this rule) bit 0: the other row count, bit 1: the other column count.
+  const long cus = device_cus();
+  auto tiles = [&](int tm, int tn) {
+    return (long)((m + tm - 1) / tm) * ((n + tn - 1) / tn) * splits;
+  };
+  int tm = 64, tn = 32;
+  if (f32 && tiles(128, 128) >= 4 * cus) tm = tn = 128;
+  else if (tiles(128, 64) >= 2 * cus) tm = 128, tn = 64;
+  else if (tiles(64, 64) >= 2 * cus) tn = 64;
+  if (f32 && (cfg & 1)) tm = tm == 64 ? 128 : 64;
+  if (f32 && (cfg & 2)) tn = tn == 64 ? 128 : 64;
+  if (tm == 128 && tn == 32) tn = 64;
+  const dim3 grid((n + tn - 1) / tn, (m + tm - 1) / tm, splits);
+  double* out = splits > 1 ? split_ws : C;
+  const long ldo = splits > 1 ? n : ldc;
+  const long sstride = splits > 1 ? 2L * m * n : 0;
+  const double a = splits > 1 ? 1.0 : alpha;
+  const long ldb = gemm_real_row(k);
+  auto go = [&](auto kern, auto* b) {
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, m, n, k, kchunk, a, A, lda, b, ldb, out, ldo,
+                       sstride, nanmix ? 1 : 0);
+  };
+  if (f32) {
+    const float* b = (const float*)B;
+    if (tm == 128) tn == 128 ? go(k_gemm_real<float, 128, 128, 16>, b) : go(k_gemm_real<float, 128, 64, 16>, b);
+    else if (tn == 128) go(k_gemm_real<float, 64, 128, 16>, b);
+    else tn == 64 ? go(k_gemm_real<float, 64, 64, 16>, b) : go(k_gemm_real<float, 64, 32, 16>, b);
+  } else {
+    const double* b = (const double*)B;
+    if (tm == 128) go(k_gemm_real<double, 128, 64, 8>, b);
+    else tn == 64 ? go(k_gemm_real<double, 64, 64, 16>, b) : go(k_gemm_real<double, 64, 32, 16>, b);
+  }
+  AFQ_HIP(hipGetLastError());
+  if (splits > 1) launch_split_reduce(s, m, n, splits, alpha, split_ws, C, ldc);
+}
+
+}  // namespace afq

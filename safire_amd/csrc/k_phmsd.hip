@@ -1269,8 +1269,12 @@ void launch_ph0_products(hipStream_t s, int nw, int nmo, int nel, int nact, int 
   AFQ_HIP(hipGetLastError());
   launch_gemm_nt_z(s, AFQ_FP64, nw * nel, nact, nmo, 1.0, Phit, nmo, A, nmo, true, TAB, nact);
   launch_gemm_nt_z(s, AFQ_FP64, nw * nel, nact, nmo, 1.0, Phit, nmo, haj, nmo, true, Hp, nact);
-  launch_gemm_nt_z(s, AFQ_FP64, nw * nel, nchol * nact, nmo, 1.0, Phit, nmo, Lna, nmo,
-                   lna_complex, P,                   (long)nchol * nact);
+  if (lna_complex)
+    launch_gemm_nt_z(s, AFQ_FP64, nw * nel, nchol * nact, nmo, 1.0, Phit, nmo, Lna, nmo, true, P,
+                     (long)nchol * nact);
+  else   // real rows padded for launch_gemm_real
+    launch_gemm_real(s, AFQ_FP64, nw * nel, nchol * nact, nmo, 1.0, Phit, nmo, Lna, P,
+                     (long)nchol * nact, true);
 }
 
 void launch_ph0_config(hipStream_t s, int nw, int nc, int nel, int nact, int nchol,

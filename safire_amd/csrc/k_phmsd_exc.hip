@@ -526,11 +526,11 @@ __global__ __launch_bounds__(256) void k_ph_density(int nup, int ndn, int nmo, i
   }
 }
 
-// out[n][lk] = Likn[lk][n], the rows l <= k only when folded
-__global__ void k_ph_rows_of_vectors(int nmo, int nchol, int fold, const double* __restrict__ Likn,
+// out[n ld + lk] = Likn[lk][n], the rows l <= k only when folded
+__global__ void k_ph_rows_of_vectors(int nmo, int nchol, int fold, int ld,
+                                     const double* __restrict__ Likn,
                                      double* __restrict__ out) {
   __shared__ double tile[32][33];
-  const int size = fold ? nmo * (nmo + 1) / 2 : nmo * nmo;
   const int l = blockIdx.z, kb = blockIdx.y * 32, nb = blockIdx.x * 32;
   for (int r = threadIdx.y; r < 32; r += 8) {
     const int k = kb + r, n = nb + threadIdx.x;
@@ -541,7 +541,7 @@ __global__ void k_ph_rows_of_vectors(int nmo, int nchol, int fold, const double*
     const int n = nb + r, k = kb + threadIdx.x;
     if (n < nchol && k < nmo && !(fold && k < l)) {
       const long at = fold ? (long)l * nmo - (long)l * (l - 1) / 2 + (k - l) : (long)l * nmo + k;
-      out[(long)n * size + at] = tile[threadIdx.x][r];
+      out[(long)n * ld + at] = tile[threadIdx.x][r];
     }
   }
 }
@@ -659,10 +659,10 @@ void launch_ph_density(hipStream_t s, int nw, int nup, int ndn, int nact, int nm
   AFQ_HIP(hipGetLastError());
 }
 
-void launch_ph_rows_of_vectors(hipStream_t s, int nmo, int nchol, bool fold, const double* Likn,
-                               double* out) {
+void launch_ph_rows_of_vectors(hipStream_t s, int nmo, int nchol, bool fold, int ld,
+                               const double* Likn, double* out) {
   hipLaunchKernelGGL(k_ph_rows_of_vectors, dim3((nchol + 31) / 32, (nmo + 31) / 32, nmo),
-                     dim3(32, 8), 0, s, nmo, nchol, fold ? 1 : 0, Likn, out);
+                     dim3(32, 8), 0, s, nmo, nchol, fold ? 1 : 0, ld, Likn, out);
   AFQ_HIP(hipGetLastError());
 }
 

@@ -195,10 +195,10 @@ void sparsify_one_body_propagator(int M, double* P) {
 // H1 = dt (h + v0) + vHS(vMF), hermitized, and P1 = exp(-H1/2) (getOneBodyPropagatorMatrix,
 // Real3IndexFactorization.hpp:99-124; generateP1, AFQMCBasePropagator.cpp:141-157) by scaling
 // and squaring of a degree-18 Taylor polynomial. Synchronises the stream (the scaling is chosen
-// on the host from ||A||_1).
+// on the host from ||A||_1). P1r [2][M][M] (f64) receives P1 and its transpose when P1 is real.
 void build_one_body_propagator(hipStream_t s, int M, int K, double dt, const double* h,
                                const double* v0, const double* Likn, const double* vMF,
-                               double* H1, double* P1) {
+                               double* H1, double* P1, double* P1r, bool* real) {
   // scratch: ms, A, P, Q [M*M] (c128)
   double* tmp = nullptr;
   AFQ_HIP(hipMalloc(&tmp, 2 * (size_t)M * M * 4 * sizeof(double)));
@@ -252,6 +252,13 @@ void build_one_body_propagator(hipStream_t s, int M, int K, double dt, const dou
     AFQ_HIP(hipStreamSynchronize(s));
     sparsify_one_body_propagator(M, hP.data());
     AFQ_HIP(hipMemcpyAsync(P1, hP.data(), hP.size() * sizeof(double), hipMemcpyHostToDevice, s));
+    *real = true;
+    for (size_t e = 0; e < (size_t)M * M; ++e) *real = *real && hP[2 * e + 1] == 0.0;
+    std::vector<double> hR(2 * (size_t)M * M);
+    for (int i = 0; i < M; ++i)
+      for (int j = 0; j < M; ++j)
+        hR[(size_t)i * M + j] = hR[(size_t)M * M + (size_t)j * M + i] = hP[2 * ((size_t)i * M + j)];
+    AFQ_HIP(hipMemcpyAsync(P1r, hR.data(), hR.size() * sizeof(double), hipMemcpyHostToDevice, s));
     AFQ_HIP(hipGetLastError());
     AFQ_HIP(hipStreamSynchronize(s));
   } catch (...) {
@@ -283,7 +290,8 @@ void setup_hamiltonian(afq_ham_s* H, hipStream_t s) {
     launch_gemm_nt_z(s, AFQ_FP64, 1, K, N * M, vscale, Gt, (long)N * M, H->Lnak, (long)N * M,
                      true, H->vMF, K);
     launch_zero_imag(s, K, H->vMF);
-    build_one_body_propagator(s, M, K, H->dt, H->h, H->v0, H->Likn, H->vMF, H->H1, H->P1);
+    build_one_body_propagator(s, M, K, H->dt, H->h, H->v0, H->Likn, H->vMF, H->H1, H->P1,
+                              H->P1r, &H->P1_real);
     // FP32 copies of the Cholesky tensors for the FP32 contraction form
     hipLaunchKernelGGL(k_to_f32, blocks(2 * nL), dim3(256), 0, s, 2 * nL, H->Lnak, H->Lnak_f);
     hipLaunchKernelGGL(k_to_f32, blocks((long)M * M * K), dim3(256), 0, s, (long)M * M * K,
