@@ -12,7 +12,7 @@ SOURCES = ["afq_api.hip", "afq_phmsd.hip", "afq_rng.hip", "k_green.hip", "k_gemm
            "k_exchange_f64.hip",
            "k_exchange_i8.hip", "k_phmsd.hip", "k_phmsd_exc.hip", "k_propagate.hip", "k_qr.hip", "k_walker.hip",
            "k_setup.hip"]
-# k_green.hip unrolls the 32 Gauss-Jordan steps of its N <= 32 kernel in full (each step indexes
+# k_green.hip unrolls the 16 Gauss-Jordan steps of its N <= 16 kernels in full (each step indexes
 # the register-resident rows with the step number); the default budget of a pragma-driven unroll
 # would leave the loop rolled and the rows in scratch memory.
 FILE_FLAGS = {"k_green.hip": ["-mllvm", "-pragma-unroll-threshold=1000000"]}

@@ -9,16 +9,12 @@
 //   G = T^-T Phi_w^T                [N,M] compact Green's function
 // Optional epilogue: E1 = E0 + scl * sum_{a,j} G[a][j] haj[a][j] (Real3IndexFactorization.hpp:505-508).
 //
-// Both products run on FP64 MFMA 16x16x4 tiles. When Phi_w, PsiT and haj fit in 96 KB of LDS
-// they are staged there first with batched loads (every load of a batch in flight before the
-// first LDS write), so the kernel waits on memory once rather than once per chunk; otherwise the
-// operands are read straight from memory (64 bytes per lane and k-chunk).
-//
-// The inverse comes from Gauss-Jordan elimination of [T | I] with partial pivoting: its pivots
-// are getrf's (the rows at and below step j see the same eliminations), so the determinant
-// convention is unchanged. Lane c holds column c of [T | I] (2N <= 64 columns) in registers; each
-// step broadcasts the pivot column through LDS. One 64-thread workgroup per walker: no
-// workgroup barrier, and W workgroups spread over all CUs.
+// Both products run on FP64 MFMA 16x16x4 tiles. The inverse comes from Gauss-Jordan elimination with
+// partial pivoting: its pivots are getrf's (the rows at and below step j see the same eliminations),
+// so the determinant convention is unchanged. Three kernels: k_green16 (up to 16 electrons, operands
+// in LDS), k_green32 (17 to 32) and k_green (up to 16 whose operands exceed 96 KB of LDS: one
+// wavefront per walker; lane c holds column c of [T | I] in registers, each step broadcasts the
+// pivot column through LDS).
 #include "afq_internal.hpp"
 
 #include <cfloat>
@@ -38,24 +34,6 @@ __device__ inline double readlane_d(double v, int lane) {
   const unsigned lo = __builtin_amdgcn_readlane((unsigned)u, lane);
   const unsigned hi = __builtin_amdgcn_readlane((unsigned)(u >> 32), lane);
   return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
-}
-
-// dst[e] = src[e] for e < n; the B loads of a batch are all in flight before the first store
-template <int B>
-__device__ inline void stage_batch(cd* dst, const cd* __restrict__ src, int n, int lane) {
-  for (int e0 = 0; e0 < n; e0 += 64 * B) {
-    double2 v[B];
-#pragma unroll
-    for (int b = 0; b < B; ++b) {
-      const int e = min(e0 + 64 * b + lane, n - 1);
-      v[b] = reinterpret_cast<const double2*>(src)[e];
-    }
-#pragma unroll
-    for (int b = 0; b < B; ++b) {
-      const int e = e0 + 64 * b + lane;
-      if (e < n) reinterpret_cast<double2*>(dst)[e] = v[b];
-    }
-  }
 }
 
 template <int N_>
@@ -95,7 +73,7 @@ __device__ inline int lowest_lane(unsigned long long mask) {
   return __builtin_ctzll(mask);
 }
 
-template <int NMAX, bool STAGE>
+template <int NMAX>
 __global__ __launch_bounds__(64) void k_green(int M, int N, const cd* __restrict__ PsiT,
                                               const cd* __restrict__ Phi, long ldw,
                                               cd* __restrict__ G, cd* __restrict__ ov,
@@ -106,21 +84,11 @@ __global__ __launch_bounds__(64) void k_green(int M, int N, const cd* __restrict
   constexpr int NB = 16 * NT;
   __shared__ cd sT[NB * NB];               // T, then T^-1, row-major
   __shared__ cd sCol[2][NMAX];             // pivot column broadcast (double-buffered)
-  extern __shared__ cd sDyn[];             // STAGE: Phi_w [M][N], PsiT [N][M], haj [N][M]
   const int lane = threadIdx.x;
   const int g = lane >> 4, r16 = lane & 15;
   const int w = blockIdx.x;
-  const cd* Pg = Phi + (long)w * ldw;
+  const cd* P = Phi + (long)w * ldw;
   const bool want_e1 = E != nullptr && haj != nullptr;
-  if (STAGE) {
-    stage_batch<16>(sDyn, Pg, M * N, lane);
-    stage_batch<16>(sDyn + M * N, PsiT, M * N, lane);
-    if (want_e1) stage_batch<16>(sDyn + 2 * M * N, haj, M * N, lane);
-    wave_sync();
-  }
-  const cd* P = STAGE ? sDyn : Pg;
-  const cd* Ps = STAGE ? sDyn + M * N : PsiT;
-  const cd* Hj = (STAGE && want_e1) ? sDyn + 2 * M * N : haj;
 
   // ---- T[a][c] = sum_i PsiT[a][i] Phi[i][c]  (MFMA; k = orbital i) ----
   {
@@ -140,7 +108,7 @@ __global__ __launch_bounds__(64) void k_green(int M, int N, const cd* __restrict
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
           const int k = k0 + 4 * g + s;
-          const cd x = (a < N && k < M) ? Ps[(long)a * M + k] : cmk(0, 0);
+          const cd x = (a < N && k < M) ? PsiT[(long)a * M + k] : cmk(0, 0);
           ar[t][s] = x.re;
           ai[t][s] = x.im;
           const int c = t * 16 + r16;
@@ -190,8 +158,7 @@ __global__ __launch_bounds__(64) void k_green(int M, int N, const cd* __restrict
   }
   cd upiv = cmk(1.0, 0.0);     // lane j keeps +-U_jj; the logs are taken in parallel afterwards
   bool singular = false;
-  int rowpos = 0;              // N > 16: the getrf position of this lane's row
-  if constexpr (NMAX <= 16) {
+  {
     // Step j is unrolled, so column j is a register of lane j: lane j finds the pivot in its own
     // column (izamax: first maximum of |re|+|im| from row j down) and readlane broadcasts it; the
     // row swap selects over a static row range; lane j publishes its swapped column to LDS, from
@@ -247,93 +214,6 @@ __global__ __launch_bounds__(64) void k_green(int M, int N, const cd* __restrict
         x[j] = xjn;
       }
     }
-  } else {
-    // 16 < N <= 32: a row layout that keeps x[] in registers through fully unrolled steps. Lane
-    // (r, h) = (lane % 32, lane / 32) holds columns 32h..32h+31 of row r of [T | I] (T in
-    // columns 0..31, I in 32..63). Rows are never moved: each row carries its getrf position,
-    // the pivot is chosen with izamax's rule over the rows at positions >= j (first maximum of
-    // |re|+|im| by position; a NaN at position j is kept, a later NaN is skipped), and positions
-    // are swapped as getrf swaps rows, so the eliminations, pivots and signs are getrf's. Each
-    // step takes two 16-lane DPP maxima, a few readlanes and one LDS round trip for the pivot
-    // row and the multipliers.
-    __shared__ cd sRow[2][64];
-    __shared__ cd sF[2][32];
-    const int r = lane & 31, h = lane >> 5;
-#pragma unroll
-    for (int e = 0; e < NMAX; ++e) {
-      cd v = cmk(0.0, 0.0);
-      if (r < N) {
-        if (h == 0) {
-          if (e < N) v = sT[r * NB + e];
-        } else if (e == r) {
-          v = cmk(1.0, 0.0);
-        }
-      }
-      x[e] = v;
-    }
-    int pos = r;
-#pragma unroll
-    for (int j = 0; j < NMAX; ++j) {
-      if (j < N) {
-        const bool cand = h == 0 && r < N && pos >= j;
-        const double v = cand ? cabs1(x[j]) : -1.0;
-        const int q = lowest_lane(__ballot(h == 0 && pos == j));
-        const double vq = readlane_d(v, q);
-        int p;
-        if (isnan(vq)) {
-          p = q;
-        } else {
-          const double m16 = row_max16(v);
-          const double m = fmax(readlane_d(m16, 0), readlane_d(m16, 16));
-          const unsigned long long mask = __ballot(cand && v == m);
-          if (__builtin_popcountll(mask) == 1) {
-            p = lowest_lane(mask);
-          } else {
-            const int k16 = row_min16(((mask >> lane) & 1ull) ? pos : 0x7fffffff);
-            const int km = min(__builtin_amdgcn_readlane(k16, 0), __builtin_amdgcn_readlane(k16, 16));
-            p = lowest_lane(__ballot(h == 0 && pos == km));
-          }
-        }
-        p = __builtin_amdgcn_readfirstlane(p);
-        const cd piv = cmk(readlane_d(x[j].re, p), readlane_d(x[j].im, p));
-        const int pp = __builtin_amdgcn_readlane(pos, p);
-        if (lane == j) upiv = (pp == j) ? piv : -piv;   // the sign flips where getrf swaps rows
-        if (cis0(piv)) {
-          singular = true;   // getrf records the zero pivot and goes on; getri_or_zero zeroes it
-        } else {
-          if (r == q) pos = pp;
-          if (r == p) pos = j;
-          cd* row = sRow[j & 1];
-          cd* fv = sF[j & 1];
-          if (r == p)
-#pragma unroll
-            for (int e = 0; e < NMAX; ++e) row[32 * h + e] = x[e];
-          if (h == 0) fv[r] = x[j];
-          wave_sync();
-          const cd inv = cdiv(cmk(1.0, 0.0), piv);
-          const cd f = fv[r];
-          const bool upd = r != p && !cis0(f);
-          const cd mlt = f * inv;
-          // the pivot row in chunks of 8 columns: each chunk's LDS reads are all in flight before
-          // the first use (one wait per chunk rather than one per column)
-#pragma unroll
-          for (int e0 = 0; e0 < NMAX; e0 += 8) {
-            cd pr[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) pr[e] = row[32 * h + e0 + e];
-            if (r == p) {
-#pragma unroll
-              for (int e = 0; e < 8; ++e) x[e0 + e] = pr[e] * inv;
-            } else if (upd) {
-#pragma unroll
-              for (int e = 0; e < 8; ++e) x[e0 + e] -= mlt * pr[e];
-            }
-          }
-        }
-      }
-    }
-    // row r is row pos of [I | T^-1]; lanes (r, 1) publish T^-1 after the zero fill below
-    rowpos = pos;
   }
 
   // sum_j log(+-U_jj + DBL_MIN): one log per lane, then a wavefront sum
@@ -361,18 +241,11 @@ __global__ __launch_bounds__(64) void k_green(int M, int N, const cd* __restrict
   wave_sync();
   for (int e = lane; e < NB * NB; e += 64) sT[e] = cmk(0, 0);
   wave_sync();
-  if constexpr (NMAX <= 16) {
-    if (lane >= N && lane < 2 * N && !singular) {
-      const int a = lane - N;
+  if (lane >= N && lane < 2 * N && !singular) {
+    const int a = lane - N;
 #pragma unroll
-      for (int r = 0; r < NMAX; ++r)
-        if (r < N) sT[r * NB + a] = x[r];
-    }
-  } else {
-    if (lane >= 32 && (lane & 31) < N && !singular)
-#pragma unroll
-      for (int e = 0; e < NMAX; ++e)
-        if (e < N) sT[rowpos * NB + e] = x[e];
+    for (int r = 0; r < NMAX; ++r)
+      if (r < N) sT[r * NB + a] = x[r];
   }
   wave_sync();
 
@@ -421,7 +294,7 @@ __global__ __launch_bounds__(64) void k_green(int M, int N, const cd* __restrict
         if (a < N && i < M) {
           const cd v = cmk(gr[t][r], gi[t][r]);
           if (Gw) Gw[(long)a * M + i] = v;
-          if (want_e1) e1 += v * Hj[(long)a * M + i];
+          if (want_e1) e1 += v * haj[(long)a * M + i];
         }
       }
   }
@@ -714,6 +587,306 @@ __global__ __launch_bounds__(64 * kGWaves) void k_green16(
   }
 }
 
+// ---- 17 to 32 electrons: four wavefronts per walker, the inverse in place ----
+//
+// T = PsiT Phi_w on MFMA, its k range (orbitals) dealt to the wavefronts in steps of four, operands
+// straight from memory (Phi_w is read twice, 16 lanes along a row each time, rather than held in
+// LDS, so that four workgroups fit a CU); the partial tiles are added in a fixed order. The Gauss-Jordan
+// elimination works in place: 8 threads hold column c (rows q, q + 8, q + 16, q + 24) and the column of
+// step j becomes the inverse's column of its pivot row, which is what [T | I] gives with half of the
+// columns. A step is one barrier: the owners of column j choose the pivot (izamax's rule over
+// the rows at getrf positions >= j: first maximum of |re| + |im| by position; a NaN at position j is
+// kept, a later NaN skipped) and publish the column, the pivot's position and its reciprocal;
+// every thread takes the pivot row's entry of its column from the 8 lanes through DPP. Rows
+// never move: each carries its getrf position. The loop stays rolled (the fully unrolled single-
+// wavefront elimination it replaces streamed ~100 KB of code per walker). Bound by the latency of
+// the serial steps. M 128, N 32, 1024 walkers: 188 -> 120 us (G and overlap), 130 -> 86 us (overlap
+// alone); M 88, N 22, 137 walkers 107 -> 45 us; M 77, N 19, 201 walkers 85 -> 40 us.
+// the bits of the one lane whose v is not all zeros
+template <int CTRL>
+__device__ inline double dpp8_or(double v) {
+  const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+  const unsigned lo = __builtin_amdgcn_update_dpp((unsigned)u, (unsigned)u, CTRL, 0xf, 0xf, false);
+  const unsigned hi = __builtin_amdgcn_update_dpp((unsigned)(u >> 32), (unsigned)(u >> 32), CTRL, 0xf,
+                                                  0xf, false);
+  return __builtin_bit_cast(double, u | ((unsigned long long)hi << 32 | lo));
+}
+template <int CTRL>
+__device__ inline double dpp8_max(double v) {
+  const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+  const unsigned lo = __builtin_amdgcn_update_dpp((unsigned)u, (unsigned)u, CTRL, 0xf, 0xf, false);
+  const unsigned hi = __builtin_amdgcn_update_dpp((unsigned)(u >> 32), (unsigned)(u >> 32), CTRL, 0xf,
+                                                  0xf, false);
+  return fmax(v, __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo));
+}
+template <int CTRL>
+__device__ inline int dpp8_min(int v) {
+  return min(v, __builtin_amdgcn_update_dpp(v, v, CTRL, 0xf, 0xf, false));
+}
+// over the 8 lanes of a column: quad permutes (lanes ^1, ^2), then the other quad (half-row mirror)
+__device__ inline double only8(double v) { return dpp8_or<0x141>(dpp8_or<0x4E>(dpp8_or<0xB1>(v))); }
+__device__ inline double max8(double v) { return dpp8_max<0x141>(dpp8_max<0x4E>(dpp8_max<0xB1>(v))); }
+__device__ inline int min8(int v) { return dpp8_min<0x141>(dpp8_min<0x4E>(dpp8_min<0xB1>(v))); }
+
+__global__ __launch_bounds__(256, 4) void k_green32(
+    int M, int N, const cd* __restrict__ PsiT, const cd* __restrict__ Phi, long ldw,
+    cd* __restrict__ G, cd* __restrict__ ov, int ov_mode, double ov_scale, cd ov_add,
+    const cd* __restrict__ haj, double E0, double e1_scale, cd* __restrict__ E, long ldE) {
+  constexpr int NB = 32, LD = 33;
+  __shared__ cd sT[2][NB * LD];            // partial T tiles; then [0]: T, later T^-1 [b][a]
+  __shared__ cd sF[2][NB];                 // column j of every row
+  __shared__ cd sInv[2];                   // 1 / pivot
+  __shared__ int sPos[2];                  // the pivot's position; -1: the pivot is exactly zero
+  __shared__ cd sPiv[NB];                  // +-U_jj
+  __shared__ int sRow[NB];                 // pivot row of step j
+  __shared__ cd sE[4];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = lane >> 4, r16 = lane & 15;
+  const int w = blockIdx.x;
+  const cd* P = Phi + (long)w * ldw;
+  const bool inverse = G != nullptr || E != nullptr;
+
+  // ---- partial T[a][c] over this wavefront's k steps ----
+  {
+    d4 tr[2][2], ti[2][2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        tr[a][b] = d4{0, 0, 0, 0};
+        ti[a][b] = d4{0, 0, 0, 0};
+      }
+    const int steps = (M + 3) >> 2;
+    auto load = [&](int t, cd (&x)[2], cd (&y)[2]) {
+      const int k = 4 * t + g;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int r = 16 * u + r16;
+        const bool ok = r < N && k < M;
+        x[u] = ok ? PsiT[r * M + k] : cmk(0, 0);
+        y[u] = ok ? P[k * N + r] : cmk(0, 0);
+      }
+    };
+    cd x[2], y[2];
+    load(wv, x, y);
+    for (int t = wv; t < steps; t += 4) {   // the next step's operands are loaded ahead
+      cd nx[2], ny[2];
+      load(t + 4, nx, ny);
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+          tr[a][b] = mfma16x16x4(x[a].re, y[b].re, tr[a][b]);
+          ti[a][b] = mfma16x16x4(x[a].re, y[b].im, ti[a][b]);
+        }
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+          tr[a][b] = mfma16x16x4(-x[a].im, y[b].im, tr[a][b]);
+          ti[a][b] = mfma16x16x4(x[a].im, y[b].re, ti[a][b]);
+        }
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        x[u] = nx[u];
+        y[u] = ny[u];
+      }
+    }
+    // wavefronts 2, 3 into [0], [1]; 0 and 1 add theirs; 1 into [1]; 0 adds it
+    auto put = [&](cd* dst, const cd* add) {
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int e = (16 * a + acc_row<double>(g, r)) * LD + 16 * b + r16;
+            cd v = cmk(tr[a][b][r], ti[a][b][r]);
+            if (add) v = add[e] + v;
+            dst[e] = v;
+          }
+    };
+    if (wv >= 2) put(sT[wv - 2], nullptr);
+    __syncthreads();
+    if (wv < 2) put(sT[wv], sT[wv]);
+    __syncthreads();
+  }
+  // ---- in-place Gauss-Jordan: thread (c, q) holds rows q + 8 i of column c ----
+  const int c = tid >> 3, q = tid & 7;
+  cd x[4];
+  int pos[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = q + 8 * i;
+    pos[i] = r;
+    x[i] = (r < N && c < N) ? sT[0][r * LD + c] + sT[1][r * LD + c] : cmk(0.0, 0.0);
+  }
+  // the owners of column j choose its pivot and publish the column
+  auto publish = [&](int j) {
+    double m = -1.0, vq = 0.0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const double v = cabs1(x[i]);
+      if (q + 8 * i < N && pos[i] >= j) m = fmax(m, v);   // drops a NaN
+      if (pos[i] == j) vq = v;
+    }
+    m = max8(m);
+    vq = only8(vq);                                        // the row at position j
+    int k = 0x7fffffff;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (q + 8 * i < N && pos[i] >= j && cabs1(x[i]) == m) k = min(k, pos[i]);
+    k = min8(k);
+    if (isnan(vq)) k = j;
+    cd pv = cmk(0.0, 0.0);
+    int row = 0x7fffffff;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (pos[i] == k) {
+        pv = x[i];
+        row = q + 8 * i;
+      }
+    row = min8(row);
+    pv.re = only8(pv.re);
+    pv.im = only8(pv.im);
+    const bool zero = cis0(pv);
+    const cd inv = zero ? cmk(0.0, 0.0) : cdiv(cmk(1.0, 0.0), pv);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sF[j & 1][q + 8 * i] = x[i];
+    if (q == 0) {
+      sInv[j & 1] = inv;
+      sPos[j & 1] = zero ? -1 : k;
+      sPiv[j] = k == j ? pv : -pv;   // the sign flips where getrf swaps rows
+      sRow[j] = row;
+    }
+  };
+  if (c == 0) publish(0);
+  __syncthreads();
+  bool singular = false;
+  for (int j = 0; j < N; ++j) {
+    const int k = sPos[j & 1];
+    if (k < 0) {
+      singular = true;   // getrf records the zero pivot and goes on; getri_or_zero zeroes T^-1
+    } else if (c < N && (inverse || c > j)) {
+      const cd inv = sInv[j & 1];
+      cd p = cmk(0.0, 0.0), f[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        f[i] = sF[j & 1][q + 8 * i];
+        if (pos[i] == k) p = x[i];
+      }
+      p.re = only8(p.re);
+      p.im = only8(p.im);
+      if (c == j) p = cmk(1.0, 0.0);   // the identity's column of the pivot row takes this place
+      p = p * inv;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const cd old = c == j ? cmk(0.0, 0.0) : x[i];
+        x[i] = pos[i] == k ? p : (cis0(f[i]) ? old : old - f[i] * p);
+      }
+    }
+    if (k >= 0) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) pos[i] = pos[i] == k ? j : (pos[i] == j ? k : pos[i]);
+    }
+    if (c == j + 1 && c < N) publish(j + 1);
+    __syncthreads();
+  }
+
+  if (wv == 0) {
+    // sum_j log(+-U_jj + DBL_MIN): one log per lane, then a wavefront sum
+    cd acc = (lane < N) ? clog_(cmk(sPiv[lane].re + DBL_MIN, sPiv[lane].im)) : cmk(0.0, 0.0);
+    for (int off = 32; off > 0; off >>= 1) {
+      acc.re += __shfl_xor(acc.re, off, 64);
+      acc.im += __shfl_xor(acc.im, off, 64);
+    }
+    if (lane == 0) {
+      if (ov_mode == 2) acc += ov[w];
+      const double pi = 3.14159265358979323846;
+      // the reference loops until the value is in range; a non-finite value would never get
+      // there, so only finite values are wrapped
+      if (!isfinite(acc.im)) {
+      } else if (acc.im > pi) {
+        while (acc.im > pi) acc.im -= 2 * pi;
+      } else if (acc.im < -pi) {
+        while (acc.im < -pi) acc.im += 2 * pi;
+      }
+      if (ov_mode != 0) ov[w] = ov_scale * acc + ov_add;
+    }
+  }
+  if (!inverse) return;
+
+  // ---- T^-1 to LDS as [b][a]: row r ends at position pos, column slot j is pivot row sRow[j]'s ----
+  cd* sI = sT[0];
+  if (c < N)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (q + 8 * i < N) sI[pos[i] * LD + sRow[c]] = singular ? cmk(0.0, 0.0) : x[i];
+  for (int e = tid; e < NB * NB; e += 256) {
+    const int b = e / NB, a = e % NB;
+    if (b >= N || a >= N) sI[b * LD + a] = cmk(0.0, 0.0);
+  }
+  __syncthreads();
+
+  // ---- G[a][i] = sum_b Tinv[b][a] Phi[i][b], 16 columns i per wavefront and turn ----
+  const bool want_e1 = E != nullptr && haj != nullptr;
+  cd e1 = cmk(0.0, 0.0);
+  cd* Gw = G ? G + (long)w * N * M : nullptr;
+  for (int i0 = 16 * wv; i0 < M; i0 += 64) {
+    asm volatile("" ::: "memory");   // T^-1 is read from LDS in every turn: hoisted, it would spill
+    const int i = i0 + r16;
+    d4 gr[2], gi[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      gr[t] = d4{0, 0, 0, 0};
+      gi[t] = d4{0, 0, 0, 0};
+    }
+    cd y[8];
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      const int b = 4 * s + g;
+      y[s] = (i < M && b < N) ? P[(long)i * N + b] : cmk(0, 0);
+    }
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      cd z[2];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) z[t] = sI[(4 * s + g) * LD + 16 * t + r16];   // Tinv^T[a][b]
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        gr[t] = mfma16x16x4(z[t].re, y[s].re, gr[t]);
+        gi[t] = mfma16x16x4(z[t].re, y[s].im, gi[t]);
+      }
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        gr[t] = mfma16x16x4(-z[t].im, y[s].im, gr[t]);
+        gi[t] = mfma16x16x4(z[t].im, y[s].re, gi[t]);
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int a = 16 * t + acc_row<double>(g, r);
+        if (a < N && i < M) {
+          const cd v = cmk(gr[t][r], gi[t][r]);
+          if (Gw) Gw[(long)a * M + i] = v;
+          if (want_e1) e1 += v * haj[(long)a * M + i];
+        }
+      }
+  }
+  if (want_e1) {
+    for (int off = 32; off > 0; off >>= 1) {
+      e1.re += __shfl_xor(e1.re, off, 64);
+      e1.im += __shfl_xor(e1.im, off, 64);
+    }
+    if (lane == 0) sE[wv] = e1;
+    __syncthreads();
+    if (tid == 0) E[(long)w * ldE] = cmk(E0, 0.0) + e1_scale * ((sE[0] + sE[1]) + (sE[2] + sE[3]));
+  }
+}
+
 }  // namespace
 
 void launch_green(hipStream_t s, int nb, int M, int N, const double* PsiT, const double* Phi,
@@ -735,24 +908,22 @@ void launch_green(hipStream_t s, int nb, int M, int N, const double* PsiT, const
     AFQ_HIP(hipGetLastError());
     return;
   }
-  // Phi_w, PsiT and haj go through LDS (batched coalesced loads) when they fit in 96 KB
-  const size_t lds = sizeof(cd) * (size_t)M * N * (e1 ? 3 : 2);
-  const bool stage = lds <= 96 * 1024;
-  auto go = [&](auto kern) {
-    if (stage) ensure_dynamic_lds((const void*)kern, lds);
-    hipLaunchKernelGGL(kern, dim3(nb), dim3(64), stage ? lds : 0, s, M, N,
-                       reinterpret_cast<const cd*>(PsiT), reinterpret_cast<const cd*>(Phi), ldw,
-                       reinterpret_cast<cd*>(G), reinterpret_cast<cd*>(ov), ov_mode, ov_scale,
-                       ov_add, reinterpret_cast<const cd*>(haj), E0, e1_scale,
-                       reinterpret_cast<cd*>(E), ldE);
-  };
-  if (stage) {
-    go(k_green<32, true>);
-  } else {
-    if (N <= 8) go(k_green<8, false>);
-    else if (N <= 16) go(k_green<16, false>);
-    else go(k_green<32, false>);
+  if (N > 16) {
+    hipLaunchKernelGGL(k_green32, dim3(nb), dim3(256), 0, s, M, N, reinterpret_cast<const cd*>(PsiT),
+                       reinterpret_cast<const cd*>(Phi), ldw, reinterpret_cast<cd*>(G),
+                       reinterpret_cast<cd*>(ov), ov_mode, ov_scale, ov_add,
+                       reinterpret_cast<const cd*>(haj), E0, e1_scale, reinterpret_cast<cd*>(E), ldE);
+    AFQ_HIP(hipGetLastError());
+    return;
   }
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(nb), dim3(64), 0, s, M, N, reinterpret_cast<const cd*>(PsiT),
+                       reinterpret_cast<const cd*>(Phi), ldw, reinterpret_cast<cd*>(G),
+                       reinterpret_cast<cd*>(ov), ov_mode, ov_scale, ov_add,
+                       reinterpret_cast<const cd*>(haj), E0, e1_scale, reinterpret_cast<cd*>(E), ldE);
+  };
+  if (N <= 8) go(k_green<8>);
+  else go(k_green<16>);
   AFQ_HIP(hipGetLastError());
 }
 
