@@ -140,3 +140,14 @@ def test_back_propagate(shape, complex_trial, symmetric):
     assert np.max(np.abs(diff.real)) < 1e-10
     assert np.max(np.abs((diff.imag + np.pi) % (2 * np.pi) - np.pi)) < 1e-10
     ham.close()
+
+
+@pytest.mark.parametrize("M,K", [(2, 1), (15, 3), (16, 64), (17, 60), (33, 257), (128, 9)])
+def test_exchange_operator(M, K):
+    rng, h, L, PsiT = system(M, 1, K, False, False)
+    got = A.HamiltonianOperations(h, L, PsiT, 0.0, 0.01).tensors()["v0"]
+    want = O.exchange_v0(L)
+    # sums of M K products, in another order: rounding below M K eps of the absolute sum
+    bound = 0.5 * np.einsum("ijn,ljn->il", np.abs(L), np.abs(L)) * M * K * 2.3e-16
+    assert np.all(np.abs(got - want) <= bound)
+    assert np.array_equal(got, got.T)
