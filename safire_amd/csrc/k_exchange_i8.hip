@@ -29,6 +29,12 @@
 // and then half of the wavefronts do that before their MFMAs and half after, so that the VALU work
 // of one wavefront of a SIMD runs under the MFMAs of the other.
 //
+// What bounds it: neither unit alone. A pass is MFMAs (8 K of 12 K cycles at M = 128), pair sums and
+// the two barriers around the LDS store, and the two wavefronts of a SIMD go through them nearly
+// together. One walker's 32 x 32 blocks with complex slices, the form before, against this one:
+// M 64, N 16, K 256, W 512 real trial: 188 -> 166 us; M 128, N 32, K 640, W 1024: 4040 -> 2560 us;
+// M 88, N 22, K 440, W 137: 1055 -> 240 us.
+//
 // M <= 128, N <= 32.
 #include "afq_internal.hpp"
 
@@ -81,6 +87,10 @@ __device__ inline unsigned pack4(int a, int b, int c, int d) {
 __device__ inline i4 mfma_i8(i4 a, i4 b, i4 c) {
   return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0);
 }
+
+// workgroup barrier after this wavefront's LDS reads and writes; its global loads and stores in flight
+// are not waited for. The memory clobber keeps the compiler from moving memory accesses across.
+__device__ inline void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // v plus the value of the lane `shift` below in the same row of 16 lanes (0 below the row)
 template <int SHIFT>
@@ -296,13 +306,16 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void k_exchange_i8(
     }
     const int col = 16 * t + r16;
     // columns past the pass read its last row and are not stored; bytes past a row meet zeros of G
-    const char* base = sB + min(col, crows - 1) * rowb + 16 * g;
+    int base = min(col, crows - 1) * rowb + 16 * g;
+    // two chunks: one opaque address per tile, not those of all slices held over the tiles in
+    // registers that are then spilled (M = 88, N = 22: 254 -> 240 us)
+    if (KC > 1) asm volatile("" : "+v"(base));
 #pragma unroll
     for (int kc = 0; kc < KC; ++kc)
 #pragma unroll
       for (int q = 0; q <= ON; ++q) {
-        const i4 br = *reinterpret_cast<const i4*>(base + q * NP * planeb + 64 * kc);
-        const i4 bi = LC ? *reinterpret_cast<const i4*>(base + (q * NP + 1) * planeb + 64 * kc) : br;
+        const i4 br = *reinterpret_cast<const i4*>(sB + base + q * NP * planeb + 64 * kc);
+        const i4 bi = LC ? *reinterpret_cast<const i4*>(sB + base + (q * NP + 1) * planeb + 64 * kc) : br;
 #pragma unroll
         for (int s = 0; s + q <= ON; ++s) {
           cR[s + q] = mfma_i8(ar[kc][s], br, cR[s + q]);
@@ -364,7 +377,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void k_exchange_i8(
     double2* T = sT + (tdbl ? tb * tsize : 0);
     const double2* Tp = sT + (tdbl ? (tb ^ 1) * tsize : 0);
     if (prev && (!tdbl || wave < NW / 2)) pairs(Tp, n0 - Cv);
-    if (!tdbl) __syncthreads();   // the previous pass's T has been read
+    if (!tdbl) lds_barrier();   // the previous pass's T has been read
     for (int t = 0; t < CT; ++t) {
       if (on == 5) tile(std::integral_constant<int, 5>(), t, T);
       else if (on == 4) tile(std::integral_constant<int, 4>(), t, T);
@@ -372,9 +385,9 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void k_exchange_i8(
       else tile(std::integral_constant<int, 2>(), t, T);
     }
     if (prev && tdbl && wave >= NW / 2) pairs(Tp, n0 - Cv);
-    __syncthreads();              // this pass's slices have been read, its T is written
+    lds_barrier();              // this pass's slices have been read, its T is written
     if (more) lstore(next);
-    __syncthreads();
+    lds_barrier();
     on = next;
     tb ^= 1;
   }
