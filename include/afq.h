@@ -44,7 +44,9 @@ enum afq_status {
 enum afq_walker_type { AFQ_CLOSED = 1, AFQ_COLLINEAR = 2 };
 
 /* Arithmetic of the Cholesky contractions (vbias, vHS, exchange/Coulomb energy). Overlaps,
- * log-determinants, inverses, QR, the propagator, weights and energy sums stay FP64. */
+ * log-determinants, inverses, QR, the propagator, weights and energy sums stay FP64. Where the
+ * exchange takes fewer operations from a table of orbital pairs (real trials with enough Cholesky
+ * vectors and walkers), exchange and Coulomb energy are FP64 in every form. */
 enum afq_precision {
   AFQ_FP64 = 0,        /* plain form: everything FP64 (FP64 MFMA)                          */
   AFQ_FP32 = 1,        /* contractions in FP32 on MFMA with FP32 accumulation               */
@@ -54,9 +56,9 @@ enum afq_precision {
                           part; vbias and vHS as in AFQ_FP32. Needs N <= 16, M <= 96 and
                           M % 8 == 0 (AFQ_EUNSUPPORTED otherwise)                           */
   AFQ_INT8_SPLIT = 3   /* mixed form: the exchange energy on int8 MFMA with every row of G
-                          and Lnak scaled by a power of two and split into 5 int8 slices
-                          (x = u (q0 + q1/254 + ... + q4/254^4)); the 15 slice products of
-                          order <= 4 accumulate exactly in int32 and are combined in FP64
+                          and Lnak scaled by a power of two and split into 6 int8 slices
+                          (x = u (q0 + q1/254 + ... + q5/254^5)); the slice products up to an
+                          order of 2 to 5, by the vector's size, accumulate exactly in int32 and are combined in FP64
                           (energy error ~1e-3 of AFQ_FP32's). vbias and vHS as in AFQ_FP32.
                           Needs N <= 32 and M <= 128 (AFQ_EUNSUPPORTED otherwise)           */
 };

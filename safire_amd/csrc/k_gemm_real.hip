@@ -15,6 +15,15 @@
 // vectors of a real trial against k_gemm_nt on the full ones (M 128, N 32, K 640, 1024 walkers):
 // vHS FP64 905 -> 474 us, FP32 660 -> 288 us; vbias FP64 475 -> 227 us, FP32 277 -> 140 us. M 64,
 // N 16, K 320, 512 walkers, FP64: vHS 68 -> 46 us.
+//
+// The exchange as a quadratic form: sum_n tr(T_n^2) with T_n = G Lnak_n^T is G B G^T over the pairs
+// (electron, orbital), B[(b, j)][(a, i)] = sum_n Lnak[n][b][i] Lnak[n][a][j] from the set-up. B is
+// symmetric: 2 (N M)^2 flops per walker instead of the 4 N^2 M K of the T_n, and with K some multiples
+// of M several times fewer, FP64 in place of the int8 split too. The Coulomb traces tr(T_n) are one
+// more product with the flat Lnak rows. Exchange and traces, per Cholesky vector -> pair table:
+//   M 128, N 32, K 640, 1024 walkers: FP64 6500, int8 2560 -> 830 + 264 us
+//   M 64, N 16, K 256, 512 walkers: int8 166 -> 56 + 23 us
+//   M 88, N 22, K 440, 137 walkers: int8 240 -> 49 + 27 us
 #include "afq_internal.hpp"
 
 #include <algorithm>
@@ -23,7 +32,11 @@ namespace afq {
 
 namespace {
 
-template <typename R, int TM, int TN, int KS>
+// DOT: the quadratic form A B A^T of each row instead of C, B being n x n and upper triangular (row q
+// holds the entries p <= q). Workgroup (x, y) takes item x, columns of tile_n times one chunk of the
+// k <= its last column, and rows of tile y; it writes sum_q (A B)[row][q] A[row][q] over its share as
+// partial x of the row (C[row][ldc]). The items of a tile_n follow one another, kchunk a multiple of TN.
+template <typename R, int TM, int TN, int KS, bool DOT = false>
 __global__ __launch_bounds__(256, 2) void k_gemm_real(int m, int n, int k, int kchunk, double alpha,
                                                       const double* __restrict__ A, long lda,
                                                       const R* __restrict__ B, long ldb,
@@ -46,8 +59,16 @@ __global__ __launch_bounds__(256, 2) void k_gemm_real(int m, int n, int k, int k
   const int wm = (wave >> 1) * (TM / 2), wn = (wave & 1) * (TN / 2);
   // column tiles fastest: consecutive workgroups (dealt round-robin to the XCDs) share rows of A,
   // and each XCD's L2 holds an eighth of B
-  const int tile_n = blockIdx.x, tile_m = blockIdx.y;
-  const int kbeg = blockIdx.z * kchunk, kend = min(k, kbeg + kchunk);
+  int tile_n = blockIdx.x, kbeg = blockIdx.z * kchunk;
+  if (DOT) {   // items of tile_n: tile_n / c + 1, so c tiles of j items each for j = 1, 2, ...
+    const int c = kchunk / TN;
+    int x = blockIdx.x, j = 1;
+    for (; x >= j * c; ++j) x -= j * c;
+    tile_n = (j - 1) * c + x / j;
+    kbeg = x % j * kchunk;
+  }
+  const int tile_m = blockIdx.y;
+  const int kend = min(DOT ? min(k, (tile_n + 1) * TN) : k, kbeg + kchunk);
   C += blockIdx.z * split_stride;
 
   double2 pa[PA];
@@ -158,6 +179,37 @@ __global__ __launch_bounds__(256, 2) void k_gemm_real(int m, int n, int k, int k
     if (more) sstore(buf ^ 1);
     __syncthreads();
   }
+  if constexpr (DOT) {
+    double2* red = reinterpret_cast<double2*>(sA);   // [2][TM], after the last barrier of the loop
+#pragma unroll
+    for (int a = 0; a < MT; ++a)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = wm + 16 * a + acc_row<R>(g, r), gm = min(tile_m * TM + row, m - 1);
+        double er = 0.0, ei = 0.0;
+#pragma unroll
+        for (int b = 0; b < NT; ++b) {
+          const int col = tile_n * TN + wn + 16 * b + r16;
+          if (col < n) {
+            const double2 x = *reinterpret_cast<const double2*>(A + 2 * ((long)gm * lda + col));
+            er += cr[a][b][r] * x.x - ci[a][b][r] * x.y;
+            ei += cr[a][b][r] * x.y + ci[a][b][r] * x.x;
+          }
+        }
+        for (int off = 8; off > 0; off >>= 1) {
+          er += __shfl_xor(er, off, 16);
+          ei += __shfl_xor(ei, off, 16);
+        }
+        if (r16 == 0) red[(wave & 1) * TM + row] = double2{er, ei};
+      }
+    __syncthreads();
+    if (tid < TM && tile_m * TM + tid < m) {
+      const double2 x = red[tid], y = red[TM + tid];
+      *reinterpret_cast<double2*>(C + 2 * ((long)(tile_m * TM + tid) * ldc + blockIdx.x)) =
+          double2{x.x + y.x, x.y + y.y};
+    }
+    return;
+  }
 #pragma unroll
   for (int a = 0; a < MT; ++a)
 #pragma unroll
@@ -195,7 +247,95 @@ __global__ void k_pad_rows(long rows, int k, int ldb, int n, int packed,
   dst[e] = c < k ? (D)src[(r * k + c) * stride] : (D)0;
 }
 
+// B[q = (b, j)][p = (a, i)] = w sum_n L[n][a][j] L[n][b][i], w = 2 for p < q, 1 for p = q and 0 above:
+// the product D^T D of D[n][(a, j)] with the second indices of its rows and columns exchanged. Each
+// wavefront computes 64 x 64 of it from L in L2 (set-up only: 0.4 ms at N M = 4096, 640 vectors).
+__global__ __launch_bounds__(256, 2) void k_pair_table(int M, int NM, int K, const double* __restrict__ L,
+                                                       long ldl, double* __restrict__ B, long ldb) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, r16 = lane & 15;
+  const int r0 = blockIdx.y * 128 + (wave >> 1) * 64, s0 = blockIdx.x * 128 + (wave & 1) * 64;
+  d4 acc[4][4];
+#pragma unroll
+  for (int a = 0; a < 4; ++a)
+#pragma unroll
+    for (int b = 0; b < 4; ++b) acc[a][b] = d4{0, 0, 0, 0};
+  for (int n0 = 0; n0 < K; n0 += 4) {
+    const int n = n0 + g;
+    const double* row = L + (long)min(n, K - 1) * ldl;
+    double x[4], y[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      x[t] = row[min(r0 + 16 * t + r16, NM - 1)];
+      y[t] = row[min(s0 + 16 * t + r16, NM - 1)];
+      if (n >= K) x[t] = y[t] = 0.0;
+    }
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int b = 0; b < 4; ++b) acc[a][b] = mfma16x16x4(x[a], y[b], acc[a][b]);
+  }
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    const int sc = s0 + 16 * b + r16, eb = sc / M, i = sc - eb * M;
+    if (sc >= NM) continue;
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int rr = r0 + 16 * a + acc_row<double>(g, r);
+        if (rr >= NM) continue;
+        const int ea = rr / M, j = rr - ea * M, q = eb * M + j, p = ea * M + i;
+        B[(long)q * ldb + p] = p < q ? 2.0 * acc[a][b][r] : (p == q ? acc[a][b][r] : 0.0);
+      }
+  }
+}
+
+// chunk of the quadratic form's k and its partials per row (DOT, columns in tiles of 64): the smallest
+// chunk from 128 on with at most max_parts partials and no more workgroups than 16 rounds of two per CU
+struct PairPlan {
+  int tm, chunk, parts;
+};
+PairPlan pair_plan(int W, int NM, int max_parts) {
+  PairPlan p;
+  // rows of a tile: the largest that pads the walkers (almost) no more than the next smaller one
+  auto pad = [&](int t) { return (long)(W + t - 1) / t * t; };
+  p.tm = pad(128) * 20 <= pad(32) * 21 ? 128 : (pad(64) * 20 <= pad(32) * 21 ? 64 : 32);
+  const int nt = (NM + 63) / 64;
+  for (p.chunk = 128;; p.chunk *= 2) {
+    const int c = p.chunk / 64;
+    p.parts = 0;
+    for (int t = 0; t < nt; ++t) p.parts += t / c + 1;
+    if (c >= nt || (p.parts <= max_parts && p.parts * (pad(p.tm) / p.tm) <= 32L * device_cus())) return p;
+  }
+}
+
 }  // namespace
+
+size_t pair_table_elems(int NM) { return (size_t)NM * gemm_real_row(NM); }
+
+void launch_pair_table(hipStream_t s, int M, int N, int K, const double* Lvb, double* B) {
+  const int NM = N * M, nt = (NM + 127) / 128;
+  AFQ_HIP(hipMemsetAsync(B, 0, pair_table_elems(NM) * sizeof(double), s));   // the rows' padding
+  hipLaunchKernelGGL(k_pair_table, dim3(nt, nt), dim3(256), 0, s, M, NM, K, Lvb, (long)gemm_real_row(NM),
+                     B, (long)gemm_real_row(NM));
+  AFQ_HIP(hipGetLastError());
+}
+
+int pair_parts(int W, int NM, int max_parts) { return pair_plan(W, NM, max_parts).parts; }
+
+void launch_pair_exchange(hipStream_t s, int W, int NM, int max_parts, const double* G, const double* B,
+                          double* part) {
+  if (W <= 0) return;
+  const PairPlan p = pair_plan(W, NM, max_parts);
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(p.parts, (W + p.tm - 1) / p.tm), dim3(256), 0, s, W, NM, NM, p.chunk, 1.0, G,
+                       (long)NM, B, (long)gemm_real_row(NM), part, (long)p.parts, 0L, 1);
+  };
+  if (p.tm == 128) go(k_gemm_real<double, 128, 64, 8, true>);
+  else if (p.tm == 64) go(k_gemm_real<double, 64, 64, 16, true>);
+  else go(k_gemm_real<double, 32, 64, 16, true>);
+  AFQ_HIP(hipGetLastError());
+}
 
 int gemm_real_row(int k) { return (k + 15) / 16 * 16; }
 

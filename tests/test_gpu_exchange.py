@@ -95,3 +95,27 @@ def test_energy_keeps_non_finite_walkers_apart(shape, complex_trial, form):
             assert not np.isfinite(got[w, 1:].real).any()
         else:
             assert np.array_equal(got[w], clean[w])
+
+
+# enough walkers and vectors for the pair table: walker tiles of 32, 64 and 128 with remainders, column
+# tiles with remainders, chunks of one and of several tiles, one tile in all, more than 128 orbitals
+PAIR_SHAPES = [(33, 17, 300, 290), (40, 3, 600, 2000), (50, 1, 3000, 5000), (64, 16, 200, 128),
+               (77, 19, 200, 65), (96, 32, 420, 33), (128, 32, 70, 300), (130, 20, 150, 70)]
+
+
+@pytest.mark.parametrize("shape", PAIR_SHAPES)
+@pytest.mark.parametrize("form", [0, 1, 3])
+def test_energy_pair_table(shape, form):
+    if form == 3 and shape[0] > 128:
+        pytest.skip("no int8 form")
+    if form and (shape[1] == 1 or shape[2] < 1.5 * shape[0]):
+        pytest.skip("one electron or few vectors: no table in the mixed forms")
+    h, L, PsiT, G = make(*shape, False)
+    G[1, 0, 3] = complex(0.5, np.inf)
+    got = energies(h, L, PsiT, G, form)
+    assert not np.isfinite(got[1, 1:].real).any()
+    some = np.r_[0, 2:12, shape[3] - 10:shape[3]]
+    want, _ = reference(h, L, PsiT, G[some])
+    _, scale = reference(np.abs(h), np.abs(L), np.abs(PsiT), np.abs(G[some]))
+    # sums of up to N M + K rounded products, whatever their order (E1: FP64 in every form)
+    assert np.max(np.abs(got[some] - want) / scale) < 1e-13
