@@ -153,29 +153,32 @@ VKind run_vhs_step(afq_ham H, hipStream_t s, int W, const double* X, double* V, 
 const double* P1r_of(afq_ham H) { return H->P1_real ? H->P1r : nullptr; }
 
 // Times (us) of the energy contractions: as T_n = G Lnak_n^T per Cholesky vector (4 N^2 M K flops per
-// walker) and with the pair table (2 (N M)^2, half of the square, and 4 N M K for the Coulomb traces).
-// The rates are those measured at M 128, N 32, K 640, 1024 walkers in FP64 and in the int8 form (FP32 and
-// BF16X3 are slower than that), the constants are the launches of small cases: M 24, N 6, K 96, 64
-// walkers take 8 us per vector and would take 15 with the table.
+// walker) and with the pair table (2 (N M)^2, half of the square, and 4 N M K for the Coulomb traces);
+// twice the flops for complex trials. The rates are those measured at M 128, N 32, K 640, 1024 walkers
+// in FP64 and in the int8 form (FP32 and BF16X3 are slower than that), the constants are the launches
+// of small cases: M 24, N 6, K 96, 64 walkers take 8 us per vector and would take 15 with the table.
 double exchange_us(afq_ham H, int W) {
   const double rows = (W + 3) / 4 * 4, rate = H->precision == AFQ_FP64 ? 50e6 : 130e6;
-  return (H->precision == AFQ_FP64 ? 4.0 : 15.0) + 4.0 * rows * H->N * H->N * H->M * H->K / rate;
+  const double flops = (H->real_trial ? 4.0 : 8.0) * rows * H->N * H->N * H->M * H->K;
+  return (H->precision == AFQ_FP64 ? 4.0 : 15.0) + flops / rate;
 }
-double pairs_us(int W, int NM, int K) {
-  const double rows = (W + 31) / 32 * 32;
-  return 15.0 + rows * NM * (2.0 * NM + 4.0 * K) / 60e6;
+double pairs_us(afq_ham H, int W) {
+  const double rows = (W + 31) / 32 * 32, NM = (double)H->N * H->M;
+  return 15.0 + (H->real_trial ? 1.0 : 2.0) * rows * NM * (2.0 * NM + 4.0 * H->K) / 60e6;
 }
-bool use_pairs(afq_ham H, int W) {
-  return H->pairs != nullptr && pairs_us(W, H->N * H->M, H->K) < exchange_us(H, W);
-}
+bool use_pairs(afq_ham H, int W) { return H->pairs != nullptr && pairs_us(H, W) < exchange_us(H, W); }
 
 // the exchange contraction in the handle's precision: Kl and per-chunk tr(T^2) partials
 void run_exchange(afq_ham H, hipStream_t s, int W, const double* G) {
   if (use_pairs(H, W)) {
     const int NM = H->N * H->M;
-    launch_gemm_real(s, AFQ_FP64, W, H->K, NM, 1.0, G, NM, H->Lvb_d, H->ws.Kl, H->K, true, H->ws.esplit,
-                     H->ws.esplit_elems);
-    launch_pair_exchange(s, W, NM, H->K + 1, G, H->pairs, H->ws.exx);
+    if (H->real_trial)
+      launch_gemm_real(s, AFQ_FP64, W, H->K, NM, 1.0, G, NM, H->Lvb_d, H->ws.Kl, H->K, true, H->ws.esplit,
+                       H->ws.esplit_elems);
+    else
+      launch_gemm_nt_z(s, AFQ_FP64, W, H->K, NM, 1.0, G, NM, H->Lnak, NM, true, H->ws.Kl, H->K, H->ws.esplit,
+                       H->ws.esplit_elems);
+    launch_pair_exchange(s, W, NM, H->real_trial, H->K + 1, G, H->pairs, H->ws.exx);
   } else if (H->precision == AFQ_BF16X3)
     launch_exchange_bf16(s, W, H->M, H->N, H->K, G, H->Lnak_b, H->ws.Kl, H->ws.exx);
   else if (H->precision == AFQ_INT8_SPLIT)
@@ -188,7 +191,7 @@ void run_exchange(afq_ham H, hipStream_t s, int W, const double* G) {
 }
 
 int exchange_chunks(afq_ham H, int W) {
-  if (use_pairs(H, W)) return pair_parts(W, H->N * H->M, H->K + 1);
+  if (use_pairs(H, W)) return pair_parts(W, H->N * H->M, H->real_trial, H->K + 1);
   if (H->precision == AFQ_BF16X3) return exchange_bf16_chunks(W, H->N, H->K);
   if (H->precision == AFQ_INT8_SPLIT) return exchange_i8_chunks(W, H->M, H->N, H->K, H->real_trial);
   if (H->precision == AFQ_FP64 && exchange_f64_supported(H->M, H->N))
@@ -312,11 +315,11 @@ int afq_ham_create(int M, int N, int K, const double* h_h, const double* h_Likn,
         launch_pad_rows(nullptr, K, (int)NM, 0, H->Lnak, true, H->Lvb_d);
         launch_pad_rows(nullptr, K, (int)NM, 0, H->Lnak, true, H->Lvb_f);
       }
-      // at most 2 GiB (N M = 16384), and only where it is the fewer operations for many walkers
-      if (H->real_trial && pair_table_elems((int)NM) <= (size_t)1 << 28 && NM / 64 + 1 <= (size_t)K &&
-          pairs_us(32768, (int)NM, K) < exchange_us(H, 32768)) {
-        if (hipMalloc(&H->pairs, pair_table_elems((int)NM) * sizeof(double)) == hipSuccess) {
-          launch_pair_table(nullptr, M, N, K, H->Lvb_d, H->pairs);
+      // at most 2 GiB (N M = 16384 for a real trial), and only where many walkers take fewer operations
+      const size_t pe = pair_table_elems((int)NM, H->real_trial);
+      if (pe <= (size_t)1 << 28 && 2 * (NM / 64 + 1) <= (size_t)K && pairs_us(H, 32768) < exchange_us(H, 32768)) {
+        if (hipMalloc(&H->pairs, pe * sizeof(double)) == hipSuccess) {
+          launch_pair_table(nullptr, M, N, K, H->real_trial ? H->Lvb_d : H->Lnak, H->real_trial, H->pairs);
         } else {
           H->pairs = nullptr;   // the exchange kernels need no table
           (void)hipGetLastError();

@@ -176,7 +176,7 @@ struct afq_ham_s {
   bool P1_real = false;
   double* Lvb_d = nullptr;   // f64 [K][N*M padded to 16]: real Lnak rows (vbias of a real trial)
   float* Lvb_f = nullptr;    // f32 copy
-  double* pairs = nullptr;   // f64 [N*M][N*M padded to 16]: pair table of the exchange (may be absent)
+  double* pairs = nullptr;   // f64 [re(, im)][N*M][N*M padded to 16]: pair table of the exchange (may be absent)
   double* Lp_d = nullptr;    // f64 [M(M+1)/2][K padded to 16]: rows i <= j of Likn (symmetric vHS)
   float* Lp_f = nullptr;     // f32 copy
   double* Lnak_r = nullptr;  // f64 [K][N][M padded to 16]: Re Lnak, only with a real trial
@@ -239,15 +239,16 @@ void launch_pad_rows(hipStream_t s, long rows, int k, int packed_n, const double
 void launch_gemm_real(hipStream_t s, int precision, int m, int n, int k, double alpha,
                       const double* A, long lda, const void* B, double* C, long ldc, bool nanmix,
                       double* split_ws = nullptr, long split_ws_elems = 0, int cfg = 0);
-// k_gemm_real.hip: the exchange sum_n tr(T_n^2) of a real trial as the quadratic form G B G^T of the
-// flat rows G[w][(a, i)], B[(b, j)][(a, i)] = sum_n Lnak[n][b][i] Lnak[n][a][j] (upper triangle, off-diagonal
-// entries doubled); Lvb: real Lnak rows of gemm_real_row(N M). At most max_parts partials per walker
-// (the smallest possible number is 1 + (N M - 1) / 64).
-size_t pair_table_elems(int NM);
-void launch_pair_table(hipStream_t s, int M, int N, int K, const double* Lvb, double* B);
-int pair_parts(int W, int NM, int max_parts);
-void launch_pair_exchange(hipStream_t s, int W, int NM, int max_parts, const double* G, const double* B,
-                          double* part);
+// k_gemm_real.hip: the exchange sum_n tr(T_n^2) as the quadratic form G B G^T of the flat rows
+// G[w][(a, i)], B[(b, j)][(a, i)] = sum_n Lnak[n][b][i] Lnak[n][a][j] (upper triangle, off-diagonal
+// entries doubled; a real and, unless Lnak is real, an imaginary table). L: Lnak (c128 [K][N M]) or its
+// real rows of gemm_real_row(N M). At most max_parts partials per walker (1 + (N M - 1) / 64 per table
+// are always possible).
+size_t pair_table_elems(int NM, bool real);
+void launch_pair_table(hipStream_t s, int M, int N, int K, const double* L, bool real, double* B);
+int pair_parts(int W, int NM, bool real, int max_parts);
+void launch_pair_exchange(hipStream_t s, int W, int NM, bool real, int max_parts, const double* G,
+                          const double* B, double* part);
 // k_energy.hip
 int device_cus();                        // compute units of the current device (cached)
 int exx_nchunks(int W, int N, int K);   // chunks of Cholesky vectors the exchange kernel uses

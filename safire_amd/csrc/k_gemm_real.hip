@@ -24,6 +24,7 @@
 //   M 128, N 32, K 640, 1024 walkers: FP64 6500, int8 2560 -> 830 + 264 us
 //   M 64, N 16, K 256, 512 walkers: int8 166 -> 56 + 23 us
 //   M 88, N 22, K 440, 137 walkers: int8 240 -> 49 + 27 us
+//   M 77, N 19, K 385, 201 walkers, complex trial: FP64 490 -> 61 + 44 us
 #include "afq_internal.hpp"
 
 #include <algorithm>
@@ -36,6 +37,7 @@ namespace {
 // holds the entries p <= q). Workgroup (x, y) takes item x, columns of tile_n times one chunk of the
 // k <= its last column, and rows of tile y; it writes sum_q (A B)[row][q] A[row][q] over its share as
 // partial x of the row (C[row][ldc]). The items of a tile_n follow one another, kchunk a multiple of TN.
+// z = 1: the imaginary part of B, which follows the real part; its partials follow, times i.
 template <typename R, int TM, int TN, int KS, bool DOT = false>
 __global__ __launch_bounds__(256, 2) void k_gemm_real(int m, int n, int k, int kchunk, double alpha,
                                                       const double* __restrict__ A, long lda,
@@ -66,10 +68,11 @@ __global__ __launch_bounds__(256, 2) void k_gemm_real(int m, int n, int k, int k
     for (; x >= j * c; ++j) x -= j * c;
     tile_n = (j - 1) * c + x / j;
     kbeg = x % j * kchunk;
+    B += blockIdx.z * (long)n * ldb;
   }
   const int tile_m = blockIdx.y;
   const int kend = min(DOT ? min(k, (tile_n + 1) * TN) : k, kbeg + kchunk);
-  C += blockIdx.z * split_stride;
+  if (!DOT) C += blockIdx.z * split_stride;
 
   double2 pa[PA];
   uint4 pb[PB];
@@ -205,8 +208,10 @@ __global__ __launch_bounds__(256, 2) void k_gemm_real(int m, int n, int k, int k
     __syncthreads();
     if (tid < TM && tile_m * TM + tid < m) {
       const double2 x = red[tid], y = red[TM + tid];
-      *reinterpret_cast<double2*>(C + 2 * ((long)(tile_m * TM + tid) * ldc + blockIdx.x)) =
-          double2{x.x + y.x, x.y + y.y};
+      const double re = x.x + y.x, im = x.y + y.y;
+      *reinterpret_cast<double2*>(
+          C + 2 * ((long)(tile_m * TM + tid) * ldc + blockIdx.z * gridDim.x + blockIdx.x)) =
+          blockIdx.z ? double2{-im, re} : double2{re, im};
     }
     return;
   }
@@ -250,8 +255,12 @@ __global__ void k_pad_rows(long rows, int k, int ldb, int n, int packed,
 // B[q = (b, j)][p = (a, i)] = w sum_n L[n][a][j] L[n][b][i], w = 2 for p < q, 1 for p = q and 0 above:
 // the product D^T D of D[n][(a, j)] with the second indices of its rows and columns exchanged. Each
 // wavefront computes 64 x 64 of it from L in L2 (set-up only: 0.4 ms at N M = 4096, 640 vectors).
+// LC: complex L, block z = 0 the real and z = 1 the imaginary part of B.
+template <bool LC>
 __global__ __launch_bounds__(256, 2) void k_pair_table(int M, int NM, int K, const double* __restrict__ L,
                                                        long ldl, double* __restrict__ B, long ldb) {
+  const bool imag = LC && blockIdx.z == 1;
+  B += blockIdx.z * (long)NM * ldb;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, r16 = lane & 15;
   const int r0 = blockIdx.y * 128 + (wave >> 1) * 64, s0 = blockIdx.x * 128 + (wave & 1) * 64;
   d4 acc[4][4];
@@ -262,17 +271,31 @@ __global__ __launch_bounds__(256, 2) void k_pair_table(int M, int NM, int K, con
   for (int n0 = 0; n0 < K; n0 += 4) {
     const int n = n0 + g;
     const double* row = L + (long)min(n, K - 1) * ldl;
-    double x[4], y[4];
+    double x[4], y[4], x2[4], y2[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-      x[t] = row[min(r0 + 16 * t + r16, NM - 1)];
-      y[t] = row[min(s0 + 16 * t + r16, NM - 1)];
-      if (n >= K) x[t] = y[t] = 0.0;
+      const int rr = min(r0 + 16 * t + r16, NM - 1), sc = min(s0 + 16 * t + r16, NM - 1);
+      if (LC) {
+        const double2 xc = reinterpret_cast<const double2*>(row)[rr];
+        const double2 yc = reinterpret_cast<const double2*>(row)[sc];
+        x[t] = xc.x;
+        x2[t] = imag ? xc.y : -xc.y;
+        y[t] = imag ? yc.y : yc.x;
+        y2[t] = imag ? yc.x : yc.y;
+      } else {
+        x[t] = row[rr];
+        y[t] = row[sc];
+        x2[t] = 0.0;
+      }
+      if (n >= K) x[t] = x2[t] = 0.0;
     }
 #pragma unroll
     for (int a = 0; a < 4; ++a)
 #pragma unroll
-      for (int b = 0; b < 4; ++b) acc[a][b] = mfma16x16x4(x[a], y[b], acc[a][b]);
+      for (int b = 0; b < 4; ++b) {
+        acc[a][b] = mfma16x16x4(x[a], y[b], acc[a][b]);
+        if (LC) acc[a][b] = mfma16x16x4(x2[a], y2[b], acc[a][b]);
+      }
   }
 #pragma unroll
   for (int b = 0; b < 4; ++b) {
@@ -311,25 +334,31 @@ PairPlan pair_plan(int W, int NM, int max_parts) {
 
 }  // namespace
 
-size_t pair_table_elems(int NM) { return (size_t)NM * gemm_real_row(NM); }
+size_t pair_table_elems(int NM, bool real) { return (real ? 1 : 2) * (size_t)NM * gemm_real_row(NM); }
 
-void launch_pair_table(hipStream_t s, int M, int N, int K, const double* Lvb, double* B) {
+void launch_pair_table(hipStream_t s, int M, int N, int K, const double* L, bool real, double* B) {
   const int NM = N * M, nt = (NM + 127) / 128;
-  AFQ_HIP(hipMemsetAsync(B, 0, pair_table_elems(NM) * sizeof(double), s));   // the rows' padding
-  hipLaunchKernelGGL(k_pair_table, dim3(nt, nt), dim3(256), 0, s, M, NM, K, Lvb, (long)gemm_real_row(NM),
-                     B, (long)gemm_real_row(NM));
+  const long ldb = gemm_real_row(NM);
+  AFQ_HIP(hipMemsetAsync(B, 0, pair_table_elems(NM, real) * sizeof(double), s));   // the rows' padding
+  if (real)
+    hipLaunchKernelGGL(k_pair_table<false>, dim3(nt, nt), dim3(256), 0, s, M, NM, K, L, ldb, B, ldb);
+  else
+    hipLaunchKernelGGL(k_pair_table<true>, dim3(nt, nt, 2), dim3(256), 0, s, M, NM, K, L, 2L * NM, B, ldb);
   AFQ_HIP(hipGetLastError());
 }
 
-int pair_parts(int W, int NM, int max_parts) { return pair_plan(W, NM, max_parts).parts; }
+int pair_parts(int W, int NM, bool real, int max_parts) {
+  return real ? pair_plan(W, NM, max_parts).parts : 2 * pair_plan(W, NM, max_parts / 2).parts;
+}
 
-void launch_pair_exchange(hipStream_t s, int W, int NM, int max_parts, const double* G, const double* B,
-                          double* part) {
+void launch_pair_exchange(hipStream_t s, int W, int NM, bool real, int max_parts, const double* G,
+                          const double* B, double* part) {
   if (W <= 0) return;
-  const PairPlan p = pair_plan(W, NM, max_parts);
+  const int planes = real ? 1 : 2;
+  const PairPlan p = pair_plan(W, NM, max_parts / planes);
   auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3(p.parts, (W + p.tm - 1) / p.tm), dim3(256), 0, s, W, NM, NM, p.chunk, 1.0, G,
-                       (long)NM, B, (long)gemm_real_row(NM), part, (long)p.parts, 0L, 1);
+    hipLaunchKernelGGL(kern, dim3(p.parts, (W + p.tm - 1) / p.tm, planes), dim3(256), 0, s, W, NM, NM, p.chunk,
+                       1.0, G, (long)NM, B, (long)gemm_real_row(NM), part, (long)planes * p.parts, 0L, 1);
   };
   if (p.tm == 128) go(k_gemm_real<double, 128, 64, 8, true>);
   else if (p.tm == 64) go(k_gemm_real<double, 64, 64, 16, true>);

@@ -103,14 +103,15 @@ PAIR_SHAPES = [(33, 17, 300, 290), (40, 3, 600, 2000), (50, 1, 3000, 5000), (64,
                (77, 19, 200, 65), (96, 32, 420, 33), (128, 32, 70, 300), (130, 20, 150, 70)]
 
 
+@pytest.mark.parametrize("complex_trial", [False, True])
 @pytest.mark.parametrize("shape", PAIR_SHAPES)
 @pytest.mark.parametrize("form", [0, 1, 3])
-def test_energy_pair_table(shape, form):
+def test_energy_pair_table(shape, form, complex_trial):
     if form == 3 and shape[0] > 128:
         pytest.skip("no int8 form")
     if form and (shape[1] == 1 or shape[2] < 1.5 * shape[0]):
         pytest.skip("one electron or few vectors: no table in the mixed forms")
-    h, L, PsiT, G = make(*shape, False)
+    h, L, PsiT, G = make(*shape, complex_trial)
     G[1, 0, 3] = complex(0.5, np.inf)
     got = energies(h, L, PsiT, G, form)
     assert not np.isfinite(got[1, 1:].real).any()
