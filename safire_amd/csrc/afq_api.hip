@@ -415,8 +415,8 @@ int afq_ham_reserve(afq_ham H, int max_walkers) {
     dalloc(&ws.exx, 2 * W * (size_t)(K + 2));   // at most K + 1 tr(T^2) partials per walker
     ws.split_elems = (long)kMaxSplits * W * K;
     dalloc(&ws.split, 2 * (size_t)ws.split_elems);
-    if (H->pairs) {   // 32 MiB at most: products with more entries fill the chip unsplit
-      ws.esplit_elems = std::min((long)kMaxSplits * max_walkers * H->K, 1L << 21);
+    if (H->pairs) {   // 128 MiB at most: products with more entries fill the chip unsplit
+      ws.esplit_elems = std::min((long)kMaxSplits * max_walkers * H->K, 1L << 23);
       dalloc(&ws.esplit, 2 * (size_t)ws.esplit_elems);
     }
     dalloc(&ws.cum, W);

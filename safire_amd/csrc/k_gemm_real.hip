@@ -28,15 +28,18 @@
 #include "afq_internal.hpp"
 
 #include <algorithm>
+#include <cmath>
 
 namespace afq {
 
 namespace {
 
+constexpr int kXcds = 8;   // workgroups are dealt to them in turn
+
 // DOT: the quadratic form A B A^T of each row instead of C, B being n x n and upper triangular (row q
-// holds the entries p <= q). Workgroup (x, y) takes item x, columns of tile_n times one chunk of the
-// k <= its last column, and rows of tile y; it writes sum_q (A B)[row][q] A[row][q] over its share as
-// partial x of the row (C[row][ldc]). The items of a tile_n follow one another, kchunk a multiple of TN.
+// holds the entries p <= q). A workgroup takes an item, columns of tile_n times one chunk of the
+// k <= its last column, and rows of a tile; it writes sum_q (A B)[row][q] A[row][q] over its share as
+// that partial of the row (C[row][ldc]). kchunk is a multiple of TN.
 // z = 1: the imaginary part of B, which follows the real part; its partials follow, times i.
 template <typename R, int TM, int TN, int KS, bool DOT = false>
 __global__ __launch_bounds__(256, 2) void k_gemm_real(int m, int n, int k, int kchunk, double alpha,
@@ -61,16 +64,21 @@ __global__ __launch_bounds__(256, 2) void k_gemm_real(int m, int n, int k, int k
   const int wm = (wave >> 1) * (TM / 2), wn = (wave & 1) * (TN / 2);
   // column tiles fastest: consecutive workgroups (dealt round-robin to the XCDs) share rows of A,
   // and each XCD's L2 holds an eighth of B
-  int tile_n = blockIdx.x, kbeg = blockIdx.z * kchunk;
-  if (DOT) {   // items of tile_n: tile_n / c + 1, so c tiles of j items each for j = 1, 2, ...
+  int tile_n = blockIdx.x, tile_m = blockIdx.y, kbeg = DOT ? 0 : blockIdx.z * kchunk, item = 0;
+  if (DOT) {
+    // each XCD takes a contiguous range of (tile_m, item), and the items of a chunk, one per tile_n from
+    // the chunk's first column on, follow one another: its L2 holds the rows of A that they share
+    const int nitem = gridDim.x, total = nitem * gridDim.y, b = blockIdx.x + nitem * blockIdx.y;
+    const int q = total / kXcds, r = total % kXcds, xcd = b % kXcds;
+    const int at = xcd * q + min(xcd, r) + b / kXcds;
+    tile_m = at / nitem;
+    item = at - tile_m * nitem;
     const int c = kchunk / TN;
-    int x = blockIdx.x, j = 1;
-    for (; x >= j * c; ++j) x -= j * c;
-    tile_n = (j - 1) * c + x / j;
-    kbeg = x % j * kchunk;
+    int x = item, len = (n + TN - 1) / TN;
+    for (; x >= len; len -= c, kbeg += kchunk) x -= len;
+    tile_n = kbeg / TN + x;
     B += blockIdx.z * (long)n * ldb;
   }
-  const int tile_m = blockIdx.y;
   const int kend = min(DOT ? min(k, (tile_n + 1) * TN) : k, kbeg + kchunk);
   if (!DOT) C += blockIdx.z * split_stride;
 
@@ -210,7 +218,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_real(int m, int n, int k, int k
       const double2 x = red[tid], y = red[TM + tid];
       const double re = x.x + y.x, im = x.y + y.y;
       *reinterpret_cast<double2*>(
-          C + 2 * ((long)(tile_m * TM + tid) * ldc + blockIdx.z * gridDim.x + blockIdx.x)) =
+          C + 2 * ((long)(tile_m * TM + tid) * ldc + blockIdx.z * gridDim.x + item)) =
           blockIdx.z ? double2{-im, re} : double2{re, im};
     }
     return;
@@ -332,6 +340,31 @@ PairPlan pair_plan(int W, int NM, int max_parts) {
   }
 }
 
+// FP64: the tile and the split of k with the shortest estimated time: workgroups of the fullest CU times
+// the work of one (234 MFLOP/s per us and CU where workgroups share it, 0.6 of it for one alone; the
+// smaller tiles at 0.95 and 0.8 of that), and the pass that adds the splits.
+void gemm_f64_plan(int m, int n, int k, long split_elems, int& tm, int& tn, int& splits) {
+  const double cus = device_cus();
+  double best = 1e300;
+  const int tiles[3][2] = {{128, 64}, {64, 64}, {64, 32}};
+  const double eff[3] = {1.0, 0.95, 0.8};
+  for (int t = 0; t < 3; ++t)
+    for (int s = 1; s <= kMaxSplits; ++s) {
+      if (s > 1 && (k / s < 128 || (long)s * m * n > split_elems)) break;
+      const double wgs = std::ceil((double)m / tiles[t][0]) * std::ceil((double)n / tiles[t][1]) * s;
+      const double share = std::ceil(wgs / cus);
+      double us = share * 4.0 * tiles[t][0] * tiles[t][1] * std::ceil((double)k / s) / (0.234e6 * eff[t]);
+      if (share < 2) us /= 0.6;
+      if (s > 1) us += 4.0 + 16e-6 * m * (double)n * (s + 1) / 4.0;
+      if (us < 0.98 * best) {
+        best = us;
+        tm = tiles[t][0];
+        tn = tiles[t][1];
+        splits = s;
+      }
+    }
+}
+
 }  // namespace
 
 size_t pair_table_elems(int NM, bool real) { return (real ? 1 : 2) * (size_t)NM * gemm_real_row(NM); }
@@ -392,21 +425,22 @@ void launch_gemm_real(hipStream_t s, int precision, int m, int n, int k, double 
   // the splits of launch_gemm_nt_z: the FP32 sums keep their order
   int splits = split_ws ? gemm_splits(m, n, k) : 1;
   if ((long)splits * m * n > split_ws_elems) splits = 1;
+  int tm = 64, tn = 32;
+  if (!f32) gemm_f64_plan(m, n, k, split_ws ? split_ws_elems : 0, tm, tn, splits);
   int kchunk = (k + splits - 1) / splits;
   kchunk = (kchunk + 31) & ~31;
   splits = std::max(1, (k + kchunk - 1) / kchunk);
-  // The largest tile that still gives two workgroups per CU (128 x 128 FP32: four, so that a partly
+  // FP32: the largest tile that still gives two workgroups per CU (128 x 128: four, so that a partly
   // filled last round costs little), else 64 x 32: 512 walkers of 64 orbitals are 264 64 x 64 tiles
   // of vHS, one workgroup on most CUs with every load exposed.
   // cfg (FP32; 0: this rule) bit 0: the other row count, bit 1: the other column count.
-  const long cus = device_cus();
-  auto tiles = [&](int tm, int tn) {
-    return (long)((m + tm - 1) / tm) * ((n + tn - 1) / tn) * splits;
-  };
-  int tm = 64, tn = 32;
-  if (f32 && tiles(128, 128) >= 4 * cus) tm = tn = 128;
-  else if (tiles(128, 64) >= 2 * cus) tm = 128, tn = 64;
-  else if (tiles(64, 64) >= 2 * cus) tn = 64;
+  if (f32) {
+    const long cus = device_cus();
+    auto tiles = [&](int a, int b) { return (long)((m + a - 1) / a) * ((n + b - 1) / b) * splits; };
+    if (tiles(128, 128) >= 4 * cus) tm = tn = 128;
+    else if (tiles(128, 64) >= 2 * cus) tm = 128, tn = 64;
+    else if (tiles(64, 64) >= 2 * cus) tn = 64;
+  }
   if (f32 && (cfg & 1)) tm = tm == 64 ? 128 : 64;
   if (f32 && (cfg & 2)) tn = tn == 64 ? 128 : 64;
   if (tm == 128 && tn == 32) tn = 64;
