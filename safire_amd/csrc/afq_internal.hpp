@@ -105,6 +105,24 @@ template <typename R> struct acc_of;
 template <> struct acc_of<double> { typedef d4 type; };
 template <> struct acc_of<float> { typedef f4 type; };
 
+// v plus the value of the lane `shift` below in the same row of 16 lanes (0 below the row)
+template <int SHIFT>
+__device__ inline double add_row_shr(double v) {
+  const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+  const unsigned lo = __builtin_amdgcn_update_dpp(0u, (unsigned)u, 0x110 + SHIFT, 0xf, 0xf, true);
+  const unsigned hi =
+      __builtin_amdgcn_update_dpp(0u, (unsigned)(u >> 32), 0x110 + SHIFT, 0xf, 0xf, true);
+  return v + __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+
+// lane 15 of each row of 16 lanes receives the sum of the row (DPP row shifts, no LDS)
+__device__ inline double row_sum16(double v) {
+  v = add_row_shr<1>(v);
+  v = add_row_shr<2>(v);
+  v = add_row_shr<4>(v);
+  return add_row_shr<8>(v);
+}
+
 // ------------------------------------------------------------------ engine state
 struct Workspace {
   int cap = 0;

@@ -92,24 +92,6 @@ __device__ inline i4 mfma_i8(i4 a, i4 b, i4 c) {
 // are not waited for. The memory clobber keeps the compiler from moving memory accesses across.
 __device__ inline void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// v plus the value of the lane `shift` below in the same row of 16 lanes (0 below the row)
-template <int SHIFT>
-__device__ inline double add_row_shr(double v) {
-  const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
-  const unsigned lo = __builtin_amdgcn_update_dpp(0u, (unsigned)u, 0x110 + SHIFT, 0xf, 0xf, true);
-  const unsigned hi =
-      __builtin_amdgcn_update_dpp(0u, (unsigned)(u >> 32), 0x110 + SHIFT, 0xf, 0xf, true);
-  return v + __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
-}
-
-// lane 15 of each row of 16 lanes receives the sum of the row (DPP row shifts, no LDS)
-__device__ inline double row_sum16(double v) {
-  v = add_row_shr<1>(v);
-  v = add_row_shr<2>(v);
-  v = add_row_shr<4>(v);
-  return add_row_shr<8>(v);
-}
-
 template <int KC, int CT, bool LC, int NW>
 __global__ __launch_bounds__(64 * NW, NW / 4) void k_exchange_i8(
     int W, int M, int N, int K, int Mp, int Rw, int Cv, int chunk, int tdbl,

@@ -207,11 +207,9 @@ __global__ __launch_bounds__(256, 2) void k_gemm_real(int m, int n, int k, int k
             ei += cr[a][b][r] * x.y + ci[a][b][r] * x.x;
           }
         }
-        for (int off = 8; off > 0; off >>= 1) {
-          er += __shfl_xor(er, off, 16);
-          ei += __shfl_xor(ei, off, 16);
-        }
-        if (r16 == 0) red[(wave & 1) * TM + row] = double2{er, ei};
+        er = row_sum16(er);
+        ei = row_sum16(ei);
+        if (r16 == 15) red[(wave & 1) * TM + row] = double2{er, ei};
       }
     __syncthreads();
     if (tid < TM && tile_m * TM + tid < m) {
@@ -322,7 +320,7 @@ __global__ __launch_bounds__(256, 2) void k_pair_table(int M, int NM, int K, con
 }
 
 // chunk of the quadratic form's k and its partials per row (DOT, columns in tiles of 64): the smallest
-// chunk from 128 on with at most max_parts partials and no more workgroups than 16 rounds of two per CU
+// chunk from 128 on with at most max_parts partials and no more than 64 workgroups per CU
 struct PairPlan {
   int tm, chunk, parts;
 };
@@ -336,7 +334,7 @@ PairPlan pair_plan(int W, int NM, int max_parts) {
     const int c = p.chunk / 64;
     p.parts = 0;
     for (int t = 0; t < nt; ++t) p.parts += t / c + 1;
-    if (c >= nt || (p.parts <= max_parts && p.parts * (pad(p.tm) / p.tm) <= 32L * device_cus())) return p;
+    if (c >= nt || (p.parts <= max_parts && p.parts * (pad(p.tm) / p.tm) <= 64L * device_cus())) return p;
   }
 }
 
