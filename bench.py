@@ -9,18 +9,19 @@ it (--extra) and its results are added under its name. Synthetic seeded inputs; 
 resident in HBM before the timed region.
 
 Every precision form of the same step is timed (--forms): the plain FP64 form and the mixed
-forms, which change only the Cholesky contractions (vbias and vHS in FP32; the exchange in FP32,
-three-slice BF16 or the int8 Ozaki split); G, overlaps, LU, QR, propagation, weights and energy
-sums stay FP64. Each form runs its timed steps twice from the same start: eagerly with region
+forms, which change only the Cholesky contractions (vbias and vHS in FP32; where the exchange runs
+per Cholesky vector, it is FP32, three-slice BF16 or the int8 Ozaki split; at these sizes it is the
+FP64 quadratic form over the pair table in every form); G, overlaps, LU, QR, propagation, weights
+and energy sums stay FP64. Each form runs its timed steps twice from the same start: eagerly with region
 timers (HIP events on the launch stream), then as one captured HIP graph replayed once; the
 graph's final walker buffer must equal the eager run's bit for bit (graph_matches_eager).
 `value` is the graph throughput of the fastest form whose largest per-walker
 |E_loc(form) - E_loc(FP64)| on identical walker states is below 1e-5 Ha; the line carries every
 form's throughput and gate error. A step = one pass over all walkers.
 
-roofline: the exchange-energy kernel (the dominant one), algorithmic FLOP per launch
-W*(8 N^2 M K + 8 N^2 K) divided by its mean duration measured with HIP events on the launch
-stream over the eager timed run. cpu_baseline: the C++ FP64 oracle (OpenMP over walkers) timed
+roofline: the exchange and Coulomb energy kernels (the dominant region), executed FP64 matrix FLOP
+per call W*(2 (N M)^2 + 4 N M K) divided by the region's mean duration measured with HIP events on
+the launch stream over the eager timed run. cpu_baseline: the C++ FP64 oracle (OpenMP over walkers) timed
 on this host on a bounded sample of the same workload.
 """
 from __future__ import annotations
@@ -37,44 +38,31 @@ if ROOT not in sys.path:
     sys.path.insert(0, ROOT)
 
 METRIC = "walker-steps/s mixed vs FP64 at |ΔE_loc|<1e-5 Ha; % MFMA/HBM peak"
-# dense MFMA peak of the arithmetic each form's exchange kernel runs on
-PEAK_TFLOPS = {"fp64": 78.6, "fp32": 157.3, "bf16x3": 2500.0, "int8": 5000.0}
-# executed MFMA flops per algorithmic flop of the exchange contraction
-# (BF16X3: 3 real products per complex product x 3 hi/lo terms = 18 flops per complex
-# multiply-add against the 8 counted; int8: the slice products per Cholesky vector, 15 for the
-# five-slice kernel of N <= 16, per-vector orders for N > 16 with their mean on the NMO=128 /
-# 32+32 / Nchol=640 workload read from the SQ_INSTS_VALU_MFMA_MOPS_I8 counter)
-EXECUTED_PER_ALGO = {"fp64": 1.0, "fp32": 1.0, "bf16x3": 18.0 / 8.0, "int8": 15.0}
-INT8_PRODUCTS = {"c3": 13.37}
-
-
-def executed_per_algo(form, workload):
-    if form == "int8":
-        return INT8_PRODUCTS.get(workload, EXECUTED_PER_ALGO["int8"])
-    return EXECUTED_PER_ALGO[form]
+# dense FP64 MFMA peak: the arithmetic of the exchange over the pair table
+PEAK_TFLOPS = {"fp64": 78.6}
 GATE_HA = 1e-5
-# HBM bytes per launch of each form's exchange kernel (FETCH_SIZE and WRITE_SIZE counter runs
-# scaled by a copy kernel of known size), as recorded in profiles/walker_step_c2_hbm_traffic.md;
-# null for a workload or form without such a measurement
-TRAFFIC_BYTES = {("c2", "int8"): 38.54e6, ("c2", "fp64"): 53.29e6,
-                 ("c3", "int8"): 586.57e6, ("c3", "fp64"): 21822.38e6,
-                 ("c3", "bf16x3"): 1739.17e6}
+# HBM bytes per launch of the quadratic form's kernel (FETCH_SIZE and WRITE_SIZE counter runs scaled
+# by a copy kernel of known size); None for a workload without such a measurement
+TRAFFIC_BYTES = {}
 TRAFFIC_SOURCE = {"c2": "profiles/walker_step_c2_hbm_traffic.md",
                   "c3": "profiles/walker_step_c3_hbm_traffic.md"}
 
 
 def exchange_flops(W, M, N, K):
-    return W * (8.0 * N * N * M * K + 8.0 * N * N * K)
+    """Executed FLOP of the energy contractions of a real trial: half of the (N M)^2 pair table and the
+    Coulomb traces, or, where those are fewer, the contractions per Cholesky vector."""
+    NM = N * M
+    return W * min(2.0 * NM * NM + 4.0 * NM * K, 4.0 * N * N * M * K)
 
 
 def step_flops(M, N, K):
-    """Algorithmic FLOP of one local-energy walker-step (complex MAC = 8, real x complex = 4)."""
+    """FLOP of one local-energy walker-step (complex MAC = 8, real x complex = 4)."""
     return (8 * M * N * N + 8 * N ** 3 + 8 * M * N * N      # T, LU + inverse, G
             + 8 * N * M * K                                  # vbias
             + 4 * M * M * K                                  # vHS
             + 16 * M * M * N + 48 * M * M * N                # 2 P1 products, Taylor-6
             + 16 * M * N * N + 8 * N ** 3 + 8 * N * M        # new G, LU/inverse, E1
-            + 8 * N * N * M * K + 8 * N * N * K              # exchange build + reduce
+            + exchange_flops(1, M, N, K)                     # exchange and Coulomb energy
             + (16 * M * N * N - 16 * N ** 3 / 3) / 5)        # QR every 5 steps
 
 
@@ -289,11 +277,14 @@ def bench_phmsd(args, A, torch, synth):
                                f"dt={s.dt}, local-energy step, QR every {ortho}",
                    "form": "FP64, eager launches", "ph_energy_algorithm": args.ph_energy,
                    "parallelism": "single GPU"},
+        # flop_per_launch counts every determinant's contractions; the rank-nex corrections of the
+        # woodbury energy execute fewer, so there is no fraction of peak for it
         "roofline": {"bound": "fp64 (vector ALU; no MFMA form)", "achieved": round(e_tf, 3),
                      "peak": PEAK_TFLOPS["fp64"], "unit": "TFLOP/s",
-                     "frac": round(e_tf / PEAK_TFLOPS["fp64"], 4), "traffic": None,
-                     "kernel": f"PHMSD local energy ({args.ph_energy}: k_ph_2body_lds "
-                               f"and companions, one call)" if args.ph_energy == "woodbury"
+                     "frac": None if args.ph_energy == "woodbury"
+                             else round(e_tf / PEAK_TFLOPS["fp64"], 4), "traffic": None,
+                     "kernel": "PHMSD local energy (woodbury: k_ph_exc and companions, one call)"
+                               if args.ph_energy == "woodbury"
                                else "PHMSD local energy (reference: k_ph0_inverse + k_ph0_chol, "
                                     "one call)",
                      "flop_per_launch": eflops, "mean_launch_ms": round(e_ms, 4)},
@@ -467,13 +458,12 @@ def bench_batch(args, A, torch, synth):
         "mixed_over_fp64": round(res["int8"]["batched_walker_steps_per_s"] /
                                  res["fp64"]["batched_walker_steps_per_s"], 3),
         "roofline": {"bound": "mfma", "achieved": res[head]["exchange_tflops"],
-                     "peak": PEAK_TFLOPS[head], "unit": "TFLOP/s",
-                     "frac": round(res[head]["exchange_tflops"] / PEAK_TFLOPS[head], 4),
+                     "peak": PEAK_TFLOPS["fp64"], "unit": "TFLOP/s",
+                     "frac": round(res[head]["exchange_tflops"] / PEAK_TFLOPS["fp64"], 4),
                      "traffic": None,
-                     "kernel": f"k_exchange ({head}) over all systems: total algorithmic FLOP / "
-                               f"total launch time, one-at-a-time timed run",
-                     "executed_frac": round(res[head]["exchange_tflops"] *
-                                            executed_per_algo(head, "c4") / PEAK_TFLOPS[head], 4)},
+                     "kernel": f"exchange and Coulomb energy ({head} form) over all systems: total "
+                               f"FLOP of the cheaper route / total launch time, one-at-a-time "
+                               f"timed run"},
         "cpu_baseline": None if args.no_cpu else batch_cpu_baseline(systems, ortho,
                                                                     args.cpu_seconds),
     }
@@ -572,8 +562,8 @@ def bench_single(args, A, torch, synth, workload, with_cpu, with_hybrid):
     ex_ms, ex_n = head["timers"]["exchange"]
     ex_avg = ex_ms / max(ex_n, 1)
     achieved = exchange_flops(W, M, N, K) / (ex_avg / 1e3) / 1e12
-    peak = PEAK_TFLOPS[mixed]
-    traffic = TRAFFIC_BYTES.get((workload, mixed))
+    peak = PEAK_TFLOPS["fp64"]
+    traffic = TRAFFIC_BYTES.get(workload)
     out = {
         "metric": METRIC,
         "value": round(value, 1),
@@ -596,11 +586,9 @@ def bench_single(args, A, torch, synth, workload, with_cpu, with_hybrid):
                      "traffic": traffic,
                      "traffic_unit": "bytes per launch",
                      "traffic_source": TRAFFIC_SOURCE.get(workload) if traffic else None,
-                     "kernel": f"k_exchange ({mixed} MFMA)",
+                     "kernel": "exchange (k_gemm_real, quadratic form) and Coulomb traces, FP64 MFMA",
                      "flop_per_launch": exchange_flops(W, M, N, K),
-                     "mean_launch_ms": round(ex_avg, 5),
-                     "executed_frac": round(achieved * executed_per_algo(mixed, workload) / peak,
-                                            4)},
+                     "mean_launch_ms": round(ex_avg, 5)},
     }
     if ref_form is not None:
         v64 = W * args.steps / (ref_form["ms"] / 1e3)
@@ -618,15 +606,14 @@ def bench_single(args, A, torch, synth, workload, with_cpu, with_hybrid):
     out["headline_form"] = mixed
     out["forms_walker_steps_per_s"] = {f: round(W * args.steps / (r["ms"] / 1e3), 1)
                                        for f, r in forms.items()}
-    # MFMA utilisation of each form's exchange kernel: executed MFMA operations per launch (the
-    # algorithmic count times the form's executed-per-algorithmic ratio) over its mean launch
-    # time, against the dense peak of the MFMA type it runs on
+    # MFMA utilisation of each form's energy region: executed FP64 matrix operations over its mean
+    # time, against the dense peak
     util = {}
     for f, r in forms.items():
         ms_, n_ = r["timers"]["exchange"]
         if n_:
             ex_rate = exchange_flops(W, M, N, K) / (ms_ / n_ / 1e3) / 1e12
-            util[f] = round(ex_rate * executed_per_algo(f, workload) / PEAK_TFLOPS[f], 4)
+            util[f] = round(ex_rate / PEAK_TFLOPS["fp64"], 4)
     out["exchange_mfma_utilisation"] = util
     if unsupported:
         out["forms_unsupported"] = unsupported
