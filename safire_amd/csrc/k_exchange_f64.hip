@@ -25,6 +25,8 @@
 //   M 128, N 32, K 640, 1024 walkers, real trial     19.2 -> 6.5 ms (73 % of what an 8192^3 FP64 GEMM reaches)
 //   M 77, N 19, K 385, 201 walkers, complex trial     1.27 -> 0.49 ms
 //   M 24, N 6, K 96, 64 walkers, real trial           27.9 -> 8.0 us
+// The first two now take the quadratic form over the pair table instead (k_gemm_real.hip); this kernel
+// runs the small calls and those with few vectors per orbital, where it is the faster one.
 #include "afq_internal.hpp"
 
 #include <algorithm>

@@ -32,8 +32,10 @@
 // What bounds it: neither unit alone. A pass is MFMAs (8 K of 12 K cycles at M = 128), pair sums and
 // the two barriers around the LDS store, and the two wavefronts of a SIMD go through them nearly
 // together. One walker's 32 x 32 blocks with complex slices, the form before, against this one:
-// M 64, N 16, K 256, W 512 real trial: 188 -> 166 us; M 128, N 32, K 640, W 1024: 4040 -> 2560 us;
+// M 64, N 16, K 320, W 512 real trial: 188 -> 166 us; M 128, N 32, K 640, W 1024: 4040 -> 2560 us;
 // M 88, N 22, K 440, W 137: 1055 -> 240 us.
+// With K of about 1.5 M and more and enough walkers the quadratic form over the pair table in FP64 is
+// still faster (k_gemm_real.hip: 61, 1020 and 69 us for these, traces included) and is taken instead.
 //
 // M <= 128, N <= 32.
 #include "afq_internal.hpp"

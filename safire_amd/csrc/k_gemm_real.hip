@@ -13,7 +13,7 @@
 // slice and wavefront; the 64 x 64 tiles of k_gemm_nt 8-byte reads of single elements for half as
 // many MFMAs, and twice the loads of B. Per launch, with the triangle of a symmetric vHS and the real
 // vectors of a real trial against k_gemm_nt on the full ones (M 128, N 32, K 640, 1024 walkers):
-// vHS FP64 905 -> 474 us, FP32 660 -> 288 us; vbias FP64 475 -> 227 us, FP32 277 -> 140 us. M 64,
+// vHS FP64 905 -> 484 us, FP32 660 -> 288 us; vbias FP64 475 -> 230 us, FP32 277 -> 140 us. M 64,
 // N 16, K 320, 512 walkers, FP64: vHS 68 -> 46 us.
 //
 // The exchange as a quadratic form: sum_n tr(T_n^2) with T_n = G Lnak_n^T is G B G^T over the pairs
@@ -21,10 +21,10 @@
 // symmetric: 2 (N M)^2 flops per walker instead of the 4 N^2 M K of the T_n, and with K some multiples
 // of M several times fewer, FP64 in place of the int8 split too. The Coulomb traces tr(T_n) are one
 // more product with the flat Lnak rows. Exchange and traces, per Cholesky vector -> pair table:
-//   M 128, N 32, K 640, 1024 walkers: FP64 6500, int8 2560 -> 830 + 264 us
-//   M 64, N 16, K 256, 512 walkers: int8 166 -> 56 + 23 us
-//   M 88, N 22, K 440, 137 walkers: int8 240 -> 49 + 27 us
-//   M 77, N 19, K 385, 201 walkers, complex trial: FP64 490 -> 61 + 44 us
+//   M 128, N 32, K 640, 1024 walkers: FP64 6500, int8 2560 -> 790 + 230 us
+//   M 64, N 16, K 320, 512 walkers: int8 166 -> 38 + 23 us
+//   M 88, N 22, K 440, 137 walkers: int8 240 -> 42 + 27 us
+//   M 77, N 19, K 385, 201 walkers, complex trial: FP64 490 -> 59 + 44 us
 #include "afq_internal.hpp"
 
 #include <algorithm>
@@ -319,23 +319,37 @@ __global__ __launch_bounds__(256, 2) void k_pair_table(int M, int NM, int K, con
   }
 }
 
-// chunk of the quadratic form's k and its partials per row (DOT, columns in tiles of 64): the smallest
-// chunk from 128 on with at most max_parts partials and no more than 64 workgroups per CU
+// Rows of a tile, chunk of k and partials per row and table of the quadratic form (columns in tiles of
+// 64). The chunk is the smallest from 128 on with at most max_parts partials and 64 workgroups per CU.
+// The tile is the largest unless a smaller one has 5 % less estimated time: rounds of the 2, 3 or 4
+// workgroups that a CU holds, a last one alone counting 1.6, times the rows (0.9 of the rate for 32).
+// 128, 64 and 32 rows take 48, 38 and 39 us at M 64, N 16 with 512 walkers; 64 and 32 rows 42 and 45
+// at M 88, N 22 with 137, and 70 and 59 at M 77, N 19 with 201 and two tables.
 struct PairPlan {
   int tm, chunk, parts;
 };
-PairPlan pair_plan(int W, int NM, int max_parts) {
-  PairPlan p;
-  // rows of a tile: the largest that pads the walkers (almost) no more than the next smaller one
-  auto pad = [&](int t) { return (long)(W + t - 1) / t * t; };
-  p.tm = pad(128) * 20 <= pad(32) * 21 ? 128 : (pad(64) * 20 <= pad(32) * 21 ? 64 : 32);
-  const int nt = (NM + 63) / 64;
-  for (p.chunk = 128;; p.chunk *= 2) {
-    const int c = p.chunk / 64;
-    p.parts = 0;
-    for (int t = 0; t < nt; ++t) p.parts += t / c + 1;
-    if (c >= nt || (p.parts <= max_parts && p.parts * (pad(p.tm) / p.tm) <= 64L * device_cus())) return p;
+PairPlan pair_plan(int W, int NM, int planes, int max_parts) {
+  const int nt = (NM + 63) / 64, cus = device_cus();
+  PairPlan best{};
+  double best_cost = 0.0;
+  for (int tm = 128, held = 2; tm >= 32; tm /= 2, ++held) {
+    const long rows = (W + tm - 1) / tm;
+    PairPlan p;
+    p.tm = tm;
+    for (p.chunk = 128;; p.chunk *= 2) {
+      const int c = p.chunk / 64;
+      p.parts = 0;
+      for (int t = 0; t < nt; ++t) p.parts += t / c + 1;
+      if (c >= nt || (p.parts <= max_parts / planes && p.parts * rows <= 64L * cus)) break;
+    }
+    const long n = (p.parts * rows * planes + cus - 1) / cus, r = n % held;
+    const double cost = (n - r + (r > 0 ? std::max((double)r, 1.6) : 0.0)) * tm * p.chunk / (tm == 32 ? 0.9 : 1.0);
+    if (tm == 128 || cost < 0.95 * best_cost) {
+      best = p;
+      best_cost = cost;
+    }
   }
+  return best;
 }
 
 // FP64: the tile and the split of k with the shortest estimated time: workgroups of the fullest CU times
@@ -379,14 +393,15 @@ void launch_pair_table(hipStream_t s, int M, int N, int K, const double* L, bool
 }
 
 int pair_parts(int W, int NM, bool real, int max_parts) {
-  return real ? pair_plan(W, NM, max_parts).parts : 2 * pair_plan(W, NM, max_parts / 2).parts;
+  const int planes = real ? 1 : 2;
+  return planes * pair_plan(W, NM, planes, max_parts).parts;
 }
 
 void launch_pair_exchange(hipStream_t s, int W, int NM, bool real, int max_parts, const double* G,
                           const double* B, double* part) {
   if (W <= 0) return;
   const int planes = real ? 1 : 2;
-  const PairPlan p = pair_plan(W, NM, max_parts / planes);
+  const PairPlan p = pair_plan(W, NM, planes, max_parts);
   auto go = [&](auto kern) {
     hipLaunchKernelGGL(kern, dim3(p.parts, (W + p.tm - 1) / p.tm, planes), dim3(256), 0, s, W, NM, NM, p.chunk,
                        1.0, G, (long)NM, B, (long)gemm_real_row(NM), part, (long)planes * p.parts, 0L, 1);
