@@ -40,10 +40,12 @@ if ROOT not in sys.path:
 METRIC = "walker-steps/s mixed vs FP64 at |ΔE_loc|<1e-5 Ha; % MFMA/HBM peak"
 # dense FP64 MFMA peak: the arithmetic of the exchange over the pair table
 PEAK_TFLOPS = {"fp64": 78.6}
+# arithmetic of vbias and vHS in each form
+VBIAS_VHS = {"fp64": "fp64", "fp32": "fp32", "bf16x3": "bf16x3", "int8": "fp32"}
 GATE_HA = 1e-5
 # HBM bytes per launch of the quadratic form's kernel (FETCH_SIZE and WRITE_SIZE counter runs scaled
 # by a copy kernel of known size); None for a workload without such a measurement
-TRAFFIC_BYTES = {}
+TRAFFIC_BYTES = {"c2": 33.37e6, "c3": 1062.14e6}
 TRAFFIC_SOURCE = {"c2": "profiles/walker_step_c2_hbm_traffic.md",
                   "c3": "profiles/walker_step_c3_hbm_traffic.md"}
 
@@ -575,11 +577,12 @@ def bench_single(args, A, torch, synth, workload, with_cpu, with_hybrid):
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": f"{mixed} contractions / fp64",
+        "dtype": "fp64" if mixed == "fp64" else f"{VBIAS_VHS[mixed]} vbias and vHS / fp64",
         "data": "synthetic",
         "config": {"workload": f"{s.name}: NMO={M}, {N}+{N} electrons, Nchol={K}, {W} walkers, "
                                f"dt={s.dt}, local-energy step, QR every {ortho}",
-                   "form": f"{mixed} Cholesky contractions, fp64 G/LU/QR/propagation/weights",
+                   "form": f"{mixed}: vbias and vHS in {VBIAS_VHS[mixed]}, exchange and Coulomb "
+                           "energy, G/LU/QR/propagation/weights in fp64",
                    "parallelism": "single GPU"},
         "roofline": {"bound": "mfma", "achieved": round(achieved, 3), "peak": peak,
                      "unit": "TFLOP/s", "frac": round(achieved / peak, 4),
