@@ -50,11 +50,10 @@ enum afq_walker_type { AFQ_CLOSED = 1, AFQ_COLLINEAR = 2 };
 enum afq_precision {
   AFQ_FP64 = 0,        /* plain form: everything FP64 (FP64 MFMA)                          */
   AFQ_FP32 = 1,        /* contractions in FP32 on MFMA with FP32 accumulation               */
-  AFQ_BF16X3 = 2,      /* mixed form: the exchange energy on BF16 MFMA with both operands
-                          split into three BF16 slices (hi/mid/lo, ~24 bits) and the six
-                          slice products of order <= 2 accumulated in FP32, per real/imag
-                          part; vbias and vHS as in AFQ_FP32. Needs N <= 16, M <= 96 and
-                          M % 8 == 0 (AFQ_EUNSUPPORTED otherwise)                           */
+  AFQ_BF16X3 = 2,      /* mixed form: vbias, vHS and the exchange energy on BF16 MFMA, each
+                          complex product as three real ones, both operands split into two
+                          BF16 parts (hi/lo, ~16 bits), FP32 accumulation. Needs N <= 32 and
+                          M <= 128 (AFQ_EUNSUPPORTED otherwise)                             */
   AFQ_INT8_SPLIT = 3   /* mixed form: the exchange energy on int8 MFMA with every row of G
                           and Lnak scaled by a power of two and split into 6 int8 slices
                           (x = u (q0 + q1/254 + ... + q5/254^5)); the slice products up to an

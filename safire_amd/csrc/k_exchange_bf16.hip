@@ -9,8 +9,8 @@
 // BF16 MFMAs per 16x16x32 complex tile, FP32 accumulation. The sums Re + Im are split on their
 // own (not summed from the parts), so every operand of an MFMA is a plain hi/lo pair.
 // Accuracy: each operand to ~2^-16 relative, each T entry to ~2^-15 of its terms, so this form
-// is ~100x less accurate than FP32 and far from a 1e-5 Ha energy gate on these Hamiltonians; it
-// is the fastest form and reports its error next to the others.
+// is ~100x less accurate than FP32 and far from a 1e-5 Ha energy gate on these Hamiltonians. It runs
+// where the pair table (k_gemm_real.hip) is not taken.
 //
 // Structure (as the int8 exchange for 17..32 electrons): a workgroup of 8 wavefronts holds 8/NT
 // walkers, NT = 1 or 2 wavefronts per walker (one per 16-row tile of T); each wavefront splits its
