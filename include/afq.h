@@ -57,9 +57,17 @@ enum afq_precision {
   AFQ_INT8_SPLIT = 3   /* mixed form: the exchange energy on int8 MFMA with every row of G
                           and Lnak scaled by a power of two and split into 6 int8 slices
                           (x = u (q0 + q1/254 + ... + q5/254^5)); the slice products up to an
-                          order of 2 to 5, by the vector's size, accumulate exactly in int32 and are combined in FP64
-                          (energy error ~1e-3 of AFQ_FP32's). vbias and vHS as in AFQ_FP32.
+                          order of 2 to 5, by the vector's size, accumulate exactly in int32 and
+                          are combined in FP64 (energy error ~1e-3 of AFQ_FP32's). vbias and vHS as in AFQ_FP32.
                           Needs N <= 32 and M <= 128 (AFQ_EUNSUPPORTED otherwise)           */
+};
+
+/* How the exchange and Coulomb energy is formed: per Cholesky vector in the handle's precision, or in
+ * FP64 over a table of orbital pairs (absent where it is too large or never the faster way). */
+enum afq_energy_route {
+  AFQ_ROUTE_AUTO = 0,     /* the faster one by estimated time, for each call's walker count */
+  AFQ_ROUTE_TABLE = 1,
+  AFQ_ROUTE_VECTORS = 2
 };
 
 /* Walker property slots (WalkerConfig.hpp:28-48, offsets WalkerSetBase.cpp:87-117). */
@@ -103,6 +111,10 @@ int afq_ham_destroy(afq_ham ham);
  * create). Re-reserving with a larger count reallocates. */
 int afq_ham_reserve(afq_ham ham, int max_walkers);
 int afq_ham_set_precision(afq_ham ham, int precision);
+/* The route of the energies of this handle (AFQ_ROUTE_AUTO after create; AFQ_EUNSUPPORTED for the table
+ * of a handle without one), and the route that the energy of W walkers takes (never AUTO). */
+int afq_ham_set_energy_route(afq_ham ham, int route);
+int afq_ham_energy_route(afq_ham ham, int W, int* route);
 int afq_ham_set_params(afq_ham ham, const afq_step_params* p);
 /* Autotuner (no counterpart in the reference, which leaves tile shapes to its libraries): times
  * every tiling of the vbias and vHS GEMMs this precision has for W walkers (afq_ham_reserve

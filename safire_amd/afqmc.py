@@ -18,6 +18,7 @@ LIB_PATH = os.path.join(HERE, "libsafire_afq.so")
 
 CLOSED, COLLINEAR = 1, 2
 FP64, FP32, BF16X3, INT8_SPLIT = 0, 1, 2, 3
+ROUTE_AUTO, ROUTE_TABLE, ROUTE_VECTORS = 0, 1, 2
 (P_WEIGHT, P_PHASE, P_PSEUDO_ELOC, P_E1, P_EXX, P_EJ, P_OVLP, P_LOGSCL_UP, P_LOGSCL_DN,
  P_IS_UNITARY, P_THETA, P_COUNT) = range(12)
 _ERRORS = {1: "AFQ_EBADSHAPE", 2: "AFQ_EHIP", 3: "AFQ_ENOMEM", 4: "AFQ_EINVAL",
@@ -49,6 +50,8 @@ SIGNATURES = {
     "afq_ham_destroy": (_i, [_vp]),
     "afq_ham_reserve": (_i, [_vp, _i]),
     "afq_ham_set_precision": (_i, [_vp, _i]),
+    "afq_ham_set_energy_route": (_i, [_vp, _i]),
+    "afq_ham_energy_route": (_i, [_vp, _i, _vp]),
     "afq_ham_set_params": (_i, [_vp, _vp]),
     "afq_ham_get_params": (_i, [_vp, _vp]),
     "afq_ham_tensors": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp]),
@@ -220,6 +223,17 @@ class HamiltonianOperations:
 
     def set_precision(self, precision):
         check(lib().afq_ham_set_precision(self.handle, precision))
+
+    def set_energy_route(self, route):
+        """ROUTE_AUTO (the faster one for each call), ROUTE_TABLE (FP64 over the table of orbital
+        pairs) or ROUTE_VECTORS (per Cholesky vector, in the handle's precision)."""
+        check(lib().afq_ham_set_energy_route(self.handle, route))
+
+    def energy_route(self, W):
+        """ROUTE_TABLE or ROUTE_VECTORS: how the energy of W walkers is formed."""
+        out = C.c_int()
+        check(lib().afq_ham_energy_route(self.handle, W, C.byref(out)))
+        return out.value
 
     def set_params(self, **kw):
         p = self.get_params()

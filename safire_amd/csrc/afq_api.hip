@@ -166,7 +166,10 @@ double pairs_us(afq_ham H, int W) {
   const double rows = (W + 31) / 32 * 32, NM = (double)H->N * H->M;
   return 15.0 + (H->real_trial ? 1.0 : 2.0) * rows * NM * (2.0 * NM + 4.0 * H->K) / 60e6;
 }
-bool use_pairs(afq_ham H, int W) { return H->pairs != nullptr && pairs_us(H, W) < exchange_us(H, W); }
+bool use_pairs(afq_ham H, int W) {
+  if (H->pairs == nullptr || H->energy_route == AFQ_ROUTE_VECTORS) return false;
+  return H->energy_route == AFQ_ROUTE_TABLE || pairs_us(H, W) < exchange_us(H, W);
+}
 
 // the exchange contraction in the handle's precision: Kl and per-chunk tr(T^2) partials
 void run_exchange(afq_ham H, hipStream_t s, int W, const double* G) {
@@ -438,6 +441,25 @@ int afq_ham_set_precision(afq_ham H, int precision) {
               "INT8_SPLIT exchange needs N <= 32 and M <= 128");
     H->precision = precision;
     H->cfg_vbias = H->cfg_vhs = 0;   // tilings are tuned per precision (afq_autotune)
+  });
+}
+
+int afq_ham_set_energy_route(afq_ham H, int route) {
+  return guard([&] {
+    check_ham(H);
+    AFQ_CHECK(route >= AFQ_ROUTE_AUTO && route <= AFQ_ROUTE_VECTORS, AFQ_EINVAL, "unknown energy route");
+    AFQ_CHECK(route != AFQ_ROUTE_TABLE || H->pairs != nullptr, AFQ_EUNSUPPORTED,
+              "this handle has no pair table");
+    H->energy_route = route;
+  });
+}
+
+int afq_ham_energy_route(afq_ham H, int W, int* route) {
+  return guard([&] {
+    check_ham(H);
+    AFQ_CHECK(W >= 0, AFQ_EBADSHAPE, "negative walker count");
+    AFQ_CHECK(route != nullptr, AFQ_EINVAL, "null route");
+    *route = use_pairs(H, W) ? AFQ_ROUTE_TABLE : AFQ_ROUTE_VECTORS;
   });
 }
 

@@ -175,6 +175,7 @@ struct afq_ham_s {
   double dt = 0.005, E0 = 0.0;
   double ci0_re = 1.0, ci0_im = 0.0;
   int precision = AFQ_FP64;
+  int energy_route = AFQ_ROUTE_AUTO;
   int cfg_vbias = 0, cfg_vhs = 0;   // GEMM tilings (afq_autotune)
   afq_step_params params;
   int device = 0;
