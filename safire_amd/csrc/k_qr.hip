@@ -11,7 +11,8 @@
 // a column's dot product takes three DPP additions over its 8 lanes. So the 2 N serial steps cost
 // an LDS read of M / 8 entries, M / 4 complex multiply-adds and a short reduction each. M 128, N 32,
 // 1024 walkers: 928 us with A and Q in LDS and a wavefront-wide shuffle reduction per column
-// (k_qr, which stays for M > 128), 252 us here; M 48, N 12, 256 walkers: 46 -> 22 us.
+// (k_qr, which stays for M > 128 and for few columns of more than 64 rows), 252 us here; M 48, N 12, 256
+// walkers: 46 -> 22 us.
 //
 // k_qr: one workgroup per walker; A (the reflectors) and Q live in LDS with rows padded to N + 1
 // complex numbers, so that the lanes of a column access (consecutive rows) fall into different
@@ -251,7 +252,14 @@ void launch_orthogonalize(hipStream_t s, int nb, int M, int N, double* Phi, long
   AFQ_CHECK(N <= 64, AFQ_EUNSUPPORTED, "orthogonalize: N > 64");
   const size_t lds = 2 * sizeof(cd) * (size_t)M * (N + 1);
   AFQ_CHECK(lds <= 160 * 1024 - 2048, AFQ_EUNSUPPORTED, "orthogonalize: walker too large");
-  if (M <= 128 && N <= M) {
+  // Up to four columns leave the 8 threads of each with all of its rows, one after the other: k_qr is
+  // faster (us, k_qr and k_qr_regs at 256 walkers: M 128, N 2 8.7 and 11.4, N 3 13.1 and 14.6, N 4 14.9
+  // and 18.1, N 5 20.1 and 20.4; M 65, N 2 8.2 and 9.1, N 4 13.4 and 14.5; M 96, N 3 12.6 and 12.0; M 64,
+  // N 2 both 8) until more walkers share a CU (M 128, N 2: 1024 10.1 and 13.1, 2048 18.5 and 16.0; N 4:
+  // 512 17.0 and 19.3, 1024 20.8 and 19.6)
+  const int cus = device_cus();
+  const bool few = M > 64 && (N <= 2 ? nb <= 4 * cus : N <= 4 && (M > 96 ? nb <= 2 * cus : N == 4 && nb <= cus));
+  if (M <= 128 && N <= M && !few) {
     auto go = [&](auto kern) {
       hipLaunchKernelGGL(kern, dim3(nb), dim3((8 * N + 63) / 64 * 64), 0, s, M, N,
                          reinterpret_cast<cd*>(Phi), ldw, reinterpret_cast<cd*>(logdetR));
