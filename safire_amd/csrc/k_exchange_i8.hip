@@ -6,8 +6,9 @@
 // A slice product accumulates in int32 without rounding, so the error left is the truncation
 // of the slice series, relative to the row maximum.
 //
-// Slices: 6 of G and 6 of each Lnak row, and per Cholesky vector a slice-product order o_n in 2..5
-// (all products s + t <= o_n kept; 21, 15, 10 or 6 products) fixed at set-up from the vector's size
+// Slices: 6 of G and 6 of each Lnak row, and per Cholesky vector a slice-product order o_n in 2..5 (4 or
+// 5 for up to 16 electrons: every T then to 254^-5 of its own vector's size, whatever the sizes of the
+// others) with all products s + t <= o_n kept (21, 15, 10 or 6), fixed at set-up from the vector's size
 // r_n = max|L_n| / max_m |L_m|: o_n = ceil(5 + 2 log_254 r_n). The error a vector adds to EXX
 // scales as r_n^2 254^-(o_n + 1) (both its T block and the truncation of its product series are
 // proportional to r_n), so every vector then contributes at most 254^-6 of the largest one's
@@ -530,7 +531,7 @@ void exchange_i8_orders(hipStream_t s, int M, int N, int K, const double* Lnak, 
     if (!(top > 0.0) || !(h[n] <= top)) continue;   // zero or non-finite: keep every product
     const double r = h[n] / top;
     int on = r > 0.0 ? (int)std::ceil(5.0 + 2.0 * std::log(r) / std::log(kBase)) : 2;
-    o[n] = std::min(kS - 1, std::max(2, on));
+    o[n] = std::min(kS - 1, std::max(N <= 16 ? 4 : 2, on));
   }
   AFQ_HIP(hipMemcpyAsync(ord, o.data(), sizeof(int) * K, hipMemcpyHostToDevice, s));
   AFQ_HIP(hipStreamSynchronize(s));
