@@ -24,9 +24,8 @@
 // the previous pass is multiplied, and stored to LDS between two barriers; only the slices that
 // the pass's order needs are loaded. Real trial orbitals give Im Lnak = 0: only real slices are
 // kept then (LC = false), with 2 MFMAs per slice product instead of 4.
-// T = uG_a uL_b sum_o 254^-o acc_o is assembled in FP64 (orders 0, 1 and 2, 3 are joined exactly in
-// int32 first; orders 4 and 5, at most 254^-4 of the sum, in FP32, whose rounding there is 2^-56 of
-// it) and goes to LDS, where the next pass forms tr(T^2) and tr(T): two T buffers when they fit,
+// T = uG_a uL_b sum_o 254^-o acc_o is assembled in FP64 (orders that fit are joined exactly in int32
+// first) and goes to LDS, where the next pass forms tr(T^2) and tr(T): two T buffers when they fit,
 // and then half of the wavefronts do that before their MFMAs and half after, so that the VALU work
 // of one wavefront of a SIMD runs under the MFMAs of the other.
 //
@@ -321,7 +320,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void k_exchange_i8(
       if (ON >= 5 && KC == 1 && !LC)   // 254 c4 + c5 < 2^31 for M <= 104
         lo = (double)(__mul24(254, c[ON >= 4 ? 4 : 0][r]) + c[ON >= 5 ? 5 : 0][r]) * (1.0 / kBase);
       else if (ON >= 5)
-        lo = (double)fmaf((float)c[ON >= 5 ? 5 : 0][r], (float)(1.0 / kBase), (float)c[ON >= 4 ? 4 : 0][r]);
+        lo = fma((double)c[ON >= 5 ? 5 : 0][r], 1.0 / kBase, (double)c[ON >= 4 ? 4 : 0][r]);
       else if (ON == 4)
         lo = (double)c[ON >= 4 ? 4 : 0][r];
       double mid;
