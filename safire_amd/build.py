@@ -10,7 +10,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libsafire_afq.so")
 SOURCES = ["afq_api.hip", "afq_phmsd.hip", "afq_rng.hip", "k_green.hip", "k_gemm.hip", "k_gemm_bf16.hip", "k_gemm_real.hip", "k_energy.hip", "k_exchange_bf16.hip",
            "k_exchange_f64.hip",
-           "k_exchange_i8.hip", "k_phmsd.hip", "k_phmsd_exc.hip", "k_propagate.hip", "k_qr.hip", "k_walker.hip",
+           "k_exchange_i8.hip", "k_exchange_i8w.hip", "k_phmsd.hip", "k_phmsd_exc.hip", "k_propagate.hip", "k_qr.hip", "k_walker.hip",
            "k_setup.hip"]
 # k_green.hip unrolls the 16 Gauss-Jordan steps of its N <= 16 kernels in full (each step indexes
 # the register-resident rows with the step number); the default budget of a pragma-driven unroll

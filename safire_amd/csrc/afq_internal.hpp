@@ -310,6 +310,10 @@ void exchange_i8_orders(hipStream_t s, int M, int N, int K, const double* Lnak, 
 void launch_exchange_i8(hipStream_t s, int W, int M, int N, int K, const double* G, bool real,
                         const int8_t* Lq, const double* Lu, const int* ord, double* Kl,
                         double* exx_part);
+// k_exchange_i8w.hip: the same per walker (17 to 32 electrons: complex trials on more than 64 orbitals)
+int exchange_i8w_chunks(int W, int N, int K);
+void launch_exchange_i8w(hipStream_t s, int W, int M, int N, int K, const double* G, bool real,
+                         const int8_t* Lq, const double* Lu, const int* ord, double* Kl, double* exx_part);
 void launch_exchange(hipStream_t s, int precision, int W, int M, int N, int K, const double* G,
                      const void* Lnak, double* Kl, double* exx_part);
 void launch_energy_finalize(hipStream_t s, int W, int K, int nchunk, int walker_type,

@@ -31,14 +31,14 @@
 //
 // What bounds it: neither unit alone. A pass is MFMAs (8 K of 12 K cycles at M = 128), pair sums and
 // the two barriers around the LDS store, and the two wavefronts of a SIMD go through them nearly
-// together. One walker's 32 x 32 blocks with complex slices, the form before, against this one:
-// M 64, N 16, K 320, W 512 real trial: 188 -> 166 us; M 128, N 32, K 640, W 1024: 4040 -> 2560 us;
-// M 88, N 22, K 440, W 137: 1055 -> 240 us.
-// With K of about 1.5 M and more and enough walkers the quadratic form over the pair table in FP64 is
-// still faster (k_gemm_real.hip: 61, 1020 and 69 us for these, traces included) and is taken instead.
+// together. One walker's 32 x 32 blocks with complex slices against this for real trials: M 128, N 32,
+// K 640, W 1024: 4040 -> 2560 us; M 88, N 22, K 440, W 137: 1055 -> 240 us. Where padding costs less than
+// that, and in small calls, k_exchange_i8w.hip is taken (per_walker below), and with enough vectors and
+// walkers the quadratic form over the pair table in FP64 (k_gemm_real.hip: 1020 and 69 us for these,
+// traces included).
 //
 // M <= 128, N <= 32.
-#include "afq_internal.hpp"
+#include "i8_split.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -48,51 +48,10 @@ namespace afq {
 
 namespace {
 
-typedef int i4 __attribute__((ext_vector_type(4)));
+using namespace i8;
 
-constexpr int kS = 6;             // slices of G and of Lnak
 constexpr int kMaxKC = 2;         // 64-wide k chunks: M <= 128
-constexpr double kBase = 254.0;   // ratio of consecutive slice units
 constexpr int kItems = 8;         // pairs of a pass per thread, at most
-
-// power-of-two unit of a row whose largest |component| is mx: |x / u| < 127 for every x of the
-// row. Rows below 2^-960 count as zero (their products are far below any energy resolution);
-// a non-finite row gets NaN so that its energies come out NaN as in FP64.
-__device__ inline double row_unit(double mx, bool& zero) {
-  zero = false;
-  if (!(mx <= 1.0e300)) return __builtin_nan("");
-  if (mx < 0x1p-960) {
-    zero = true;
-    return 1.0;
-  }
-  int e;
-  frexp(mx * (128.0 / 127.0), &e);
-  return ldexp(1.0, e - 7);
-}
-
-// the first S slices of r = x / u (|r| < 127; x * inv_u is exact, inv_u being a power of two)
-template <int S>
-__device__ inline void slice(double r, int (&q)[S]) {
-#pragma unroll
-  for (int s = 0; s < S; ++s) {
-    const double qs = rint(r);
-    q[s] = (int)qs;
-    r = (r - qs) * kBase;
-  }
-}
-
-__device__ inline unsigned pack4(int a, int b, int c, int d) {
-  return (unsigned)(a & 0xff) | ((unsigned)(b & 0xff) << 8) | ((unsigned)(c & 0xff) << 16) |
-         ((unsigned)(d & 0xff) << 24);
-}
-
-__device__ inline i4 mfma_i8(i4 a, i4 b, i4 c) {
-  return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0);
-}
-
-// workgroup barrier after this wavefront's LDS reads and writes; its global loads and stores in flight
-// are not waited for. The memory clobber keeps the compiler from moving memory accesses across.
-__device__ inline void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 template <int KC, int CT, bool LC, int NW>
 __global__ __launch_bounds__(64 * NW, NW / 4) void k_exchange_i8(
@@ -123,52 +82,10 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void k_exchange_i8(
 
   // ---- slices of the wavefront's rows of G: row 16 wave + r16, k = 64 kc + 16 g + j (j < 16)
   i4 ar[KC][kS], ai[KC][kS];
-  double uG;
-  {
-    const int row = 16 * wave + r16;
-    const bool ok = row < nw * N;
-    const double2* Gr = reinterpret_cast<const double2*>(G) + ((long)w0 * N + (ok ? row : 0)) * M;
-    double mx = 0.0;
-    if (ok) {
-      for (int kc = 0; kc < KC; ++kc)
-        for (int j = 0; j < 16; ++j) {
-          const int k = 64 * kc + 16 * g + j;
-          if (k < M) {
-            const double2 x = Gr[k];
-            const double xr = fabs(x.x), xi = fabs(x.y);
-            // a NaN or Inf anywhere in the row must survive the max (fmax drops NaN)
-            mx = (xr <= 1.0e300 && xi <= 1.0e300) ? fmax(mx, fmax(xr, xi)) : INFINITY;
-          }
-        }
-    }
-    mx = fmax(mx, __shfl_xor(mx, 16, 64));
-    mx = fmax(mx, __shfl_xor(mx, 32, 64));
-    bool zero;
-    uG = row_unit(mx, zero);
-    const bool finite = uG == uG;
-    const double inv = (finite && !zero) ? 1.0 / uG : 0.0;
-#pragma unroll
-    for (int kc = 0; kc < KC; ++kc) {
-#pragma unroll
-      for (int d = 0; d < 4; ++d) {   // bytes 4d..4d+3 of each fragment
-        int qr[4][kS], qi[4][kS];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int k = 64 * kc + 16 * g + 4 * d + j;
-          double2 x = double2{0.0, 0.0};
-          if (ok && k < M && inv != 0.0) x = Gr[k];
-          slice<kS>(x.x * inv, qr[j]);
-          slice<kS>(x.y * inv, qi[j]);
-        }
-#pragma unroll
-        for (int s = 0; s < kS; ++s) {
-          ar[kc][s][d] = (int)pack4(qr[0][s], qr[1][s], qr[2][s], qr[3][s]);
-          ai[kc][s][d] = (int)pack4(qi[0][s], qi[1][s], qi[2][s], qi[3][s]);
-        }
-        __builtin_amdgcn_sched_barrier(0);   // four elements at a time (registers)
-      }
-    }
-  }
+  const int grow = 16 * wave + r16;
+  const bool gok = grow < nw * N;
+  const double uG = slice_row<KC>(reinterpret_cast<const double2*>(G) + ((long)w0 * N + (gok ? grow : 0)) * M, gok,
+                                  M, g, ar, ai);
   // units of the rows, over 254: the joined orders 0 and 1 carry one factor 254
   if (lane < 16) sR[16 * wave + lane] = uG * (1.0 / kBase);
 
@@ -313,34 +230,12 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void k_exchange_i8(
     if (LC)
 #pragma unroll
       for (int o = 0; o <= ON; ++o) cR[o] -= cQ[LC ? o : 0];
-    // 254 sum_o 254^-o c_o. |c_o| <= (o + 1) 128 127^2 NP: 254 c0 + c1 fits int32 always and
-    // 254 c2 + c3 with real Lnak (24-bit factors: |c0|, |c2| < 2^23)
-    auto join = [&](const i4* c, int r) {
-      double lo = 0.0;
-      if (ON >= 5 && KC == 1 && !LC)   // 254 c4 + c5 < 2^31 for M <= 104
-        lo = (double)(__mul24(254, c[ON >= 4 ? 4 : 0][r]) + c[ON >= 5 ? 5 : 0][r]) * (1.0 / kBase);
-      else if (ON >= 5)
-        lo = fma((double)c[ON >= 5 ? 5 : 0][r], 1.0 / kBase, (double)c[ON >= 4 ? 4 : 0][r]);
-      else if (ON == 4)
-        lo = (double)c[ON >= 4 ? 4 : 0][r];
-      double mid;
-      if (LC || ON < 3) {
-        // c2 + c3 / 254, times 254
-        mid = (double)c[2][r];
-        if (ON >= 3) mid = fma((double)c[ON >= 3 ? 3 : 0][r], 1.0 / kBase, mid);
-        mid *= kBase;
-      } else {
-        mid = (double)(__mul24(254, c[2][r]) + c[ON >= 3 ? 3 : 0][r]);
-      }
-      if (ON >= 4) mid = fma(lo, 1.0 / kBase, mid);
-      return fma(mid, 1.0 / (kBase * kBase), (double)(__mul24(254, c[0][r]) + c[1][r]));
-    };
     const double uL = sU[min(col, crows - 1)];
     if (col < crows) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const double u = sR[16 * wave + 4 * g + r] * uL;
-        T[(16 * wave + 4 * g + r) * ldt + col] = double2{join(cR, r) * u, join(cI, r) * u};
+        T[(16 * wave + 4 * g + r) * ldt + col] = double2{join_orders<ON, KC, LC>(cR, r) * u, join_orders<ON, KC, LC>(cI, r) * u};
       }
     }
   };
@@ -431,7 +326,7 @@ __global__ __launch_bounds__(256) void k_split_lnak_i8(int rows, int M, int Mp, 
   for (int k = lane; k < Mp; k += 64)
     for (int p = 0; p < np; ++p) {
       int q[kS];
-      slice<kS>(k < M && inv != 0.0 ? x[2 * k + p] * inv : 0.0, q);
+      slice(k < M && inv != 0.0 ? x[2 * k + p] * inv : 0.0, q);
 #pragma unroll
       for (int t = 0; t < kS; ++t) Lq[(t * np + p) * plane + (size_t)row * Mp + k] = (int8_t)q[t];
     }
@@ -456,12 +351,13 @@ size_t lds_of(int nw, int ct, int cv, int N, int Mp, int np, int tdbl) {
 // SIMD), or 4 where workgroups of 8 would leave CUs without work. The vectors are split into
 // chunks that minimise the rounds of workgroups times (passes + 2), the 2 standing for reading and
 // slicing the workgroup's G.
-Plan plan_of(int W, int M, int N, int K, int np) {
+Plan tiles_of(int W, int M, int N, int K, int np, double* eff) {
   const int Mp = exchange_i8_row(M);
   const long cus = device_cus();
   Plan p{};
+  double best = -1.0;
   auto shape = [&](int nw) {
-    double best = -1.0;
+    best = -1.0;
     for (int ct = 2; ct <= 3; ++ct) {
       const int cv = std::min(16 * ct / N, K);
       if (cv < 1) continue;
@@ -485,6 +381,14 @@ Plan plan_of(int W, int M, int N, int K, int np) {
   if (np == 2 && Mp > 64) shape(4);
   else shape(8);
   if (((long)(W + p.rw - 1) / p.rw) * ((K + p.cv - 1) / p.cv) < cus) shape(4);
+  *eff = best * p.rw * N / (16 * p.nw);
+  return p;
+}
+
+Plan plan_of(int W, int M, int N, int K, int np) {
+  const long cus = device_cus();
+  double eff;
+  Plan p = tiles_of(W, M, N, K, np, &eff);
   const long passes = (K + p.cv - 1) / p.cv, groups = (W + p.rw - 1) / p.rw;
   long best = -1;
   for (long nch = 1; nch <= passes; ++nch) {
@@ -497,6 +401,28 @@ Plan plan_of(int W, int M, int N, int K, int np) {
   }
   p.nchunk = (K + p.chunk - 1) / p.chunk;
   return p;
+}
+
+// Whether the kernels of k_exchange_i8w.hip take the call. Up to 16 electrons: estimated times, a constant
+// and a term per walker and vector (ns, times the share of tiles that holds data for the packed product);
+// more than 64 orbitals besides: not for many real products (M 128, N 16, K 640, W 1024: 734 us packed and
+// 847) nor for middling numbers of complex ones (K 64, W 64: 36 and 42 us; K 384, W 64: 97 and 86). Fitted to
+// 670 calls of M 16 to 128, N 3 to 16, K 8 to 640, W 1 to 1024: the choice is 0.8 % slower than the faster
+// kernel in the mean, over 6 % in 1 of 20. 17 to 32 electrons: 2 x 2 tiles of complex products on more
+// than 64 orbitals, unless packing saves a third of the tiles (N 28: both 23 % padding, 1570 -> 1160 us at
+// M 110, K 330, W 512; N 19: 70 % of the tiles, 1010 and 1340 us at M 77, K 385) or the call is small
+// (M 128, N 32, K 192, W 16: 64 and 68 us). Real trials gain little from those (mean 1 %).
+bool per_walker(int W, int M, int N, int K, bool real) {
+  double eff;
+  tiles_of(W, M, N, K, real ? 1 : 2, &eff);
+  const double pairs = (double)W * K, share = (N > 16 ? N / 32.0 : N / 16.0) * (N > 16 ? N / 32.0 : N / 16.0);
+  if (N > 16) return !real && M > 64 && pairs >= 4096 && 1.5 * share > eff;
+  if (M > 64 && (real ? pairs > 1e5 : pairs > 2000 && pairs < 12000)) return false;
+  if (M > 64 && W < 8 && K > 500) return false;   // M 128, N 16, K 640, one walker: 34 and 41 us
+  const double packed[2][2] = {{1.6, 2.8}, {1.3, 2.0}}, alone[2][2] = {{1.0, 2.0}, {1.0, 2.0}};   // ns
+  const int lc = real ? 0 : 1, kc = M > 64 ? 1 : 0;
+  const double base = kc ? 16.0 : (lc ? 14.0 : 12.0);
+  return base + 1e-3 * alone[lc][kc] * pairs < 18.0 + 1e-3 * packed[lc][kc] * pairs * share / eff;
 }
 
 }  // namespace
@@ -537,6 +463,7 @@ void exchange_i8_orders(hipStream_t s, int M, int N, int K, const double* Lnak, 
 }
 
 int exchange_i8_chunks(int W, int M, int N, int K, bool real) {
+  if (per_walker(W, M, N, K, real)) return exchange_i8w_chunks(W, N, K);
   return plan_of(W, M, N, K, real ? 1 : 2).nchunk;
 }
 
@@ -558,6 +485,10 @@ void launch_exchange_i8(hipStream_t s, int W, int M, int N, int K, const double*
   AFQ_CHECK((size_t)(N > 16 ? 12 : 10) * K * N * Mp < (1UL << 31), AFQ_EUNSUPPORTED,
             "int8 exchange: the Cholesky slices exceed 2 GiB");
   AFQ_CHECK(ord != nullptr, AFQ_EINVAL, "int8 exchange: no slice orders");
+  if (per_walker(W, M, N, K, real)) {
+    launch_exchange_i8w(s, W, M, N, K, G, real, Lq, Lu, ord, Kl, exx_part);
+    return;
+  }
   const Plan p = plan_of(W, M, N, K, real ? 1 : 2);
   const dim3 grid((W + p.rw - 1) / p.rw, p.nchunk);
   auto go = [&](auto kern) {
