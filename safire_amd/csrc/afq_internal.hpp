@@ -239,6 +239,9 @@ void launch_green(hipStream_t s, int nb, int M, int N, const double* PsiT, const
 // split_ws (c128, split_ws_elems complex numbers) enables a deterministic split of k; NULL = none.
 constexpr int kMaxSplits = 8;
 int gemm_splits(int m, int n, int k);
+// estimated us of launch_gemm_nt_z in FP64 with a complex B (two workgroups share a CU's rate, one alone
+// reaches 0.6 of it, and the pass over the splits)
+double gemm_nt_z_f64_us(int m, int n, int k, long split_elems);
 // tilings launch_gemm_nt_z can run for a precision and kind of B (the cfg argument: 0 .. n-1)
 int gemm_tile_configs(int precision, bool b_complex);
 void launch_gemm_nt_z(hipStream_t s, int precision, int m, int n, int k, double alpha,
@@ -268,6 +271,10 @@ void launch_pair_table(hipStream_t s, int M, int N, int K, const double* L, bool
 int pair_parts(int W, int NM, bool real, int max_parts);
 void launch_pair_exchange(hipStream_t s, int W, int NM, bool real, int max_parts, const double* G,
                           const double* B, double* part);
+// the work of launch_pair_exchange's fullest CU (rows times columns of its tiles), and estimated us of
+// launch_gemm_real in FP64
+double pair_exchange_cost(int W, int NM, bool real, int max_parts);
+double gemm_f64_us(int m, int n, int k, long split_elems);
 // k_energy.hip
 int device_cus();                        // compute units of the current device (cached)
 int exx_nchunks(int W, int N, int K);   // chunks of Cholesky vectors the exchange kernel uses

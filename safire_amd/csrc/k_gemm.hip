@@ -18,6 +18,8 @@
 // vbias has few output tiles (W x K = 512 x 320 is 40 tiles) and a long k (N*M), so k is split
 // over grid.z: each split writes its partial tile to a workspace and a second kernel sums the
 // splits in a fixed order (deterministic, no atomics) and applies alpha.
+#include <cmath>
+
 #include "afq_internal.hpp"
 
 namespace afq {
@@ -203,6 +205,18 @@ int gemm_splits(int m, int n, int k) {
   int s = (512 + tiles - 1) / tiles;
   s = std::min(s, std::max(1, k / 128));
   return std::max(1, std::min(s, kMaxSplits));
+}
+
+double gemm_nt_z_f64_us(int m, int n, int k, long split_elems) {
+  const double tiles = std::ceil((double)m / kTile) * std::ceil((double)n / kTile);
+  int splits = gemm_splits(m, n, k);
+  if ((long)splits * m * n > split_elems) splits = 1;
+  const int kchunk = ((k + splits - 1) / splits + 31) & ~31;
+  splits = (k + kchunk - 1) / kchunk;
+  const double share = std::ceil(tiles * splits / device_cus());
+  double us = share * 8.0 * kTile * kTile * kchunk / 0.234e6;   // FLOP per us and CU
+  if (share < 2) us /= 0.6;
+  return splits > 1 ? us + 4.0 + 16e-6 * m * (double)n * (splits + 1) / 4.0 : us;
 }
 
 int gemm_tile_configs(int precision, bool b_complex) {

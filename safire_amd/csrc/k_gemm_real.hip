@@ -327,6 +327,7 @@ __global__ __launch_bounds__(256, 2) void k_pair_table(int M, int NM, int K, con
 // at M 88, N 22 with 137, and 70 and 59 at M 77, N 19 with 201 and two tables.
 struct PairPlan {
   int tm, chunk, parts;
+  double cost;   // rounds times rows times columns of a chunk
 };
 PairPlan pair_plan(int W, int NM, int planes, int max_parts) {
   const int nt = (NM + 63) / 64, cus = device_cus();
@@ -343,8 +344,10 @@ PairPlan pair_plan(int W, int NM, int planes, int max_parts) {
       if (c >= nt || (p.parts <= max_parts / planes && p.parts * rows <= 64L * cus)) break;
     }
     const long n = (p.parts * rows * planes + cus - 1) / cus, r = n % held;
-    const double cost = (n - r + (r > 0 ? std::max((double)r, 1.6) : 0.0)) * tm * p.chunk / (tm == 32 ? 0.9 : 1.0);
+    const double rounds = (n - r + (r > 0 ? std::max((double)r, 1.6) : 0.0)) / (tm == 32 ? 0.9 : 1.0);
+    const double cost = rounds * tm * p.chunk;
     if (tm == 128 || cost < 0.95 * best_cost) {
+      p.cost = rounds * tm * std::min(p.chunk, NM);
       best = p;
       best_cost = cost;
     }
@@ -354,8 +357,8 @@ PairPlan pair_plan(int W, int NM, int planes, int max_parts) {
 
 // FP64: the tile and the split of k with the shortest estimated time: workgroups of the fullest CU times
 // the work of one (234 MFLOP/s per us and CU where workgroups share it, 0.6 of it for one alone; the
-// smaller tiles at 0.95 and 0.8 of that), and the pass that adds the splits.
-void gemm_f64_plan(int m, int n, int k, long split_elems, int& tm, int& tn, int& splits) {
+// smaller tiles at 0.95 and 0.8 of that), and the pass that adds the splits. Returns that time in us.
+double gemm_f64_plan(int m, int n, int k, long split_elems, int& tm, int& tn, int& splits) {
   const double cus = device_cus();
   double best = 1e300;
   const int tiles[3][2] = {{128, 64}, {64, 64}, {64, 32}};
@@ -375,6 +378,7 @@ void gemm_f64_plan(int m, int n, int k, long split_elems, int& tm, int& tn, int&
         splits = s;
       }
     }
+  return best;
 }
 
 }  // namespace
@@ -395,6 +399,15 @@ void launch_pair_table(hipStream_t s, int M, int N, int K, const double* L, bool
 int pair_parts(int W, int NM, bool real, int max_parts) {
   const int planes = real ? 1 : 2;
   return planes * pair_plan(W, NM, planes, max_parts).parts;
+}
+
+double pair_exchange_cost(int W, int NM, bool real, int max_parts) {
+  return pair_plan(W, NM, real ? 1 : 2, max_parts).cost;
+}
+
+double gemm_f64_us(int m, int n, int k, long split_elems) {
+  int tm, tn, splits;
+  return gemm_f64_plan(m, n, k, split_elems, tm, tn, splits);
 }
 
 void launch_pair_exchange(hipStream_t s, int W, int NM, bool real, int max_parts, const double* G,

@@ -110,3 +110,21 @@ def test_route_without_a_table():
     assert e.value.code == 4
     assert ham.energy_route(100000) == A.ROUTE_VECTORS
     ham.close()
+
+
+# us measured per vector and over the table; sizes at which one is at least 1.2 times the other
+@pytest.mark.parametrize("M,N,K,complex_trial,W,form,vectors,table", [
+    (128, 32, 192, True, 64, A.FP32, 235, 297), (128, 32, 192, True, 64, A.BF16X3, 61, 297),
+    (128, 32, 192, True, 64, A.INT8_SPLIT, 129, 297), (128, 32, 640, True, 1024, A.FP32, 12478, 1857),
+    (128, 32, 640, True, 1024, A.INT8_SPLIT, 3803, 1857), (128, 32, 640, False, 1024, A.BF16X3, 2056, 949),
+    (128, 16, 640, True, 64, A.BF16X3, 63, 99), (64, 16, 96, True, 128, A.INT8_SPLIT, 32, 63),
+    (64, 16, 320, False, 512, A.FP32, 316, 69), (64, 16, 320, False, 512, A.INT8_SPLIT, 139, 69),
+    (64, 16, 320, False, 512, A.FP64, 250, 69), (24, 6, 120, False, 64, A.FP64, 14, 25),
+])
+def test_route_is_the_faster_one(M, N, K, complex_trial, W, form, vectors, table):
+    h, L, PsiT, _ = make(M, N, K, 1, complex_trial)
+    ham = A.HamiltonianOperations(h, L, PsiT, 0.0, 0.01)
+    ham.reserve(W)
+    ham.set_precision(form)
+    assert ham.energy_route(W) == (A.ROUTE_TABLE if table < vectors else A.ROUTE_VECTORS)
+    ham.close()
