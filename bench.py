@@ -19,9 +19,9 @@ graph's final walker buffer must equal the eager run's bit for bit (graph_matche
 |E_loc(form) - E_loc(FP64)| on identical walker states is below 1e-5 Ha; the line carries every
 form's throughput and gate error. A step = one pass over all walkers.
 
-roofline: the exchange and Coulomb energy kernels (the dominant region), executed FP64 matrix FLOP
-per call W*(2 (N M)^2 + 4 N M K) divided by the region's mean duration measured with HIP events on
-the launch stream over the eager timed run. cpu_baseline: the C++ FP64 oracle (OpenMP over walkers) timed
+roofline: the exchange and Coulomb energy kernels (the dominant region), executed matrix FLOP per
+call of the route they took (over the pair table W*(2 (N M)^2 + 4 N M K), FP64) divided by the region's
+mean duration measured with HIP events on the launch stream over the eager timed run. cpu_baseline: the C++ FP64 oracle (OpenMP over walkers) timed
 on this host on a bounded sample of the same workload.
 """
 from __future__ import annotations
@@ -38,8 +38,8 @@ if ROOT not in sys.path:
     sys.path.insert(0, ROOT)
 
 METRIC = "walker-steps/s mixed vs FP64 at |ΔE_loc|<1e-5 Ha; % MFMA/HBM peak"
-# dense FP64 MFMA peak: the arithmetic of the exchange over the pair table
-PEAK_TFLOPS = {"fp64": 78.6}
+# dense MFMA peaks
+PEAK_TFLOPS = {"fp64": 78.6, "fp32": 157.3, "bf16x3": 2500.0}
 # arithmetic of vbias and vHS in each form
 VBIAS_VHS = {"fp64": "fp64", "fp32": "fp32", "bf16x3": "bf16x3", "int8": "fp32"}
 GATE_HA = 1e-5
@@ -50,21 +50,38 @@ TRAFFIC_SOURCE = {"c2": "profiles/walker_step_c2_hbm_traffic.md",
                   "c3": "profiles/walker_step_c3_hbm_traffic.md"}
 
 
-def exchange_flops(W, M, N, K):
-    """Executed FLOP of the energy contractions of a real trial: half of the (N M)^2 pair table and the
-    Coulomb traces, or, where those are fewer, the contractions per Cholesky vector."""
+def energy_work(form, table, W, M, N, K):
+    """(executed matrix FLOP of one call's exchange and Coulomb contractions for a real trial, the dense
+    peak in TFLOP/s of the arithmetic they run on). Over the pair table: half of its (N M)^2 entries and
+    the traces, FP64 in every form. Per Cholesky vector: real FP64 vectors, complex FP32 ones, three
+    real products of three hi/lo terms in BF16X3; the int8 form's slice products differ per vector, so
+    it counts the FP64 contractions and has no peak (None)."""
     NM = N * M
-    return W * min(2.0 * NM * NM + 4.0 * NM * K, 4.0 * N * N * M * K)
+    if table:
+        return W * (2.0 * NM * NM + 4.0 * NM * K), PEAK_TFLOPS["fp64"]
+    per = {"fp64": 4.0, "fp32": 8.0, "bf16x3": 18.0, "int8": 4.0}[form]
+    return W * per * N * N * M * K, PEAK_TFLOPS.get(form)
 
 
-def step_flops(M, N, K):
-    """FLOP of one local-energy walker-step (complex MAC = 8, real x complex = 4)."""
+def energy_roofline(calls):
+    """TFLOP/s of (flop, peak, ms) calls and the fraction of the time that they take at their peaks
+    (None where one has no peak)."""
+    ms = sum(c[2] for c in calls)
+    if ms <= 0:
+        return 0.0, None
+    frac = None if any(c[1] is None for c in calls) else sum(c[0] / c[1] for c in calls) / (ms * 1e9)
+    return sum(c[0] for c in calls) / (ms * 1e9), frac
+
+
+def step_flops(M, N, K, energy):
+    """FLOP of one local-energy walker-step (complex MAC = 8, real x complex = 4) whose exchange and
+    Coulomb contractions are `energy`."""
     return (8 * M * N * N + 8 * N ** 3 + 8 * M * N * N      # T, LU + inverse, G
             + 8 * N * M * K                                  # vbias
             + 4 * M * M * K                                  # vHS
             + 16 * M * M * N + 48 * M * M * N                # 2 P1 products, Taylor-6
             + 16 * M * N * N + 8 * N ** 3 + 8 * N * M        # new G, LU/inverse, E1
-            + exchange_flops(1, M, N, K)                     # exchange and Coulomb energy
+            + energy                                         # exchange and Coulomb energy
             + (16 * M * N * N - 16 * N ** 3 / 3) / 5)        # QR every 5 steps
 
 
@@ -405,12 +422,14 @@ def bench_batch(args, A, torch, synth):
             it["ham"].enable_timers(16 * steps + 16)
         b.run_sequential()
         torch.cuda.synchronize()
-        ex_flop, ex_ms = 0.0, 0.0
+        calls, ex_ms = [], 0.0
         for it in b.items:
             tm = it["ham"].read_timers()
             it["ham"].enable_timers(0)
             sy = it["sys"]
-            ex_flop += tm["exchange"][1] * exchange_flops(it["W"], sy.M, sy.N, sy.K)
+            flop, peak = energy_work(name, it["ham"].energy_route(it["W"]) == A.ROUTE_TABLE, it["W"],
+                                     sy.M, sy.N, sy.K)
+            calls.append((tm["exchange"][1] * flop, peak, tm["exchange"][0]))
             ex_ms += tm["exchange"][0]
         ref = [it["wset"].buf.clone() for it in b.items]
         b.reset()
@@ -426,8 +445,11 @@ def bench_batch(args, A, torch, synth):
         bat = start.elapsed_time(stop) / 1e3
         same = all(same_bits(torch, it["wset"].buf, r) for it, r in zip(b.items, ref))
         ws = b.walker_steps()
-        ex_tf = ex_flop / (ex_ms / 1e3) / 1e12 if ex_ms > 0 else 0.0
+        ex_tf, ex_frac = energy_roofline(calls)
         res[name] = {"exchange_tflops": round(ex_tf, 3),
+                     "exchange_frac": None if ex_frac is None else round(ex_frac, 4),
+                     "systems_over_pair_table": sum(it["ham"].energy_route(it["W"]) == A.ROUTE_TABLE
+                                                    for it in b.items),
                      "exchange_ms_per_step": round(ex_ms / steps, 4),
                      "tilings_autotuned": len(b.tilings),
                      "batched_walker_steps_per_s": round(ws / bat, 1),
@@ -461,11 +483,12 @@ def bench_batch(args, A, torch, synth):
                                  res["fp64"]["batched_walker_steps_per_s"], 3),
         "roofline": {"bound": "mfma", "achieved": res[head]["exchange_tflops"],
                      "peak": PEAK_TFLOPS["fp64"], "unit": "TFLOP/s",
-                     "frac": round(res[head]["exchange_tflops"] / PEAK_TFLOPS["fp64"], 4),
+                     "frac": res[head]["exchange_frac"],
                      "traffic": None,
                      "kernel": f"exchange and Coulomb energy ({head} form) over all systems: total "
-                               f"FLOP of the cheaper route / total launch time, one-at-a-time "
-                               f"timed run"},
+                               f"FLOP of the route each system takes / total launch time, "
+                               f"one-at-a-time timed run; frac: each against the peak of its "
+                               f"arithmetic"},
         "cpu_baseline": None if args.no_cpu else batch_cpu_baseline(systems, ortho,
                                                                     args.cpu_seconds),
     }
@@ -563,9 +586,12 @@ def bench_single(args, A, torch, synth, workload, with_cpu, with_hybrid):
     value = W * args.steps / (head["ms"] / 1e3)
     ex_ms, ex_n = head["timers"]["exchange"]
     ex_avg = ex_ms / max(ex_n, 1)
-    achieved = exchange_flops(W, M, N, K) / (ex_avg / 1e3) / 1e12
-    peak = PEAK_TFLOPS["fp64"]
-    traffic = TRAFFIC_BYTES.get(workload)
+    table = {f: r["ham"].energy_route(W) == A.ROUTE_TABLE for f, r in forms.items()}
+    work = {f: energy_work(f, table[f], W, M, N, K) for f in forms}
+    flop, peak = work[mixed]
+    achieved, frac = energy_roofline([(flop, peak, ex_avg)])
+    traffic = TRAFFIC_BYTES.get(workload) if table[mixed] else None
+    arith = "fp64" if table[mixed] else mixed
     out = {
         "metric": METRIC,
         "value": round(value, 1),
@@ -577,31 +603,34 @@ def bench_single(args, A, torch, synth, workload, with_cpu, with_hybrid):
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "fp64" if mixed == "fp64" else f"{VBIAS_VHS[mixed]} vbias and vHS / fp64",
+        "dtype": "fp64" if mixed == "fp64" else f"{VBIAS_VHS[mixed]} vbias and vHS / fp64"
+                 if table[mixed] else f"{mixed} contractions / fp64",
         "data": "synthetic",
         "config": {"workload": f"{s.name}: NMO={M}, {N}+{N} electrons, Nchol={K}, {W} walkers, "
                                f"dt={s.dt}, local-energy step, QR every {ortho}",
                    "form": f"{mixed}: vbias and vHS in {VBIAS_VHS[mixed]}, exchange and Coulomb "
-                           "energy, G/LU/QR/propagation/weights in fp64",
+                           f"energy in {arith}, G/LU/QR/propagation/weights in fp64",
                    "parallelism": "single GPU"},
         "roofline": {"bound": "mfma", "achieved": round(achieved, 3), "peak": peak,
-                     "unit": "TFLOP/s", "frac": round(achieved / peak, 4),
+                     "unit": "TFLOP/s", "frac": None if frac is None else round(frac, 4),
                      "traffic": traffic,
                      "traffic_unit": "bytes per launch",
                      "traffic_source": TRAFFIC_SOURCE.get(workload) if traffic else None,
-                     "kernel": "exchange (k_gemm_real, quadratic form) and Coulomb traces, FP64 MFMA",
-                     "flop_per_launch": exchange_flops(W, M, N, K),
+                     "kernel": "exchange (k_gemm_real, quadratic form) and Coulomb traces, FP64 MFMA"
+                               if table[mixed] else f"exchange and Coulomb traces per Cholesky vector "
+                                                    f"({mixed})",
+                     "flop_per_launch": flop,
                      "mean_launch_ms": round(ex_avg, 5)},
     }
     if ref_form is not None:
         v64 = W * args.steps / (ref_form["ms"] / 1e3)
         ex64 = ref_form["timers"]["exchange"]
         ex64_avg = ex64[0] / max(ex64[1], 1)
-        tf64 = exchange_flops(W, M, N, K) / (ex64_avg / 1e3) / 1e12
+        tf64, frac64 = energy_roofline([(*work["fp64"], ex64_avg)])
         out["fp64"] = {"value": round(v64, 1),
                        "ms_per_step": round(ref_form["ms"] / args.steps, 4),
                        "exchange_tflops": round(tf64, 3),
-                       "exchange_frac_fp64_peak": round(tf64 / PEAK_TFLOPS["fp64"], 4)}
+                       "exchange_frac_fp64_peak": frac64 and round(frac64, 4)}
         out["mixed_over_fp64"] = round(value / v64, 3)
     out["max_abs_dEloc_Ha"] = {f: gate[f] for f in gate}
     out["contraction_rel_err_vs_fp64"] = {f: {k: float(f"{e:.3g}") for k, e in c.items()}
@@ -609,21 +638,22 @@ def bench_single(args, A, torch, synth, workload, with_cpu, with_hybrid):
     out["headline_form"] = mixed
     out["forms_walker_steps_per_s"] = {f: round(W * args.steps / (r["ms"] / 1e3), 1)
                                        for f, r in forms.items()}
-    # MFMA utilisation of each form's energy region: executed FP64 matrix operations over its mean
-    # time, against the dense peak
+    # MFMA utilisation of each form's energy region: executed matrix operations over its mean time,
+    # against the dense peak of their arithmetic
     util = {}
     for f, r in forms.items():
         ms_, n_ = r["timers"]["exchange"]
         if n_:
-            ex_rate = exchange_flops(W, M, N, K) / (ms_ / n_ / 1e3) / 1e12
-            util[f] = round(ex_rate / PEAK_TFLOPS["fp64"], 4)
+            fr = energy_roofline([(*work[f], ms_ / n_)])[1]
+            util[f] = None if fr is None else round(fr, 4)
+    out["energy_over_pair_table"] = table
     out["exchange_mfma_utilisation"] = util
     if unsupported:
         out["forms_unsupported"] = unsupported
     if fastest != mixed:
         out["note"] = (f"{fastest} is faster but misses |dE_loc| < {GATE_HA} Ha "
                        f"({gate[fastest]:.2e} Ha); value is the fastest form within the gate")
-    out["step_tflops"] = round(W * step_flops(M, N, K) / (ms_step / 1e3) / 1e12, 3)
+    out["step_tflops"] = round(W * step_flops(M, N, K, flop / W) / (ms_step / 1e3) / 1e12, 3)
     out["regions_ms_per_step"] = {k: round(v[0] / args.steps, 4) for k, v in head["timers"].items()
                                   if v[1]}
     out["timing"] = ("one HIP graph of the timed steps, replayed once" if head["graph"] is not None
@@ -657,7 +687,7 @@ def bench_single(args, A, torch, synth, workload, with_cpu, with_hybrid):
 # keys of a secondary workload's line kept under its name in the headline line
 EXTRA_KEYS = ("value", "ms_per_step", "config", "headline_form", "fp64", "mixed_over_fp64",
               "max_abs_dEloc_Ha", "forms_walker_steps_per_s", "forms_unsupported", "roofline",
-              "exchange_mfma_utilisation", "contraction_rel_err_vs_fp64",
+              "exchange_mfma_utilisation", "energy_over_pair_table", "contraction_rel_err_vs_fp64",
               "regions_ms_per_step", "graph_matches_eager")
 
 
