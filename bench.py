@@ -16,8 +16,9 @@ and energy sums stay FP64. Each form runs its timed steps twice from the same st
 timers (HIP events on the launch stream), then as one captured HIP graph replayed once; the
 graph's final walker buffer must equal the eager run's bit for bit (graph_matches_eager).
 `value` is the graph throughput of the fastest form whose largest per-walker
-|E_loc(form) - E_loc(FP64)| on identical walker states is below 1e-5 Ha; the line carries every
-form's throughput and gate error. A step = one pass over all walkers.
+|E_loc(form) - E_loc(FP64)| on identical walker states is below 1e-5 Ha and whose vbias and vHS there
+are within 4e-6 of FP64's largest (E_loc over the pair table is the same in every form); the line
+carries every form's throughput and both errors. A step = one pass over all walkers.
 
 roofline: the exchange and Coulomb energy kernels (the dominant region), executed matrix FLOP per
 call of the route they took (over the pair table W*(2 (N M)^2 + 4 N M K), FP64) divided by the region's
@@ -43,6 +44,10 @@ PEAK_TFLOPS = {"fp64": 78.6, "fp32": 157.3, "bf16x3": 2500.0}
 # arithmetic of vbias and vHS in each form
 VBIAS_VHS = {"fp64": "fp64", "fp32": "fp32", "bf16x3": "bf16x3", "int8": "fp32"}
 GATE_HA = 1e-5
+# vbias and vHS on identical states, max |x - x64| / max |x64|: 2^-24 times the square root of a sum of
+# 4096 products, the most of the workloads here. FP32 operands keep it (5e-7 to 1.5e-6); BF16X3's of 16
+# to 17 bits do not (7e-6 to 8e-6).
+GATE_CONTRACTION = 4e-6
 # HBM bytes per launch of the quadratic form's kernel (FETCH_SIZE and WRITE_SIZE counter runs scaled
 # by a copy kernel of known size); None for a workload without such a measurement
 TRAFFIC_BYTES = {"c2": 33.37e6, "c3": 1062.14e6}
@@ -71,6 +76,15 @@ def energy_roofline(calls):
         return 0.0, None
     frac = None if any(c[1] is None for c in calls) else sum(c[0] / c[1] for c in calls) / (ms * 1e9)
     return sum(c[0] for c in calls) / (ms * 1e9), frac
+
+
+def meets_gate(form, dEloc, contraction):
+    """Whether a form may be the headline: its E_loc within GATE_HA of FP64's on identical walker states
+    and, as E_loc does not depend on them, its vbias and vHS within GATE_CONTRACTION. A form without
+    these measurements does not."""
+    return form == "fp64" or (
+        dEloc.get(form, 1.0) < GATE_HA
+        and all(contraction.get(form, {}).get(k, 1.0) < GATE_CONTRACTION for k in ("vbias", "vHS")))
 
 
 def step_flops(M, N, K, energy):
@@ -576,7 +590,7 @@ def bench_single(args, A, torch, synth, workload, with_cpu, with_hybrid):
                   f"vHS {cerr[f]['vHS']:.2e} (G is FP64 in every form)", file=sys.stderr,
                   flush=True)
         del states, run
-    passing = [f for f in forms if f == "fp64" or gate.get(f, 1.0) < GATE_HA]
+    passing = [f for f in forms if meets_gate(f, gate, cerr)]
     # the headline: the fastest form that meets the accuracy gate
     mixed = min(passing, key=lambda f: forms[f]["ms"])
     fastest = min(forms, key=lambda f: forms[f]["ms"])
@@ -651,8 +665,9 @@ def bench_single(args, A, torch, synth, workload, with_cpu, with_hybrid):
     if unsupported:
         out["forms_unsupported"] = unsupported
     if fastest != mixed:
-        out["note"] = (f"{fastest} is faster but misses |dE_loc| < {GATE_HA} Ha "
-                       f"({gate[fastest]:.2e} Ha); value is the fastest form within the gate")
+        out["note"] = (f"{fastest} is faster but misses |dE_loc| < {GATE_HA} Ha or a relative error "
+                       f"of vbias and vHS below {GATE_CONTRACTION} ({gate.get(fastest)} Ha, "
+                       f"{cerr.get(fastest)}); value is the fastest form within the gate")
     out["step_tflops"] = round(W * step_flops(M, N, K, flop / W) / (ms_step / 1e3) / 1e12, 3)
     out["regions_ms_per_step"] = {k: round(v[0] / args.steps, 4) for k, v in head["timers"].items()
                                   if v[1]}

@@ -22,3 +22,15 @@ def test_energy_roofline_weighs_each_call_by_its_own_peak():
     assert frac == pytest.approx((0.02 + 0.009) / 0.2)      # ms at the peaks over the ms taken
     assert bench.energy_roofline([(2e9, 100.0, 0.05), (9e9, None, 0.15)]) == (pytest.approx(55.0), None)
     assert bench.energy_roofline([]) == (0.0, None)
+
+
+def test_gate_sees_the_contractions_that_the_forms_change():
+    dE = {"fp32": 0.0, "bf16x3": 0.0, "int8": 2e-10}     # over the pair table E_loc is FP64's
+    errors = {"fp32": {"vbias": 1.1e-6, "vHS": 1.5e-6}, "bf16x3": {"vbias": 8.0e-6, "vHS": 7.9e-6},
+              "int8": {"vbias": 1.1e-6, "vHS": 4.1e-6}}
+    assert bench.meets_gate("fp64", {}, {})
+    assert bench.meets_gate("fp32", dE, errors)
+    assert not bench.meets_gate("bf16x3", dE, errors)
+    assert not bench.meets_gate("int8", dE, errors)
+    assert not bench.meets_gate("fp32", {"fp32": 1e-5}, errors)
+    assert not bench.meets_gate("fp32", dE, {}) and not bench.meets_gate("fp32", {}, errors)
