@@ -214,7 +214,8 @@ class HamiltonianOperations:
 
     def autotune(self, W, cache_path=None, stream=None):
         """Picks the fastest GEMM tilings for W walkers (cached in cache_path, a JSON file);
-        returns the (vbias, vHS) tilings."""
+        returns the (vbias, vHS) entries (vHS: the full product's tiling + 4 times that of the
+        step's packed triangle)."""
         self.reserve(W)
         out = (C.c_int * 2)()
         path = None if cache_path is None else os.fsencode(cache_path)

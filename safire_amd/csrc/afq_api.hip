@@ -474,7 +474,7 @@ int afq_ham_set_precision(afq_ham H, int precision) {
     AFQ_CHECK(precision != AFQ_INT8_SPLIT || H->Lnak_q != nullptr, AFQ_EUNSUPPORTED,
               "INT8_SPLIT exchange needs N <= 32 and M <= 128");
     H->precision = precision;
-    H->cfg_vbias = H->cfg_vhs = 0;   // tilings are tuned per precision (afq_autotune)
+    H->cfg_vbias = H->cfg_vhs = H->cfg_vhs_step = 0;   // tilings are tuned per precision (afq_autotune)
   });
 }
 
@@ -549,6 +549,9 @@ int afq_ham_stats(afq_ham H, long long* eloc3, long long* weight2, long long* po
 }  // extern "C"
 
 namespace {
+
+// the vHS entry: the tiling of afq_vhs's product plus this many times that of the step's packed triangle
+constexpr int kVhsTilings = 4;
 
 // the cache: a JSON object of "key": tiling entries (string keys, integer values)
 std::map<std::string, int> read_tile_cache(const char* path) {
@@ -630,36 +633,46 @@ int afq_autotune(afq_ham H, int W, const char* cache_path, int* cfg_out, void* s
     const long NM = (long)N * M;
     Workspace& ws = H->ws;
     auto cache = read_tile_cache(cache_path);
-    auto key = [&](const char* what, long a, long b) {
-      std::ostringstream k;
-      k << what << "/p" << p << "/W" << W << "/" << a << "x" << b;
+    auto key = [&](const char* what, bool real_kernel, long a, long b) {
+      std::ostringstream k;   // a tiling belongs to its kernel: launch_gemm_real or launch_gemm_nt_z
+      k << what << (real_kernel ? "/real" : "/nt") << "/p" << p << "/W" << W << "/" << a << "x" << b;
       return k.str();
     };
-    auto tune = [&](const std::string& k, bool bc, auto&& launch) {
-      const auto it = cache.find(k);
-      if (it != cache.end() && it->second >= 0 && it->second < gemm_tile_configs(p, bc))
-        return it->second;
+    auto fastest = [&](int n, auto&& launch) {
       int best = 0;
       float tbest = 0.0f;
-      for (int c = 0; c < gemm_tile_configs(p, bc); ++c) {
+      for (int c = 0; c < n; ++c) {
         const float t = time_launches(s, 10, [&] { launch(c); });
         if (c == 0 || t < tbest) {
           best = c;
           tbest = t;
         }
       }
-      cache[k] = best;
       return best;
     };
-    H->cfg_vbias = tune(key("vbias", K, NM), true,
-                        [&](int c) { run_vbias(H, s, W, ws.G, ws.X, c); });
-    H->cfg_vhs = tune(key("vhs", (long)M * M, K), false,
-                      [&](int c) { run_vhs_step(H, s, W, ws.X, ws.V, c); });
+    auto cached = [&](const std::string& k, int n) {
+      const auto it = cache.find(k);
+      return it != cache.end() && it->second >= 0 && it->second < n ? it->second : -1;
+    };
+    const bool vb_real = H->real_trial && p != AFQ_BF16X3, packed = H->sym && p != AFQ_BF16X3;
+    const int n_vb = vb_real ? gemm_real_tile_configs(p) : gemm_tile_configs(p, true);
+    const int n_full = gemm_tile_configs(p, false), n_step = packed ? gemm_real_tile_configs(p) : 1;
+    const std::string kv = key("vbias", vb_real, K, NM), kh = key("vhs", packed, (long)M * M, K);
+    int vb = cached(kv, n_vb), vh = cached(kh, n_full + kVhsTilings * (n_step - 1));
+    if (vb < 0) vb = fastest(n_vb, [&](int c) { run_vbias(H, s, W, ws.G, ws.X, c); });
+    if (vh < 0 || vh % kVhsTilings >= n_full) {
+      vh = fastest(n_full, [&](int c) { run_vhs(H, s, W, ws.X, ws.V, c); });
+      if (packed) vh += kVhsTilings * fastest(n_step, [&](int c) { run_vhs_step(H, s, W, ws.X, ws.V, c); });
+    }
+    cache[kv] = H->cfg_vbias = vb;
+    cache[kh] = vh;
+    H->cfg_vhs = vh % kVhsTilings;
+    H->cfg_vhs_step = packed ? vh / kVhsTilings : H->cfg_vhs;
     AFQ_HIP(hipStreamSynchronize(s));
     write_tile_cache(cache_path, cache);
     if (cfg_out) {
       cfg_out[0] = H->cfg_vbias;
-      cfg_out[1] = H->cfg_vhs;
+      cfg_out[1] = vh;
     }
   });
 }
@@ -843,7 +856,7 @@ int afq_step(afq_ham H, int W, double* wbuf, long ldw, const double* xi, double 
     VKind kind = VKind::full;
     {
       RegionScope r(tm, s, R_VHS);
-      kind = run_vhs_step(H, s, W, ws.X, ws.V, H->cfg_vhs);
+      kind = run_vhs_step(H, s, W, ws.X, ws.V, H->cfg_vhs_step);
     }
     {
       RegionScope r(tm, s, R_PROPAGATE);

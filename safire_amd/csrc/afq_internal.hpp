@@ -176,7 +176,7 @@ struct afq_ham_s {
   double ci0_re = 1.0, ci0_im = 0.0;
   int precision = AFQ_FP64;
   int energy_route = AFQ_ROUTE_AUTO;
-  int cfg_vbias = 0, cfg_vhs = 0;   // GEMM tilings (afq_autotune)
+  int cfg_vbias = 0, cfg_vhs = 0, cfg_vhs_step = 0;   // GEMM tilings (afq_autotune): vbias, afq_vhs, a step's vHS
   afq_step_params params;
   int device = 0;
   // device tensors (built on the GPU at create)
@@ -252,6 +252,7 @@ void launch_gemm_nt_z(hipStream_t s, int precision, int m, int n, int k, double 
 // for AFQ_FP64, else f32). nanmix: an Inf or NaN in A makes both parts of its row's sums NaN, as the
 // zero imaginary part of a complex B does. FP32 gives launch_gemm_nt_z's bits.
 int gemm_real_row(int k);
+int gemm_real_tile_configs(int precision);   // its tilings (cfg: 0 .. n-1)
 // padded rows dst[row][0..gemm_real_row(k)) = src[row][0..k) (the real part of a complex src);
 // packed_n > 0: the packed_n (packed_n + 1) / 2 rows i <= j of the n x n rows of src
 void launch_pad_rows(hipStream_t s, long rows, int k, int packed_n, const double* src, bool complex_src,

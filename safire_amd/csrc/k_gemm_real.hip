@@ -425,6 +425,9 @@ void launch_pair_exchange(hipStream_t s, int W, int NM, bool real, int max_parts
   AFQ_HIP(hipGetLastError());
 }
 
+// FP64 takes the tile of gemm_f64_plan
+int gemm_real_tile_configs(int precision) { return precision == AFQ_FP64 ? 1 : 4; }
+
 int gemm_real_row(int k) { return (k + 15) / 16 * 16; }
 
 void launch_pad_rows(hipStream_t s, long rows, int k, int packed_n, const double* src, bool complex_src,
