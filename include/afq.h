@@ -108,7 +108,9 @@ int afq_ham_create(int M, int N, int K, const double* h_h, const double* h_Likn,
                    const double* h_PsiT, double E0, double dt, int walker_type, afq_ham* out);
 int afq_ham_destroy(afq_ham ham);
 /* Sizes the per-step workspace for up to max_walkers walkers (the only allocation after
- * create). Re-reserving with a larger count reallocates. */
+ * create). Re-reserving with a larger count reallocates. Where memory is short, the pair table and the
+ * other copies that only faster paths read are given back first (afq_ham_create makes them only where
+ * each takes at most an eighth of the free memory); a route set to the table keeps it. */
 int afq_ham_reserve(afq_ham ham, int max_walkers);
 int afq_ham_set_precision(afq_ham ham, int precision);
 /* The route of the energies of this handle (AFQ_ROUTE_AUTO after create; AFQ_EUNSUPPORTED for the table

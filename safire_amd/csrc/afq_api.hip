@@ -68,6 +68,19 @@ void dfree(T*& p) {
   p = nullptr;
 }
 
+// A buffer that only a faster path needs: allocated where it takes at most an eighth of the free memory
+// (what the caller allocates next has to fit beside it), else *p stays NULL.
+template <typename T>
+bool dalloc_optional(T** p, size_t n) {
+  size_t free_bytes = 0, total = 0;
+  if (hipMemGetInfo(&free_bytes, &total) == hipSuccess && n * sizeof(T) <= free_bytes / 8 &&
+      hipMalloc(reinterpret_cast<void**>(p), n * sizeof(T)) == hipSuccess)
+    return true;
+  *p = nullptr;
+  (void)hipGetLastError();
+  return false;
+}
+
 void free_workspace(Workspace& ws) {
   dfree(ws.G);
   dfree(ws.X);
@@ -87,6 +100,95 @@ void free_workspace(Workspace& ws) {
   dfree(ws.src);
   dfree(ws.ok);
   ws.cap = 0;
+}
+
+// The pair table is kept where 32768 walkers take less time with it in FP64: 2 (N M)^2 operations, half
+// of the square, and 4 N M K for the Coulomb traces (T_n = G Lnak_n^T: 4 N^2 M K), twice that for complex
+// trials, at the 60 and 50 TFLOP/s of M 128, N 32, K 640 with 1024 walkers.
+bool pair_table_pays(afq_ham H) {
+  const double NM = (double)H->N * H->M, rows = 32768.0, z = H->real_trial ? 1.0 : 2.0;
+  return 15.0 + z * rows * NM * (2.0 * NM + 4.0 * H->K) / 60e6 < 4.0 + 4.0 * z * rows * NM * H->N * H->K / 50e6;
+}
+
+// The tensors of the faster paths, after all those that the handle cannot do without: real rows of Lnak
+// (vbias and the FP64 exchange of a real trial), the triangle of symmetric vectors (vHS of a step) and the
+// pair table. Without one of them the general kernels run.
+void add_optional_tensors(afq_ham H) {
+  const int M = H->M, N = H->N, K = H->K;
+  const size_t NM = (size_t)N * M;
+  if (H->real_trial) {
+    if (dalloc_optional(&H->Lnak_r, (size_t)K * N * real_lnak_row(M)))
+      launch_real_rows(nullptr, (long)K * N, M, real_lnak_row(M), H->Lnak, H->Lnak_r);
+    const size_t n = (size_t)K * gemm_real_row((int)NM);
+    if (dalloc_optional(&H->Lvb_d, n) && !dalloc_optional(&H->Lvb_f, n)) dfree(H->Lvb_d);
+    if (H->Lvb_d) {
+      launch_pad_rows(nullptr, K, (int)NM, 0, H->Lnak, true, H->Lvb_d);
+      launch_pad_rows(nullptr, K, (int)NM, 0, H->Lnak, true, H->Lvb_f);
+    }
+  }
+  if (likn_symmetric(nullptr, M, K, H->Likn)) {
+    const long np = (long)M * (M + 1) / 2;
+    const size_t n = (size_t)np * gemm_real_row(K);
+    if (dalloc_optional(&H->Lp_d, n) && !dalloc_optional(&H->Lp_f, n)) dfree(H->Lp_d);
+    H->sym = H->Lp_d != nullptr;
+    if (H->sym) {
+      launch_pad_rows(nullptr, np, K, M, H->Likn, false, H->Lp_d);
+      launch_pad_rows(nullptr, np, K, M, H->Likn, false, H->Lp_f);
+    }
+  }
+  // at most 2 GiB (N M = 16384 for a real trial), and only where many walkers take fewer operations
+  const size_t pe = pair_table_elems((int)NM, H->real_trial);
+  if (pe <= (size_t)1 << 28 && 2 * (NM / 64 + 1) <= (size_t)K && pair_table_pays(H) &&
+      (H->Lvb_d || !H->real_trial) && dalloc_optional(&H->pairs, pe))
+    launch_pair_table(nullptr, M, N, K, H->real_trial ? H->Lvb_d : H->Lnak, H->real_trial, H->pairs);
+}
+
+// Gives back what the workspace may need more: the pair table first, then the other tensors of the faster
+// paths (a route set to the table keeps it, with the rows that its traces read). False: nothing is left.
+bool drop_optional_tensors(afq_ham H) {
+  const bool keep = H->energy_route == AFQ_ROUTE_TABLE;
+  if (H->pairs && !keep) {
+    dfree(H->pairs);
+    return true;
+  }
+  if (!H->Lnak_r && !H->Lp_d && (keep || !H->Lvb_d)) return false;
+  dfree(H->Lnak_r);
+  H->sym = false;
+  dfree(H->Lp_d);
+  dfree(H->Lp_f);
+  if (!keep) {
+    dfree(H->Lvb_d);
+    dfree(H->Lvb_f);
+  }
+  H->cfg_vbias = H->cfg_vhs = H->cfg_vhs_step = 0;   // tuned for other kernels
+  return true;
+}
+
+void reserve_workspace(afq_ham H, int max_walkers) {
+  free_workspace(H->ws);
+  const size_t W = max_walkers;
+  const size_t M = H->M, N = H->N, K = H->K;
+  Workspace& ws = H->ws;
+  dalloc(&ws.G, 2 * W * N * M);
+  dalloc(&ws.X, 2 * W * K);
+  dalloc(&ws.V, 2 * W * M * M);
+  dalloc(&ws.HW, 2 * W);
+  dalloc(&ws.mf, 2 * W);
+  dalloc(&ws.ov, 2 * W);
+  dalloc(&ws.E, 6 * W);
+  dalloc(&ws.Kl, 2 * W * K);
+  dalloc(&ws.exx, 2 * W * (size_t)(K + 2));   // at most K + 1 tr(T^2) partials per walker
+  ws.split_elems = (long)kMaxSplits * W * K;
+  dalloc(&ws.split, 2 * (size_t)ws.split_elems);
+  dalloc(&ws.cum, W);
+  dalloc(&ws.off, W);
+  dalloc(&ws.src, W);
+  dalloc(&ws.ok, 1);
+  if (H->pairs) {   // 128 MiB at most: products with more entries fill the chip unsplit
+    ws.esplit_elems = std::min((long)kMaxSplits * max_walkers * H->K, 1L << 23);
+    if (!dalloc_optional(&ws.esplit, 2 * (size_t)ws.esplit_elems)) ws.esplit_elems = 0;
+  }
+  ws.cap = max_walkers;
 }
 
 void check_ham(afq_ham H) { AFQ_CHECK(H != nullptr, AFQ_EINVAL, "null afq_ham"); }
@@ -118,7 +220,7 @@ void run_vbias(afq_ham H, hipStream_t s, int W, const double* G, double* v, int 
   if (H->precision == AFQ_BF16X3)
     launch_gemm_bf16(s, W, H->K, (int)NM, alpha, G, NM, H->Lnak_g, true, v, H->K, H->ws.split,
                      H->ws.split_elems);
-  else if (H->real_trial)
+  else if (H->Lvb_d)
     launch_gemm_real(s, H->precision, W, H->K, (int)NM, alpha, G, NM,
                      H->precision == AFQ_FP64 ? (const void*)H->Lvb_d : (const void*)H->Lvb_f, v,
                      H->K, true, H->ws.split, H->ws.split_elems, cfg);
@@ -151,14 +253,6 @@ VKind run_vhs_step(afq_ham H, hipStream_t s, int W, const double* X, double* V, 
 }
 
 const double* P1r_of(afq_ham H) { return H->P1_real ? H->P1r : nullptr; }
-
-// The pair table is kept where 32768 walkers take less time with it in FP64: 2 (N M)^2 operations, half
-// of the square, and 4 N M K for the Coulomb traces (T_n = G Lnak_n^T: 4 N^2 M K), twice that for complex
-// trials, at the 60 and 50 TFLOP/s of M 128, N 32, K 640 with 1024 walkers.
-bool pair_table_pays(afq_ham H) {
-  const double NM = (double)H->N * H->M, rows = 32768.0, z = H->real_trial ? 1.0 : 2.0;
-  return 15.0 + z * rows * NM * (2.0 * NM + 4.0 * H->K) / 60e6 < 4.0 + 4.0 * z * rows * NM * H->N * H->K / 50e6;
-}
 
 // Estimated us of the energy's contractions per Cholesky vector in the handle's form and over the pair
 // table: linear in the work that the launches of each do, padding and rounds of workgroups included.
@@ -344,32 +438,6 @@ int afq_ham_create(int M, int N, int K, const double* h_h, const double* h_Likn,
       H->real_trial = true;
       for (size_t e = 0; e < NM; ++e) H->real_trial = H->real_trial && h_PsiT[2 * e + 1] == 0.0;
       setup_hamiltonian(H, nullptr);
-      if (H->real_trial) {
-        dalloc(&H->Lnak_r, (size_t)K * N * real_lnak_row(M));
-        launch_real_rows(nullptr, (long)K * N, M, real_lnak_row(M), H->Lnak, H->Lnak_r);
-        dalloc(&H->Lvb_d, (size_t)K * gemm_real_row((int)NM));
-        dalloc(&H->Lvb_f, (size_t)K * gemm_real_row((int)NM));
-        launch_pad_rows(nullptr, K, (int)NM, 0, H->Lnak, true, H->Lvb_d);
-        launch_pad_rows(nullptr, K, (int)NM, 0, H->Lnak, true, H->Lvb_f);
-      }
-      // at most 2 GiB (N M = 16384 for a real trial), and only where many walkers take fewer operations
-      const size_t pe = pair_table_elems((int)NM, H->real_trial);
-      if (pe <= (size_t)1 << 28 && 2 * (NM / 64 + 1) <= (size_t)K && pair_table_pays(H)) {
-        if (hipMalloc(&H->pairs, pe * sizeof(double)) == hipSuccess) {
-          launch_pair_table(nullptr, M, N, K, H->real_trial ? H->Lvb_d : H->Lnak, H->real_trial, H->pairs);
-        } else {
-          H->pairs = nullptr;   // the exchange kernels need no table
-          (void)hipGetLastError();
-        }
-      }
-      H->sym = likn_symmetric(nullptr, M, K, H->Likn);
-      if (H->sym) {
-        const long np = (long)M * (M + 1) / 2;
-        dalloc(&H->Lp_d, (size_t)np * gemm_real_row(K));
-        dalloc(&H->Lp_f, (size_t)np * gemm_real_row(K));
-        launch_pad_rows(nullptr, np, K, M, H->Likn, false, H->Lp_d);
-        launch_pad_rows(nullptr, np, K, M, H->Likn, false, H->Lp_f);
-      }
       if (exchange_bf16_supported(M, N)) {
         dalloc(&H->Lnak_b, exchange_bf16_elems(M, N, K));
         split_lnak_bf16(nullptr, M, N, K, H->Lnak, H->Lnak_b);
@@ -385,6 +453,7 @@ int afq_ham_create(int M, int N, int K, const double* h_h, const double* h_Likn,
         dalloc(&H->Lnak_ord, (size_t)K);
         exchange_i8_orders(nullptr, M, N, K, H->Lnak, H->Lnak_ord);
       }
+      add_optional_tensors(H);
       AFQ_HIP(hipDeviceSynchronize());
     } catch (...) {
       afq_ham_destroy(H);
@@ -437,30 +506,16 @@ int afq_ham_reserve(afq_ham H, int max_walkers) {
     AFQ_CHECK(max_walkers >= 0, AFQ_EBADSHAPE, "negative walker count");
     if (max_walkers <= H->ws.cap) return;
     AFQ_HIP(hipDeviceSynchronize());
-    free_workspace(H->ws);
-    const size_t W = max_walkers;
-    const size_t M = H->M, N = H->N, K = H->K;
-    Workspace& ws = H->ws;
-    dalloc(&ws.G, 2 * W * N * M);
-    dalloc(&ws.X, 2 * W * K);
-    dalloc(&ws.V, 2 * W * M * M);
-    dalloc(&ws.HW, 2 * W);
-    dalloc(&ws.mf, 2 * W);
-    dalloc(&ws.ov, 2 * W);
-    dalloc(&ws.E, 6 * W);
-    dalloc(&ws.Kl, 2 * W * K);
-    dalloc(&ws.exx, 2 * W * (size_t)(K + 2));   // at most K + 1 tr(T^2) partials per walker
-    ws.split_elems = (long)kMaxSplits * W * K;
-    dalloc(&ws.split, 2 * (size_t)ws.split_elems);
-    if (H->pairs) {   // 128 MiB at most: products with more entries fill the chip unsplit
-      ws.esplit_elems = std::min((long)kMaxSplits * max_walkers * H->K, 1L << 23);
-      dalloc(&ws.esplit, 2 * (size_t)ws.esplit_elems);
+    for (;;) {
+      try {
+        reserve_workspace(H, max_walkers);
+        return;
+      } catch (const Error& e) {
+        free_workspace(H->ws);
+        (void)hipGetLastError();
+        if (e.code != AFQ_ENOMEM || !drop_optional_tensors(H)) throw;
+      }
     }
-    dalloc(&ws.cum, W);
-    dalloc(&ws.off, W);
-    dalloc(&ws.src, W);
-    dalloc(&ws.ok, 1);
-    ws.cap = max_walkers;
   });
 }
 
@@ -654,7 +709,7 @@ int afq_autotune(afq_ham H, int W, const char* cache_path, int* cfg_out, void* s
       const auto it = cache.find(k);
       return it != cache.end() && it->second >= 0 && it->second < n ? it->second : -1;
     };
-    const bool vb_real = H->real_trial && p != AFQ_BF16X3, packed = H->sym && p != AFQ_BF16X3;
+    const bool vb_real = H->Lvb_d && p != AFQ_BF16X3, packed = H->sym && p != AFQ_BF16X3;
     const int n_vb = vb_real ? gemm_real_tile_configs(p) : gemm_tile_configs(p, true);
     const int n_full = gemm_tile_configs(p, false), n_step = packed ? gemm_real_tile_configs(p) : 1;
     const std::string kv = key("vbias", vb_real, K, NM), kh = key("vhs", packed, (long)M * M, K);
