@@ -301,6 +301,7 @@ bool use_pairs(afq_ham H, int W) {
 
 // the exchange contraction in the handle's precision: Kl and per-chunk tr(T^2) partials
 void run_exchange(afq_ham H, hipStream_t s, int W, const double* G) {
+  if (H->precision == AFQ_INT8_SPLIT && W > 0) exchange_i8_check(H->M, H->N, H->K);   // on either route
   if (use_pairs(H, W)) {
     const int NM = H->N * H->M;
     if (H->real_trial)

@@ -314,6 +314,7 @@ int exchange_i8_chunks(int W, int M, int N, int K, bool real);   // tr(T^2) part
 void split_lnak_i8(hipStream_t s, int M, int N, int K, const double* Lnak, bool real, int8_t* Lq,
                    double* Lu);
 // per Cholesky vector the slice-product order (set-up, synchronous)
+void exchange_i8_check(int M, int N, int K);   // AFQ_EUNSUPPORTED for shapes that the int8 form refuses
 void exchange_i8_orders(hipStream_t s, int M, int N, int K, const double* Lnak, int* ord);
 void launch_exchange_i8(hipStream_t s, int W, int M, int N, int K, const double* G, bool real,
                         const int8_t* Lq, const double* Lu, const int* ord, double* Kl,

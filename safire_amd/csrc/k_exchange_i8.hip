@@ -475,15 +475,19 @@ void split_lnak_i8(hipStream_t s, int M, int N, int K, const double* Lnak, bool 
   AFQ_HIP(hipGetLastError());
 }
 
+void exchange_i8_check(int M, int N, int K) {
+  AFQ_CHECK(exchange_i8_supported(M, N), AFQ_EUNSUPPORTED,
+            "int8 exchange: needs N <= 32 and M <= 128");
+  AFQ_CHECK((size_t)(N > 16 ? 12 : 10) * K * N * exchange_i8_row(M) < (1UL << 31), AFQ_EUNSUPPORTED,
+            "int8 exchange: the Cholesky slices exceed 2 GiB");
+}
+
 void launch_exchange_i8(hipStream_t s, int W, int M, int N, int K, const double* G, bool real,
                         const int8_t* Lq, const double* Lu, const int* ord, double* Kl,
                         double* exx_part) {
   if (W <= 0 || K <= 0) return;
-  AFQ_CHECK(exchange_i8_supported(M, N), AFQ_EUNSUPPORTED,
-            "int8 exchange: needs N <= 32 and M <= 128");
+  exchange_i8_check(M, N, K);
   const int Mp = exchange_i8_row(M);
-  AFQ_CHECK((size_t)(N > 16 ? 12 : 10) * K * N * Mp < (1UL << 31), AFQ_EUNSUPPORTED,
-            "int8 exchange: the Cholesky slices exceed 2 GiB");
   AFQ_CHECK(ord != nullptr, AFQ_EINVAL, "int8 exchange: no slice orders");
   if (per_walker(W, M, N, K, real)) {
     launch_exchange_i8w(s, W, M, N, K, G, real, Lq, Lu, ord, Kl, exx_part);

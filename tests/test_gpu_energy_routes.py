@@ -128,3 +128,27 @@ def test_route_is_the_faster_one(M, N, K, complex_trial, W, form, vectors, table
     ham.set_precision(form)
     assert ham.energy_route(W) == (A.ROUTE_TABLE if table < vectors else A.ROUTE_VECTORS)
     ham.close()
+
+
+def test_int8_slices_of_2_gib_are_refused_on_both_routes():
+    M = N = 32
+    for K, refused in ((174763, True), (174762, False)):    # 12 K N 32 bytes around 2^31
+        L = np.zeros((M, M, K))
+        L[0, 0, ::97] = 0.01
+        ham = A.HamiltonianOperations(np.eye(M), L, np.eye(M, dtype=np.complex128), 0.0, 0.01)
+        del L
+        W = 8
+        ham.reserve(W)
+        ham.set_precision(A.INT8_SPLIT)
+        G = A.to_device(np.full((W, N * M), 0.1 + 0.0j))
+        E = torch.zeros((W, 3), dtype=torch.complex128, device="cuda")
+        for route in (A.ROUTE_TABLE, A.ROUTE_VECTORS):
+            ham.set_energy_route(route)
+            if refused:
+                with pytest.raises(A.AfqError) as e:
+                    ham.energy(G, E)
+                assert e.value.code == 5
+            else:
+                ham.energy(G, E)
+                torch.cuda.synchronize()
+        ham.close()
