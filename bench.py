@@ -45,12 +45,12 @@ PEAK_TFLOPS = {"fp64": 78.6, "fp32": 157.3, "bf16x3": 2500.0}
 VBIAS_VHS = {"fp64": "fp64", "fp32": "fp32", "bf16x3": "bf16x3", "int8": "fp32"}
 GATE_HA = 1e-5
 # vbias and vHS on identical states, max |x - x64| / max |x64|: 2^-24 times the square root of a sum of
-# 4096 products, the most of the workloads here. FP32 operands keep it (5e-7 to 1.5e-6); BF16X3's of 16
-# to 17 bits do not (7e-6 to 8e-6).
+# 4096 products, the most of the workloads here. FP32 operands keep it (3e-7 to 1.5e-6); BF16X3's of 16
+# to 17 bits do not (7e-6 to 1e-5).
 GATE_CONTRACTION = 4e-6
 # HBM bytes per launch of the quadratic form's kernel (FETCH_SIZE and WRITE_SIZE counter runs scaled
 # by a copy kernel of known size); None for a workload without such a measurement
-TRAFFIC_BYTES = {"c2": 33.37e6, "c3": 1062.14e6}
+TRAFFIC_BYTES = {"c2": 53.24e6, "c3": 1062.99e6}
 TRAFFIC_SOURCE = {"c2": "profiles/walker_step_c2_hbm_traffic.md",
                   "c3": "profiles/walker_step_c3_hbm_traffic.md"}
 

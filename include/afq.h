@@ -44,9 +44,10 @@ enum afq_status {
 enum afq_walker_type { AFQ_CLOSED = 1, AFQ_COLLINEAR = 2 };
 
 /* Arithmetic of the Cholesky contractions (vbias, vHS, exchange/Coulomb energy). Overlaps,
- * log-determinants, inverses, QR, the propagator, weights and energy sums stay FP64. Where the
- * exchange takes fewer operations from a table of orbital pairs (real trials with enough Cholesky
- * vectors and walkers), exchange and Coulomb energy are FP64 in every form. */
+ * log-determinants, inverses, QR, the propagator, weights and energy sums stay FP64. Where a table of
+ * orbital pairs is estimated to take less time than the form's kernels per Cholesky vector (enough
+ * vectors and walkers, real and complex trials), exchange and Coulomb energy are FP64 in every form;
+ * afq_ham_energy_route tells which, afq_ham_set_energy_route fixes it. */
 enum afq_precision {
   AFQ_FP64 = 0,        /* plain form: everything FP64 (FP64 MFMA)                          */
   AFQ_FP32 = 1,        /* contractions in FP32 on MFMA with FP32 accumulation               */

@@ -13,7 +13,8 @@
 // slice and wavefront; the 64 x 64 tiles of k_gemm_nt 8-byte reads of single elements for half as
 // many MFMAs, and twice the loads of B. Per launch, with the triangle of a symmetric vHS and the real
 // vectors of a real trial against k_gemm_nt on the full ones (M 128, N 32, K 640, 1024 walkers):
-// vHS FP64 905 -> 484 us, FP32 660 -> 288 us; vbias FP64 475 -> 230 us, FP32 277 -> 140 us. M 64,
+// vHS FP64 905 -> 484 us, FP32 660 -> 288 us (128 x 128 tiles by the rule below; 247 with the 64 x 64
+// that afq_autotune takes); vbias FP64 475 -> 230 us, FP32 277 -> 140 us. M 64,
 // N 16, K 320, 512 walkers, FP64: vHS 68 -> 46 us.
 //
 // The exchange as a quadratic form: sum_n tr(T_n^2) with T_n = G Lnak_n^T is G B G^T over the pairs
@@ -356,7 +357,7 @@ PairPlan pair_plan(int W, int NM, int planes, int max_parts) {
 }
 
 // FP64: the tile and the split of k with the shortest estimated time: workgroups of the fullest CU times
-// the work of one (234 MFLOP/s per us and CU where workgroups share it, 0.6 of it for one alone; the
+// the work of one (234 GFLOP/s per CU, 0.234e6 FLOP per us, where workgroups share it, 0.6 of it for one alone; the
 // smaller tiles at 0.95 and 0.8 of that), and the pass that adds the splits. Returns that time in us.
 double gemm_f64_plan(int m, int n, int k, long split_elems, int& tm, int& tn, int& splits) {
   const double cus = device_cus();
