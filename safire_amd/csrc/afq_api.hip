@@ -68,14 +68,23 @@ void dfree(T*& p) {
   p = nullptr;
 }
 
-// A buffer that only a faster path needs: allocated where it takes at most an eighth of the free memory
-// (what the caller allocates next has to fit beside it), else *p stays NULL.
-template <typename T>
-bool dalloc_optional(T** p, size_t n) {
+size_t free_memory() {
   size_t free_bytes = 0, total = 0;
-  if (hipMemGetInfo(&free_bytes, &total) == hipSuccess && n * sizeof(T) <= free_bytes / 8 &&
-      hipMalloc(reinterpret_cast<void**>(p), n * sizeof(T)) == hipSuccess)
+  if (hipMemGetInfo(&free_bytes, &total) == hipSuccess) return free_bytes;
+  (void)hipGetLastError();
+  return 0;
+}
+
+// A buffer that only a faster path needs: allocated where it takes at most an eighth of the free memory
+// (what the caller allocates next has to fit beside it), else *p stays NULL. free_bytes: of free_memory(),
+// less what has been allocated since (a query takes longer than an allocation).
+template <typename T>
+bool dalloc_optional(T** p, size_t n, size_t& free_bytes) {
+  if (n * sizeof(T) <= free_bytes / 8 &&
+      hipMalloc(reinterpret_cast<void**>(p), n * sizeof(T)) == hipSuccess) {
+    free_bytes -= n * sizeof(T);
     return true;
+  }
   *p = nullptr;
   (void)hipGetLastError();
   return false;
@@ -116,11 +125,12 @@ bool pair_table_pays(afq_ham H) {
 void add_optional_tensors(afq_ham H) {
   const int M = H->M, N = H->N, K = H->K;
   const size_t NM = (size_t)N * M;
+  size_t free_bytes = free_memory();
   if (H->real_trial) {
-    if (dalloc_optional(&H->Lnak_r, (size_t)K * N * real_lnak_row(M)))
+    if (dalloc_optional(&H->Lnak_r, (size_t)K * N * real_lnak_row(M), free_bytes))
       launch_real_rows(nullptr, (long)K * N, M, real_lnak_row(M), H->Lnak, H->Lnak_r);
     const size_t n = (size_t)K * gemm_real_row((int)NM);
-    if (dalloc_optional(&H->Lvb_d, n) && !dalloc_optional(&H->Lvb_f, n)) dfree(H->Lvb_d);
+    if (dalloc_optional(&H->Lvb_d, n, free_bytes) && !dalloc_optional(&H->Lvb_f, n, free_bytes)) dfree(H->Lvb_d);
     if (H->Lvb_d) {
       launch_pad_rows(nullptr, K, (int)NM, 0, H->Lnak, true, H->Lvb_d);
       launch_pad_rows(nullptr, K, (int)NM, 0, H->Lnak, true, H->Lvb_f);
@@ -129,7 +139,7 @@ void add_optional_tensors(afq_ham H) {
   if (likn_symmetric(nullptr, M, K, H->Likn)) {
     const long np = (long)M * (M + 1) / 2;
     const size_t n = (size_t)np * gemm_real_row(K);
-    if (dalloc_optional(&H->Lp_d, n) && !dalloc_optional(&H->Lp_f, n)) dfree(H->Lp_d);
+    if (dalloc_optional(&H->Lp_d, n, free_bytes) && !dalloc_optional(&H->Lp_f, n, free_bytes)) dfree(H->Lp_d);
     H->sym = H->Lp_d != nullptr;
     if (H->sym) {
       launch_pad_rows(nullptr, np, K, M, H->Likn, false, H->Lp_d);
@@ -139,7 +149,7 @@ void add_optional_tensors(afq_ham H) {
   // at most 2 GiB (N M = 16384 for a real trial), and only where many walkers take fewer operations
   const size_t pe = pair_table_elems((int)NM, H->real_trial);
   if (pe <= (size_t)1 << 28 && 2 * (NM / 64 + 1) <= (size_t)K && pair_table_pays(H) &&
-      (H->Lvb_d || !H->real_trial) && dalloc_optional(&H->pairs, pe))
+      (H->Lvb_d || !H->real_trial) && dalloc_optional(&H->pairs, pe, free_bytes))
     launch_pair_table(nullptr, M, N, K, H->real_trial ? H->Lvb_d : H->Lnak, H->real_trial, H->pairs);
 }
 
@@ -186,7 +196,8 @@ void reserve_workspace(afq_ham H, int max_walkers) {
   dalloc(&ws.ok, 1);
   if (H->pairs) {   // 128 MiB at most: products with more entries fill the chip unsplit
     ws.esplit_elems = std::min((long)kMaxSplits * max_walkers * H->K, 1L << 23);
-    if (!dalloc_optional(&ws.esplit, 2 * (size_t)ws.esplit_elems)) ws.esplit_elems = 0;
+    size_t free_bytes = free_memory();
+    if (!dalloc_optional(&ws.esplit, 2 * (size_t)ws.esplit_elems, free_bytes)) ws.esplit_elems = 0;
   }
   ws.cap = max_walkers;
 }
