@@ -268,46 +268,39 @@ const double* P1r_of(afq_ham H) { return H->P1_real ? H->P1r : nullptr; }
 // Estimated us of the energy's contractions per Cholesky vector in the handle's form and over the pair
 // table: linear in the work that the launches of each do, padding and rounds of workgroups included.
 // Fitted to 1040 measured sizes (M 16 to 256, N 3 to 32, K 0.5 M to 5 M, 1 to 1024 walkers, real and
-// complex trials, each form and the table; 90 % within a factor of 1.3 per vector, 1.2 over the table).
+// complex trials, each form and the table; 90 % within a factor of 1.15, 1.3 in INT8).
 // One crossover for all forms does not do: M 128, N 32, K 192, 64 walkers, complex trial takes 297 us
 // over the table and 260 (FP64), 235 (FP32), 61 (BF16X3), 129 (INT8) per vector, and M 128, N 32, K 640,
 // 1024 walkers 1857 against 12067, 12478, 2059 and 3803. Over the sizes measured the route taken is on the
-// average within 1 % of the faster one (4 % with one crossover; 19 % INT8 and 47 % BF16X3, complex).
+// average within 0.2 % of the faster one, 1.2 % in INT8 (with one crossover 2 to 12 %, complex trials 19 %
+// in INT8 and 47 % in BF16X3).
 double vectors_us(afq_ham H, int W) {
-  const double M = H->M, N = H->N, K = H->K, kNM = N * M * 1e-3;
-  const int nt = (H->N + 15) / 16;
-  auto mega = [&](int pad, double n, double m) { return (W + pad - 1) / pad * pad * n * n * m * K * 1e-6; };
+  const int M = H->M, N = H->N, K = H->K;
+  if (H->precision == AFQ_BF16X3) return exchange_bf16_us(W, M, N, K);
   if (H->precision == AFQ_INT8_SPLIT) {   // 6.8 to 7.2 us per 1000 elements of G to scale and slice them
-    const double c = mega(2, 16 * nt, (H->M + 63) / 64 * 64);
+    const double kNM = 1e-3 * N * M, rows = 16 * ((N + 15) / 16);
+    const double c = 1e-6 * ((W + 1) / 2 * 2) * rows * rows * ((M + 63) / 64 * 64) * K;
     const int n = N <= 8 ? 0 : N <= 16 ? 1 : 2;
     const double real[3] = {0.0163, 0.0360, 0.0296}, cplx[3] = {0.0219, 0.0615, 0.0510};
     return H->real_trial ? 13.3 + real[n] * c + 7.15 * kNM : 14.4 + cplx[n] * c + 6.81 * kNM;
   }
-  if (H->precision == AFQ_BF16X3) {       // rounds of workgroups that load G and then their vectors
-    const int cus = device_cus(), wgs = (W * nt + 7) / 8 * (exchange_bf16_chunks(W, H->N, H->K) / nt);
-    const double rounds = (wgs + cus - 1) / cus * ((H->M + 31) / 32);
-    return 10.8 + rounds * (0.486 * nt * exchange_bf16_chunk(W, H->N, H->K) + 2.39) + 0.32 * kNM;
-  }
-  if (H->precision == AFQ_FP64 && exchange_f64_supported(H->M, H->N))
-    return H->real_trial ? 13.8 + 0.092 * mega(4, N, M) + 1.5 * kNM : 14.1 + 0.161 * mega(4, N, M) + 4.45 * kNM;
-  const double c = mega(8, 16 * nt, M);   // the general kernel: FP64 takes 1.5 times the FP32 time
-  return (H->precision == AFQ_FP64 ? 1.5 : 1.0) *
-         (nt == 1 ? 18.3 + 0.0932 * c + 0.196 * M : 18.3 + 0.138 * c - 0.114 * M);
+  if (H->precision == AFQ_FP64 && exchange_f64_supported(M, N)) return exchange_f64_us(W, M, N, K, H->real_trial);
+  return exchange_general_us(H->precision, W, M, N, K);
 }
 double table_us(afq_ham H, int W) {
   const int NM = H->N * H->M;
+  const long split = std::min((long)kMaxSplits * W * H->K, 1L << 23);   // not by the reserved walkers
   const double pairs = pair_exchange_cost(W, NM, H->real_trial, H->K + 1);
-  if (H->real_trial)
-    return 8.0 + 1.30e-3 * pairs + 0.80 * gemm_f64_us(W, H->K, NM, H->ws.esplit_elems) + 1.9e-3 * NM;
-  return 8.4 + 1.18e-3 * pairs + 0.71 * gemm_nt_z_f64_us(W, H->K, NM, H->ws.esplit_elems) + 5.7e-3 * NM;
+  if (H->real_trial) return 7.7 + 1.54e-3 * pairs + 0.83 * gemm_f64_us(W, H->K, NM, split) + 1.1e-3 * NM;
+  return 6.8 + 1.54e-3 * pairs + 0.73 * gemm_nt_z_f64_us(W, H->K, NM, split) + 4.4e-3 * NM;
 }
-// INT8 on up to 16 electrons and a complex trial stays over the table, whose sums are FP64's, up to 1.2
+// INT8 on 9 to 16 electrons and a complex trial stays over the table, whose sums are FP64's, up to 1.25
 // times the estimate: M 64, N 16, K 200, 128 walkers takes 58 us there and 48 per vector.
 bool use_pairs(afq_ham H, int W) {
   if (H->pairs == nullptr || H->energy_route == AFQ_ROUTE_VECTORS) return false;
   if (H->energy_route == AFQ_ROUTE_TABLE) return true;
-  const bool near = H->precision == AFQ_INT8_SPLIT && H->N <= 16 && !H->real_trial;
-  return table_us(H, W) < (near ? 1.2 : 1.0) * vectors_us(H, W);
+  const bool near = H->precision == AFQ_INT8_SPLIT && H->N > 8 && H->N <= 16 && !H->real_trial;
+  return table_us(H, W) < (near ? 1.25 : 1.0) * vectors_us(H, W);
 }
 
 // the exchange contraction in the handle's precision: Kl and per-chunk tr(T^2) partials

@@ -272,17 +272,19 @@ void launch_pair_table(hipStream_t s, int M, int N, int K, const double* L, bool
 int pair_parts(int W, int NM, bool real, int max_parts);
 void launch_pair_exchange(hipStream_t s, int W, int NM, bool real, int max_parts, const double* G,
                           const double* B, double* part);
-// the work of launch_pair_exchange's fullest CU (rows times columns of its tiles), and estimated us of
+// the work of launch_pair_exchange's fullest CU (rows of its tiles times their mean k), and estimated us of
 // launch_gemm_real in FP64
 double pair_exchange_cost(int W, int NM, bool real, int max_parts);
 double gemm_f64_us(int m, int n, int k, long split_elems);
 // k_energy.hip
 int device_cus();                        // compute units of the current device (cached)
 int exx_nchunks(int W, int N, int K);   // chunks of Cholesky vectors the exchange kernel uses
+double exchange_general_us(int precision, int W, int M, int N, int K);   // estimated us of launch_exchange
 // k_exchange_f64.hip: the exchange of the FP64 form on up to 128 orbitals; Lreal (may be NULL) is
 // the zero-padded real Lnak of a real trial
 bool exchange_f64_supported(int M, int N);
 int exchange_f64_chunks(int W, int N, int K);   // tr(T^2) partials per walker
+double exchange_f64_us(int W, int M, int N, int K, bool real);   // estimated us of launch_exchange_f64
 int real_lnak_row(int M);                       // padded row length of Lreal
 void launch_exchange_f64(hipStream_t s, int W, int M, int N, int K, const double* G,
                          const double* Lnak, const double* Lreal, double* Kl, double* part);
@@ -302,6 +304,7 @@ bool exchange_bf16_supported(int M, int N);
 size_t exchange_bf16_elems(int M, int N, int K);   // bf16 elements of the exchange planes
 int exchange_bf16_chunk(int W, int N, int K);
 int exchange_bf16_chunks(int W, int N, int K);
+double exchange_bf16_us(int W, int M, int N, int K);   // estimated us of launch_exchange_bf16
 void split_lnak_bf16(hipStream_t s, int M, int N, int K, const double* Lnak, __bf16* Lb);
 void launch_exchange_bf16(hipStream_t s, int W, int M, int N, int K, const double* G,
                           const __bf16* Lb, double* Kl, double* exx_part);

@@ -315,6 +315,16 @@ int exx_nchunks(int W, int N, int K) {
   return (K + chunk - 1) / chunk;
 }
 
+// Fitted to 1212 measured calls (FP32: M 16 to 256, N 3 to 32, 1 to 1024 walkers; FP64: M from 130): 90 %
+// within 0.92 to 1.09 of the time. Per staged group of vectors its slices of 16 orbitals and the pair sums.
+double exchange_general_us(int precision, int W, int M, int N, int K) {
+  const int nv = exx_nv(N), wpb = exx_wpb(N), chunk = choose_chunk(W, K, nv, wpb), cus = device_cus();
+  const long wgs = (long)((W + wpb - 1) / wpb) * ((K + chunk - 1) / chunk);
+  const double groups = (double)((wgs + cus - 1) / cus) * std::min(chunk, K) / nv, slices = (M + 15) / 16;
+  if (precision == AFQ_FP64) return 5.7 + groups * (N <= 16 ? 10.7 * slices - 12.0 : 8.25 * slices - 20.0);
+  return 6.0 + groups * (N <= 16 ? 5.33 * slices + 8.3 : 4.35 * slices + 0.7);
+}
+
 void launch_exchange(hipStream_t s, int precision, int W, int M, int N, int K, const double* G,
                      const void* Lnak, double* Kl, double* exx_part) {
   if (W <= 0 || K <= 0) return;

@@ -328,7 +328,7 @@ __global__ __launch_bounds__(256, 2) void k_pair_table(int M, int NM, int K, con
 // at M 88, N 22 with 137, and 70 and 59 at M 77, N 19 with 201 and two tables.
 struct PairPlan {
   int tm, chunk, parts;
-  double cost;   // rounds times rows times columns of a chunk
+  double cost;   // rounds times rows times the mean k of an item
 };
 PairPlan pair_plan(int W, int NM, int planes, int max_parts) {
   const int nt = (NM + 63) / 64, cus = device_cus();
@@ -348,7 +348,7 @@ PairPlan pair_plan(int W, int NM, int planes, int max_parts) {
     const double rounds = (n - r + (r > 0 ? std::max((double)r, 1.6) : 0.0)) / (tm == 32 ? 0.9 : 1.0);
     const double cost = rounds * tm * p.chunk;
     if (tm == 128 || cost < 0.95 * best_cost) {
-      p.cost = rounds * tm * std::min(p.chunk, NM);
+      p.cost = rounds * tm * 32.0 * nt * (nt + 1) / p.parts;
       best = p;
       best_cost = cost;
     }

@@ -120,6 +120,8 @@ def test_route_without_a_table():
     (128, 16, 640, True, 64, A.BF16X3, 63, 99), (64, 16, 96, True, 128, A.INT8_SPLIT, 32, 63),
     (64, 16, 320, False, 512, A.FP32, 316, 69), (64, 16, 320, False, 512, A.INT8_SPLIT, 139, 69),
     (64, 16, 320, False, 512, A.FP64, 250, 69), (24, 6, 120, False, 64, A.FP64, 14, 25),
+    (64, 8, 32, True, 512, A.FP32, 36, 61), (160, 24, 480, False, 1, A.FP32, 47, 70),
+    (32, 16, 160, True, 1024, A.BF16X3, 98, 72), (40, 10, 200, True, 256, A.FP64, 73, 52),
 ])
 def test_route_is_the_faster_one(M, N, K, complex_trial, W, form, vectors, table):
     h, L, PsiT, _ = make(M, N, K, 1, complex_trial)
