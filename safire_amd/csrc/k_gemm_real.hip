@@ -17,6 +17,11 @@
 // that afq_autotune takes); vbias FP64 475 -> 230 us, FP32 277 -> 140 us. M 64,
 // N 16, K 320, 512 walkers, FP64: vHS 68 -> 46 us.
 //
+// The compiler keeps the prefetched pieces of B (pb) of the 64- and 32-row FP64 tiles and of the 64 x 128
+// FP32 ones in scratch, 48 bytes per lane: their loads are waited for before the MFMAs that they should
+// run under, and vHS at M 128 writes 307 MB for 135 MB of V. The rates above and the plans below, fitted
+// to measured times, contain that.
+//
 // The exchange as a quadratic form: sum_n tr(T_n^2) with T_n = G Lnak_n^T is G B G^T over the pairs
 // (electron, orbital), B[(b, j)][(a, i)] = sum_n Lnak[n][b][i] Lnak[n][a][j] from the set-up. B is
 // symmetric: 2 (N M)^2 flops per walker instead of the 4 N^2 M K of the T_n, and with K some multiples
